@@ -22,39 +22,14 @@
 //   atomics are used (deterministic).
 // fp32 path: one wavefront per query (or key) row, fp32 FMA, for the fp32
 //   parity configuration.
-#include <math.h>
-
 #include <atomic>
 #include <mutex>
 
-#include "common.h"
-#include "dropout_math.h"
-#include "lds_dma.h"
+#include "attention_common.h"
+#include "attention_generic.h"
 
 namespace nmb {
 namespace {
-
-constexpr int kMaxBlocks = 8;
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLn2 = 0.6931471805599453f;
-
-struct KVBlocks {
-  const void* k[kMaxBlocks];
-  const void* v[kMaxBlocks];
-  void* dk[kMaxBlocks];
-  void* dv[kMaxBlocks];
-  int64_t koff[kMaxBlocks];
-};
-
-struct AttnShape {
-  int B, Hq, Hkv, Sq, Sk, nblk, causal;
-  int64_t q_sb, q_ss, q_sh;
-  int64_t kv_sb, kv_ss, kv_sh;
-  int64_t o_sb, o_ss, o_sh;
-  int64_t q_offset;
-  float scale;       // softmax scale
-  float scale_log2;  // scale * log2(e)
-};
 
 // The RoPE backward fused into the dQ / dK stores: the gradient of the
 // rotated q (k) is rotated by -theta (reference nn/rotary.py:27-38; the
@@ -87,85 +62,6 @@ __device__ __forceinline__ int64_t rope_pos(const RopeGrad& rg, int b, int i, bo
   return *bad ? 0 : pos;
 }
 
-__device__ __forceinline__ f32x4 mfma16(const bf16x8& a, const bf16x8& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ bf16x8 zero8() {
-  bf16x8 z;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) z[i] = static_cast<bf16>(0.f);
-  return z;
-}
-
-__device__ __forceinline__ bf16x8 ld8(const bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
-
-// exp2 as the raw v_exp_f32: results below 2^-126 flush to 0, which is
-// immaterial for softmax weights (the library exp2 adds a 5-instruction
-// denormal range fix-up around every exponential).
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-// Number of 64-key tiles of a block that any query up to absolute position
-// q_last can see.
-__device__ __forceinline__ int visible_key_tiles(const AttnShape& p, int64_t koff, int64_t q_last) {
-  int n = (p.Sk + 63) >> 6;
-  if (p.causal) {
-    const int64_t lim = q_last - koff;
-    if (lim < 0) return 0;
-    const int64_t t = (lim >> 6) + 1;
-    if (t < n) n = static_cast<int>(t);
-  }
-  return n;
-}
-
-// Blocks are dispatched round-robin over the 8 XCDs (block L runs on XCD L % 8,
-// each XCD with its own L2).  Work item w = (L % 8) * per_xcd + L / 8 puts
-// consecutive items -- the q-tiles of one head, which read the same K/V -- on
-// the same XCD.  Returns -1 for the padding blocks of the last round.
-__device__ __forceinline__ int xcd_item(int items, int per_xcd) {
-  const int L = static_cast<int>(blockIdx.x);
-  const int w = (L % 8) * per_xcd + L / 8;
-  return w < items ? w : -1;
-}
-
-// Advance (blk, kt) to the next visible K/V tile of the concatenated blocks;
-// nt holds the visible tile count of block blk (recomputed only when the
-// block changes).
-__device__ __forceinline__ void next_tile(const AttnShape& p, const KVBlocks& kv, int64_t q_last,
-                                          int& blk, int& kt, int& nt) {
-  if (++kt < nt) return;
-  kt = 0;
-  for (++blk; blk < p.nblk; ++blk) {
-    nt = visible_key_tiles(p, kv.koff[blk], q_last);
-    if (nt > 0) return;
-  }
-}
-
-__device__ __forceinline__ int first_block(const AttnShape& p, const KVBlocks& kv, int64_t q_last,
-                                           int& nt) {
-  int blk = 0;
-  nt = 0;
-  for (; blk < p.nblk; ++blk) {
-    nt = visible_key_tiles(p, kv.koff[blk], q_last);
-    if (nt > 0) break;
-  }
-  return blk;
-}
-
-// Largest tile-relative key index (key = k0 + index) visible to a query at
-// absolute position qa: keys beyond Sk are never visible, and with causal
-// masking key position koff + k0 + index must not exceed qa.
-__device__ __forceinline__ int mask_limit(const AttnShape& p, int64_t koff, int k0, int64_t qa) {
-  int64_t lim = static_cast<int64_t>(p.Sk) - 1 - k0;
-  if (p.causal) {
-    const int64_t c = qa - koff - k0;
-    if (c < lim) lim = c;
-  }
-  if (lim < -1) lim = -1;
-  if (lim > 1 << 20) lim = 1 << 20;
-  return static_cast<int>(lim);
-}
-
 // ---------------------------------------------------------------- forward
 // Workgroup = NWV wavefronts x TQ column tiles of 16 queries of one (batch,
 // head): column tile t of wave w holds queries 16 NWV t + 16 w .. +15 of the
@@ -179,65 +75,6 @@ __device__ __forceinline__ int mask_limit(const AttnShape& p, int64_t koff, int 
 __device__ __forceinline__ float lse_to_log2(float v) {
   return v == -__builtin_inff() ? __builtin_inff() : v * kLog2e;
 }
-
-// 64-row x D bf16 tiles (K, V, Q, dO) stream from HBM straight into LDS
-// (buffer_load ... lds: no register round trip), kStages deep, so kStages - 1
-// tiles are in flight while one is computed.  A tile keeps the row-major
-// layout with its 16-byte chunks swizzled: chunk c of row r in slot
-// c ^ swz(r).  The swizzle serves both fragment kinds without bank conflicts
-// (SQ_LDS_BANK_CONFLICT reads zero for each kind alone on gfx950):
-//  * row fragments (an MFMA operand holding 8 consecutive columns of a row per
-//    lane; 16 rows per lane group): one ds_read_b128;
-//  * column fragments (8 rows of one column per lane: rows r0 + 4g .. +3 and
-//    r0 + 16 + 4g .. +3 of a 32-row chunk, the key/query order in which the
-//    score accumulators hold P and dS): two ds_read_b64_tr_b16.
-// (2 ((r >> 1) & 3) + ((r >> 3) & 1) at D 64 and 2 (r & 7) + ((r >> 3) & 1) at
-// D 128 keep the column reads conflict-free but give every row read a two-way
-// conflict; r & 15 at D 128 the reverse.)
-template <int D>
-struct Tile64 {
-  static constexpr int kElems = 64 * D;
-  __device__ static int swz(int r) { return D == 64 ? (r & 7) : 2 * (r & 7); }
-  __device__ static int at(int r, int col) { return r * D + 8 * ((col >> 3) ^ swz(r)) + (col & 7); }
-  // row r, columns col .. col + 7 (col a multiple of 8)
-  __device__ static bf16x8 row8(const bf16* t, int r, int col) { return ld8(t + at(r, col)); }
-  // lane (l16, g): column c0 + l16, rows r0 + 4g .. +3 then r0 + 16 + 4g .. +3
-  __device__ static bf16x8 col8(const bf16* t, int r0, int c0, int l16, int g) {
-    const int r = r0 + 4 * g + (l16 >> 2), cc = c0 + 4 * (l16 & 3);
-    return ld_tr(t + at(r, cc), t + at(r + 16, cc));
-  }
-};
-
-// One wave's share (of NW waves) of the direct loads of a 64-row tile: load j
-// fills LDS bytes [1024 (wave P + j), + 1024) of the tile; lane l's 16 bytes
-// are chunk slot s of row r there, read from global chunk s ^ swz(r).
-template <int D, int NW = 4>
-struct TileStream {
-  using Tile = Tile64<D>;
-  static constexpr int P = Tile::kElems * 2 / 1024 / NW;  // 1 KB loads per wave per tile
-  static_assert(P >= 1 && Tile::kElems * 2 % (1024 * NW) == 0, "a tile splits evenly over the waves");
-  uint32_t off[P];  // byte offset from row 0 of the tile
-  int row[P];
-
-  __device__ void init(int64_t row_stride, int wave, int lane) {
-#pragma unroll
-    for (int j = 0; j < P; ++j) {
-      const int e = (1024 * (wave * P + j) + 16 * lane) / 2;  // element offset within the tile
-      const int r = e / D, sl = (e % D) / 8;
-      row[j] = r;
-      off[j] = static_cast<uint32_t>(r * row_stride * 2) + 16u * static_cast<uint32_t>(sl ^ Tile::swz(r));
-    }
-  }
-
-  // rows r0 .. r0 + 63 (r0 * row bytes = r0_bytes) of a matrix of nrows rows;
-  // rows at and past nrows read as zeros
-  __device__ __forceinline__ void issue(const i32x4& rs, bf16* dst, int r0, int nrows, uint32_t r0_bytes,
-                                        int wave) const {
-#pragma unroll
-    for (int j = 0; j < P; ++j)
-      load_lds16(rs, dst + 512 * (wave * P + j), r0 + row[j] < nrows ? r0_bytes + off[j] : kOOB);
-  }
-};
 
 // FL (from LSE): the softmax statistics are given (lse read, not written), so
 // P = exp2(S * scale_log2 - lse2) directly: no running maximum, rescale or
@@ -554,27 +391,6 @@ __global__ __launch_bounds__(64 * NWV, (D == 64 && NWV == 4) ? (TQ <= 2 ? 3 : 2)
 #pragma unroll
   for (int t = 0; t < TQ; ++t)
     if (!stored[t]) store_tile(t);
-}
-
-// ---------------------------------------------------------------- delta (fp32 path)
-// delta[b, h, i] = sum_d dO[b, i, h, d] * O[b, i, h, d] (fp32).
-template <typename T>
-__global__ __launch_bounds__(256) void attn_delta_kernel(const T* __restrict__ o,
-                                                         const T* __restrict__ dout,
-                                                         float* __restrict__ delta, AttnShape p,
-                                                         int D) {
-  const int64_t rows = static_cast<int64_t>(p.B) * p.Sq * p.Hq;
-  for (int64_t r = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; r < rows;
-       r += static_cast<int64_t>(gridDim.x) * 256) {
-    const int h = static_cast<int>(r % p.Hq);
-    const int64_t bi = r / p.Hq;
-    const int i = static_cast<int>(bi % p.Sq);
-    const int b = static_cast<int>(bi / p.Sq);
-    const int64_t off = b * p.o_sb + static_cast<int64_t>(i) * p.o_ss + h * p.o_sh;
-    float s = 0.f;
-    for (int d = 0; d < D; ++d) s += to_f32(o[off + d]) * to_f32(dout[off + d]);
-    delta[(static_cast<int64_t>(b) * p.Hq + h) * p.Sq + i] = s;
-  }
 }
 
 // ---------------------------------------------------------------- dQ
@@ -1271,271 +1087,12 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel
   finish();
 }
 
-// ---------------------------------------------------------------- generic path
-// One wavefront per query row; lane owns head_dim elements lane and lane + 64
-// (head_dim <= 128).  The fp32 configuration's attention, and attention with
-// an explicit mask in any supported dtype (the reference passes attention_mask
-// to SDPA, nn/kernels/torch_backend.py:60-76): MK 0 no mask, 1 a boolean mask
-// (one byte per entry, nonzero = attend), 2 an additive mask in the attention
-// dtype (added to the scaled scores; -inf drops the key).  A query row with no
-// visible key gives zeros and lse = -inf, as the safe softmax of the
-// reference's SDPA does.  Attention dropout (SDPA's dropout_p, applied to the
-// normalised probabilities): probability (b, h, i, j) is multiplied by the
-// dropout_math.h factor of index ((b * Hq + h) * Sq + i) * Sk + j; l and the
-// lse stay those of the undropped softmax.
-struct MaskRef {
-  const void* p;
-  int64_t sb, sh, sq, sk;  // element strides of [batch, q_heads, seq_q, seq_k] (0: broadcast)
-};
-
-template <typename T, int MK>
-__device__ __forceinline__ bool visible(const MaskRef& mr, int b, int h, int64_t i, int64_t j, float& add) {
-  if constexpr (MK == 0) {
-    return true;
-  } else {
-    const int64_t off = b * mr.sb + h * mr.sh + i * mr.sq + j * mr.sk;
-    if constexpr (MK == 1) {
-      return static_cast<const uint8_t*>(mr.p)[off] != 0;
-    } else {
-      add = to_f32(static_cast<const T*>(mr.p)[off]);
-      return add != -__builtin_inff();
-    }
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ float dot_row(const T* a, const T* b, int D, int lane) {
-  float s = 0.f;
-  for (int d = lane; d < D; d += 64) s += to_f32(a[d]) * to_f32(b[d]);
-  return wave_sum(s);
-}
-
-template <typename T, int MK>
-__global__ __launch_bounds__(64) void attn_fwd_generic_kernel(const T* __restrict__ q, KVBlocks kv,
-                                                              T* __restrict__ o, float* __restrict__ lse,
-                                                              AttnShape p, int D, MaskRef mr,
-                                                              DropoutParams dp) {
-  const int lane = threadIdx.x;
-  const int i = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int hk = h / (p.Hq / p.Hkv);
-  const T* qr = q + b * p.q_sb + static_cast<int64_t>(i) * p.q_ss + h * p.q_sh;
-  const int64_t qa = p.q_offset + i;
-  const uint64_t prow = ((static_cast<uint64_t>(b) * p.Hq + h) * p.Sq + i) * p.Sk;  // dropout index base
-  float m = -__builtin_inff(), l = 0.f;
-  float acc[2] = {0.f, 0.f};
-  for (int blk = 0; blk < p.nblk; ++blk) {
-    const T* kb = static_cast<const T*>(kv.k[blk]) + b * p.kv_sb + hk * p.kv_sh;
-    const T* vb = static_cast<const T*>(kv.v[blk]) + b * p.kv_sb + hk * p.kv_sh;
-    const int64_t koff = kv.koff[blk];
-    for (int j = 0; j < p.Sk; ++j) {
-      if (p.causal && koff + j > qa) break;
-      float add = 0.f;
-      if (!visible<T, MK>(mr, b, h, i, j, add)) continue;
-      const T* kr = kb + static_cast<int64_t>(j) * p.kv_ss;
-      const T* vr = vb + static_cast<int64_t>(j) * p.kv_ss;
-      const float sc = dot_row(qr, kr, D, lane) * p.scale + add;
-      const float mnew = fmaxf(m, sc);
-      const float alpha = expf(m - mnew);
-      const float pv = expf(sc - mnew);
-      l = l * alpha + pv;
-      const float pz = pv * drop_factor(dp, prow + j);  // dropout acts after the normalisation
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const int d = lane + 64 * c;
-        if (d < D) acc[c] = acc[c] * alpha + pz * to_f32(vr[d]);
-      }
-      m = mnew;
-    }
-  }
-  T* orow = o + b * p.o_sb + static_cast<int64_t>(i) * p.o_ss + h * p.o_sh;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int d = lane + 64 * c;
-    if (d < D) orow[d] = from_f32<T>(acc[c] * inv);
-  }
-  if (lane == 0)
-    lse[(static_cast<int64_t>(b) * p.Hq + h) * p.Sq + i] = l > 0.f ? m + logf(l) : -__builtin_inff();
-}
-
-template <typename T, int MK>
-__global__ __launch_bounds__(64) void attn_bwd_dq_generic_kernel(
-    const T* __restrict__ q, KVBlocks kv, const T* __restrict__ dout,
-    const float* __restrict__ lse, const float* __restrict__ delta, T* __restrict__ dq,
-    AttnShape p, int D, MaskRef mr, DropoutParams dp) {
-  const int lane = threadIdx.x;
-  const int i = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int hk = h / (p.Hq / p.Hkv);
-  const T* qr = q + b * p.q_sb + static_cast<int64_t>(i) * p.q_ss + h * p.q_sh;
-  const T* dr = dout + b * p.o_sb + static_cast<int64_t>(i) * p.o_ss + h * p.o_sh;
-  const int64_t row = (static_cast<int64_t>(b) * p.Hq + h) * p.Sq + i;
-  const uint64_t prow = static_cast<uint64_t>(row) * p.Sk;
-  const float ls = lse[row], dl = delta[row];
-  const int64_t qa = p.q_offset + i;
-  float acc[2] = {0.f, 0.f};
-  if (ls != -__builtin_inff()) {
-    for (int blk = 0; blk < p.nblk; ++blk) {
-      const T* kb = static_cast<const T*>(kv.k[blk]) + b * p.kv_sb + hk * p.kv_sh;
-      const T* vb = static_cast<const T*>(kv.v[blk]) + b * p.kv_sb + hk * p.kv_sh;
-      const int64_t koff = kv.koff[blk];
-      for (int j = 0; j < p.Sk; ++j) {
-        if (p.causal && koff + j > qa) break;
-        float add = 0.f;
-        if (!visible<T, MK>(mr, b, h, i, j, add)) continue;
-        const T* kr = kb + static_cast<int64_t>(j) * p.kv_ss;
-        const T* vr = vb + static_cast<int64_t>(j) * p.kv_ss;
-        const float pv = expf(dot_row(qr, kr, D, lane) * p.scale + add - ls);
-        // dropout: dP = Z (dO . V) with Z = keep / (1 - p); delta = rowsum(dO o O) still
-        // equals sum_j P Z (dO . V), so dS = P (dP - delta)
-        const float ds = pv * (drop_factor(dp, prow + j) * dot_row(dr, vr, D, lane) - dl);
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const int d = lane + 64 * c;
-          if (d < D) acc[c] += ds * to_f32(kr[d]);
-        }
-      }
-    }
-  }
-  T* out = dq + b * p.q_sb + static_cast<int64_t>(i) * p.q_ss + h * p.q_sh;
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int d = lane + 64 * c;
-    if (d < D) out[d] = from_f32<T>(acc[c] * p.scale);
-  }
-}
-
-template <typename T, int MK>
-__global__ __launch_bounds__(64) void attn_bwd_dkdv_generic_kernel(
-    const T* __restrict__ q, KVBlocks kv, const T* __restrict__ dout,
-    const float* __restrict__ lse, const float* __restrict__ delta, AttnShape p, int D, MaskRef mr,
-    DropoutParams dp) {
-  const int lane = threadIdx.x;
-  const int j = blockIdx.x, hk = blockIdx.y;
-  const int blk = static_cast<int>(blockIdx.z) % p.nblk;
-  const int b = static_cast<int>(blockIdx.z) / p.nblk;
-  const int group = p.Hq / p.Hkv;
-  const int64_t koff = kv.koff[blk];
-  const int64_t kvo = b * p.kv_sb + static_cast<int64_t>(j) * p.kv_ss + hk * p.kv_sh;
-  const T* kr = static_cast<const T*>(kv.k[blk]) + kvo;
-  const T* vr = static_cast<const T*>(kv.v[blk]) + kvo;
-  float dk[2] = {0.f, 0.f}, dv[2] = {0.f, 0.f};
-  int i0 = 0;
-  if (p.causal) {
-    const int64_t fq = koff + j - p.q_offset;
-    i0 = fq <= 0 ? 0 : (fq >= p.Sq ? p.Sq : static_cast<int>(fq));
-  }
-  for (int hi = 0; hi < group; ++hi) {
-    const int h = hk * group + hi;
-    for (int i = i0; i < p.Sq; ++i) {
-      const int64_t row = (static_cast<int64_t>(b) * p.Hq + h) * p.Sq + i;
-      const float ls = lse[row];
-      if (ls == -__builtin_inff()) continue;
-      float add = 0.f;
-      if (!visible<T, MK>(mr, b, h, i, j, add)) continue;
-      const T* qr = q + b * p.q_sb + static_cast<int64_t>(i) * p.q_ss + h * p.q_sh;
-      const T* dr = dout + b * p.o_sb + static_cast<int64_t>(i) * p.o_ss + h * p.o_sh;
-      const float pv = expf(dot_row(qr, kr, D, lane) * p.scale + add - ls);
-      const float z = drop_factor(dp, static_cast<uint64_t>(row) * p.Sk + j);
-      const float ds = pv * (z * dot_row(dr, vr, D, lane) - delta[row]);
-      const float pz = pv * z;
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const int d = lane + 64 * c;
-        if (d < D) {
-          dv[c] += pz * to_f32(dr[d]);
-          dk[c] += ds * to_f32(qr[d]);
-        }
-      }
-    }
-  }
-  T* dkr = static_cast<T*>(kv.dk[blk]) + kvo;
-  T* dvr = static_cast<T*>(kv.dv[blk]) + kvo;
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int d = lane + 64 * c;
-    if (d < D) {
-      dkr[d] = from_f32<T>(dk[c] * p.scale);
-      dvr[d] = from_f32<T>(dv[c]);
-    }
-  }
-}
-
-// ---------------------------------------------------------------- host side
-int fill_shape(AttnShape* p, KVBlocks* kv, const void* q, const void* const* kb,
-               const void* const* vb, const int64_t* koff, int nblk, int64_t B, int64_t Hq,
-               int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D, const int64_t* qs,
-               const int64_t* kvs, const int64_t* os, int causal, int64_t q_offset, float scale,
-               int dtype) {
-  NMB_REQUIRE(q != nullptr && kb != nullptr && vb != nullptr && koff != nullptr && qs != nullptr &&
-                  kvs != nullptr && os != nullptr,
-              "attention: null argument");
-  NMB_REQUIRE(nblk >= 1 && nblk <= kMaxBlocks, "attention: n_blocks must be in [1, %d], got %d",
-              kMaxBlocks, nblk);
-  NMB_REQUIRE(B >= 0 && Hq > 0 && Hkv > 0 && Sq >= 0 && Sk >= 0 && D > 0,
-              "attention: invalid shape");
-  NMB_REQUIRE(Hq % Hkv == 0, "query heads (%lld) must be divisible by KV heads (%lld)",
-              (long long)Hq, (long long)Hkv);
-  NMB_REQUIRE(B <= 65535 && Hq <= 65535 && Sq <= 0x3fffffff && Sk <= 0x3fffffff,
-              "attention: shape exceeds the launch grid");
-  if (dtype == NMB_BF16) {
-    NMB_REQUIRE_SUPPORTED(D == 64 || D == 128, "attention (bf16): head_dim must be 64 or 128, got %lld",
-                          (long long)D);
-    for (int i = 0; i < 3; ++i)
-      NMB_REQUIRE_SUPPORTED(qs[i] % 8 == 0 && kvs[i] % 8 == 0 && os[i] % 8 == 0,
-                            "attention (bf16): strides must be multiples of 8 elements");
-    NMB_REQUIRE(aligned16(q), "attention: q must be 16-byte aligned");
-  } else if (dtype == NMB_F32) {
-    NMB_REQUIRE_SUPPORTED(D <= 128, "attention (fp32): head_dim must be <= 128, got %lld",
-                          (long long)D);
-  } else {
-    NMB_REQUIRE_SUPPORTED(false, "attention: unsupported dtype code %d", dtype);
-  }
-  for (int i = 0; i < nblk; ++i) {
-    NMB_REQUIRE(kb[i] != nullptr && vb[i] != nullptr, "attention: null K/V block %d", i);
-    NMB_REQUIRE(dtype != NMB_BF16 || (aligned16(kb[i]) && aligned16(vb[i])),
-                "attention: K/V blocks must be 16-byte aligned");
-    kv->k[i] = kb[i];
-    kv->v[i] = vb[i];
-    kv->koff[i] = koff[i];
-    kv->dk[i] = nullptr;
-    kv->dv[i] = nullptr;
-  }
-  p->B = static_cast<int>(B);
-  p->Hq = static_cast<int>(Hq);
-  p->Hkv = static_cast<int>(Hkv);
-  p->Sq = static_cast<int>(Sq);
-  p->Sk = static_cast<int>(Sk);
-  p->nblk = nblk;
-  p->causal = causal ? 1 : 0;
-  p->q_sb = qs[0];
-  p->q_ss = qs[1];
-  p->q_sh = qs[2];
-  p->kv_sb = kvs[0];
-  p->kv_ss = kvs[1];
-  p->kv_sh = kvs[2];
-  p->o_sb = os[0];
-  p->o_ss = os[1];
-  p->o_sh = os[2];
-  p->q_offset = q_offset;
-  p->scale = scale > 0.f ? scale : static_cast<float>(1.0 / sqrt(static_cast<double>(D)));
-  p->scale_log2 = p->scale * kLog2e;
-  return NMB_OK;
-}
-
 }  // namespace
 }  // namespace nmb
 
 using nmb::AttnShape;
 using nmb::KVBlocks;
 
-namespace {
-// Launch geometry of the XCD-mapped kernels: a 1-D grid of 8 * per_xcd blocks.
-void xcd_grid(int64_t items, int* per_xcd, unsigned* blocks) {
-  const int64_t per = (items + 7) / 8;
-  *per_xcd = static_cast<int>(per);
-  *blocks = static_cast<unsigned>(per * 8);
-}
-}  // namespace
 
 namespace nmb {
 namespace {
@@ -1773,158 +1330,6 @@ extern "C" int nmb_attn_bwd(const void* q, const void* const* k_blocks,
                             dv_blocks, workspace, workspace_bytes, batch, q_heads, kv_heads, seq_q,
                             seq_k, head_dim, q_strides, kv_strides, o_strides, causal, q_offset,
                             scale, dtype, stream, nullptr);
-}
-
-namespace nmb {
-namespace {
-
-// Shape, mask and dropout of the masked entry points: one K/V block at key
-// offset 0; the generic kernels load elements one at a time, so any head_dim
-// <= 128 and any strides (of bf16 or fp32 data) are accepted.  mask_kind 0
-// (no mask) serves attention with dropout alone.
-int masked_setup(AttnShape* p, KVBlocks* kv, MaskRef* mr, DropoutParams* dp, const void* q, const void* k,
-                 const void* v, int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
-                 int64_t seq_k, int64_t head_dim, const int64_t* qs, const int64_t* kvs, const int64_t* os,
-                 const void* mask, int mask_kind, const int64_t* ms, int causal, int64_t q_offset,
-                 float scale, float dropout_p, uint64_t seed, int dtype) {
-  NMB_REQUIRE_SUPPORTED(dtype == NMB_BF16 || dtype == NMB_F32, "attention (masked): unsupported dtype code %d",
-                        dtype);
-  NMB_REQUIRE(mask_kind == 0 || mask_kind == 1 || mask_kind == 2,
-              "attention (masked): mask_kind must be 0 (none), 1 (boolean) or 2 (additive), got %d",
-              mask_kind);
-  NMB_REQUIRE(dropout_p >= 0.f && dropout_p < 1.f, "attention (masked): dropout_p must be in [0, 1), got %g",
-              static_cast<double>(dropout_p));
-  if (mask_kind != 0) {
-    NMB_REQUIRE(mask != nullptr && ms != nullptr, "attention (masked): null mask");
-    NMB_REQUIRE(ms[0] >= 0 && ms[1] >= 0 && ms[2] >= 0 && ms[3] >= 0,
-                "attention (masked): mask strides must be non-negative");
-  }
-  const void* kb[1] = {k};
-  const void* vb[1] = {v};
-  const int64_t koff[1] = {0};
-  const int st = fill_shape(p, kv, q, kb, vb, koff, 1, batch, q_heads, kv_heads, seq_q, seq_k, head_dim,
-                            qs, kvs, os, causal, q_offset, scale, NMB_F32);
-  if (st != NMB_OK) return st;
-  *mr = mask_kind != 0 ? MaskRef{mask, ms[0], ms[1], ms[2], ms[3]} : MaskRef{};
-  *dp = make_dropout(static_cast<double>(dropout_p), seed);
-  return NMB_OK;
-}
-
-template <typename T>
-void masked_fwd_launch(const AttnShape& p, const KVBlocks& kv, const MaskRef& mr, const DropoutParams& dp,
-                       int kind, const void* q, void* o, float* lse, int D, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(p.Sq), static_cast<unsigned>(p.Hq), static_cast<unsigned>(p.B));
-  const T* qp = static_cast<const T*>(q);
-  T* op = static_cast<T*>(o);
-  if (kind == 0)
-    hipLaunchKernelGGL((attn_fwd_generic_kernel<T, 0>), grid, dim3(64), 0, stream, qp, kv, op, lse, p, D, mr, dp);
-  else if (kind == 1)
-    hipLaunchKernelGGL((attn_fwd_generic_kernel<T, 1>), grid, dim3(64), 0, stream, qp, kv, op, lse, p, D, mr, dp);
-  else
-    hipLaunchKernelGGL((attn_fwd_generic_kernel<T, 2>), grid, dim3(64), 0, stream, qp, kv, op, lse, p, D, mr, dp);
-}
-
-template <typename T>
-void masked_bwd_launch(const AttnShape& p, const KVBlocks& kv, const MaskRef& mr, const DropoutParams& drop,
-                       int kind, const void* q, const void* o, const void* dout, const float* lse, float* delta,
-                       void* dq, int D, hipStream_t stream) {
-  const T* qp = static_cast<const T*>(q);
-  const T* dp = static_cast<const T*>(dout);
-  const int64_t rows = static_cast<int64_t>(p.B) * p.Hq * p.Sq;
-  if (rows > 0) {
-    int64_t blocks = (rows + 255) / 256;
-    if (blocks > 8192) blocks = 8192;
-    hipLaunchKernelGGL(attn_delta_kernel<T>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
-                       static_cast<const T*>(o), dp, delta, p, D);
-    const dim3 grid(static_cast<unsigned>(p.Sq), static_cast<unsigned>(p.Hq), static_cast<unsigned>(p.B));
-    T* dqp = static_cast<T*>(dq);
-    if (kind == 0)
-      hipLaunchKernelGGL((attn_bwd_dq_generic_kernel<T, 0>), grid, dim3(64), 0, stream, qp, kv, dp, lse, delta,
-                         dqp, p, D, mr, drop);
-    else if (kind == 1)
-      hipLaunchKernelGGL((attn_bwd_dq_generic_kernel<T, 1>), grid, dim3(64), 0, stream, qp, kv, dp, lse, delta,
-                         dqp, p, D, mr, drop);
-    else
-      hipLaunchKernelGGL((attn_bwd_dq_generic_kernel<T, 2>), grid, dim3(64), 0, stream, qp, kv, dp, lse, delta,
-                         dqp, p, D, mr, drop);
-  }
-  if (p.Sk > 0 && p.B > 0) {
-    const dim3 grid(static_cast<unsigned>(p.Sk), static_cast<unsigned>(p.Hkv), static_cast<unsigned>(p.B));
-    if (kind == 0)
-      hipLaunchKernelGGL((attn_bwd_dkdv_generic_kernel<T, 0>), grid, dim3(64), 0, stream, qp, kv, dp, lse,
-                         delta, p, D, mr, drop);
-    else if (kind == 1)
-      hipLaunchKernelGGL((attn_bwd_dkdv_generic_kernel<T, 1>), grid, dim3(64), 0, stream, qp, kv, dp, lse,
-                         delta, p, D, mr, drop);
-    else
-      hipLaunchKernelGGL((attn_bwd_dkdv_generic_kernel<T, 2>), grid, dim3(64), 0, stream, qp, kv, dp, lse,
-                         delta, p, D, mr, drop);
-  }
-}
-
-}  // namespace
-}  // namespace nmb
-
-extern "C" int nmb_attn_masked_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
-                                   int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
-                                   int64_t seq_k, int64_t head_dim, const int64_t* q_strides,
-                                   const int64_t* kv_strides, const int64_t* o_strides, const void* mask,
-                                   int mask_kind, const int64_t* mask_strides, int causal,
-                                   int64_t q_offset, float scale, float dropout_p, uint64_t seed, int dtype,
-                                   hipStream_t stream) {
-  AttnShape p;
-  KVBlocks kv;
-  nmb::MaskRef mr;
-  nmb::DropoutParams dp;
-  const int st = nmb::masked_setup(&p, &kv, &mr, &dp, q, k, v, batch, q_heads, kv_heads, seq_q, seq_k,
-                                   head_dim, q_strides, kv_strides, o_strides, mask, mask_kind, mask_strides,
-                                   causal, q_offset, scale, dropout_p, seed, dtype);
-  if (st != NMB_OK) return st;
-  NMB_REQUIRE(o != nullptr && lse != nullptr, "attn_masked_fwd: null output");
-  if (batch == 0 || seq_q == 0) return NMB_OK;
-  if (dtype == NMB_BF16)
-    nmb::masked_fwd_launch<nmb::bf16>(p, kv, mr, dp, mask_kind, q, o, lse, static_cast<int>(head_dim), stream);
-  else
-    nmb::masked_fwd_launch<float>(p, kv, mr, dp, mask_kind, q, o, lse, static_cast<int>(head_dim), stream);
-  NMB_CHECK_LAUNCH("attn_masked_fwd");
-  return NMB_OK;
-}
-
-extern "C" int nmb_attn_masked_bwd(const void* q, const void* k, const void* v, const void* o,
-                                   const void* dout, const float* lse, void* dq, void* dk, void* dv,
-                                   void* workspace, size_t workspace_bytes, int64_t batch,
-                                   int64_t q_heads, int64_t kv_heads, int64_t seq_q, int64_t seq_k,
-                                   int64_t head_dim, const int64_t* q_strides, const int64_t* kv_strides,
-                                   const int64_t* o_strides, const void* mask, int mask_kind,
-                                   const int64_t* mask_strides, int causal, int64_t q_offset, float scale,
-                                   float dropout_p, uint64_t seed, int dtype, hipStream_t stream) {
-  AttnShape p;
-  KVBlocks kv;
-  nmb::MaskRef mr;
-  nmb::DropoutParams dp;
-  const int st = nmb::masked_setup(&p, &kv, &mr, &dp, q, k, v, batch, q_heads, kv_heads, seq_q, seq_k,
-                                   head_dim, q_strides, kv_strides, o_strides, mask, mask_kind, mask_strides,
-                                   causal, q_offset, scale, dropout_p, seed, dtype);
-  if (st != NMB_OK) return st;
-  NMB_REQUIRE(o != nullptr && dout != nullptr && lse != nullptr && dq != nullptr && dk != nullptr &&
-                  dv != nullptr,
-              "attn_masked_bwd: null argument");
-  const size_t need = static_cast<size_t>(batch * q_heads * seq_q) * sizeof(float);
-  NMB_REQUIRE(workspace != nullptr && workspace_bytes >= need,
-              "attn_masked_bwd: workspace of %zu bytes is smaller than the %zu required", workspace_bytes,
-              need);
-  kv.dk[0] = dk;
-  kv.dv[0] = dv;
-  if (batch == 0) return NMB_OK;
-  float* delta = static_cast<float*>(workspace);
-  if (dtype == NMB_BF16)
-    nmb::masked_bwd_launch<nmb::bf16>(p, kv, mr, dp, mask_kind, q, o, dout, lse, delta, dq,
-                                      static_cast<int>(head_dim), stream);
-  else
-    nmb::masked_bwd_launch<float>(p, kv, mr, dp, mask_kind, q, o, dout, lse, delta, dq,
-                                  static_cast<int>(head_dim), stream);
-  NMB_CHECK_LAUNCH("attn_masked_bwd");
-  return NMB_OK;
 }
 
 extern "C" int nmb_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o,

@@ -1,0 +1,88 @@
+"""The MFMA kernels of masked and dropped-out attention (bf16, head dims 64 and
+128) at their edges, against the oracle in fp32: 64-row tiles and remainders,
+the mask layouts with kernels of their own (one bit per key, boolean per score,
+additive; four at a time or one by one), skipped tiles, grouped heads, offsets
+and dropout over even and odd key counts."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import nano_megatron_amd.functional as Fn
+from oracle import reference as R
+from tests.parity import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # (mask, causal, offset, hq, hkv, sq, sk, d, p)
+    ("none", True, 0, 2, 2, 1, 1, 64, 0.3),
+    ("none", True, 3, 4, 2, 130, 191, 64, 0.1),  # odd key count: dropout pairs straddle rows
+    ("none", False, 0, 4, 1, 64, 128, 128, 0.1),
+    ("keys", True, 0, 4, 4, 200, 200, 64, 0.0),
+    ("keys", False, 0, 4, 2, 65, 321, 128, 0.0),
+    ("keys", True, 16400, 1, 1, 5, 16384, 64, 0.0),  # the most keys kept as bits in LDS
+    ("keys", True, 16400, 1, 1, 5, 16385, 64, 0.0),  # one more: read per score
+    ("keys_heads", True, 0, 4, 2, 129, 129, 64, 0.2),
+    ("bool", True, 0, 2, 2, 63, 64, 64, 0.0),  # four mask bytes per load
+    ("bool", False, 0, 2, 1, 70, 131, 128, 0.15),  # one by one
+    ("add", False, 0, 4, 4, 96, 128, 64, 0.0),
+    ("add", False, 0, 2, 2, 33, 50, 128, 0.1),
+]
+
+
+@pytest.mark.parametrize("kind,causal,offset,hq,hkv,sq,sk,d,p", CASES)
+def test_masked_mfma_attention_matches_oracle(kind, causal, offset, hq, hkv, sq, sk, d, p) -> None:
+    """Probabilities stay at fp32 precision, so O and dV carry one bf16
+    rounding: at most 2^-9 of each element, hence of the norm (bf16
+    probabilities would add as much again).  dQ and dK also see delta formed
+    from the rounded O: twice that bound.  Keys hidden from every query may
+    hold NaN; a row of masks of the lowest value averages over all keys."""
+    g = torch.Generator().manual_seed(11)
+    b = 2
+    q, do = (torch.randn(b, hq, sq, d, generator=g).bfloat16() for _ in range(2))
+    k, v = (torch.randn(b, hkv, sk, d, generator=g).bfloat16() for _ in range(2))
+    mask = None
+    if kind == "keys":  # leading, trailing and whole-tile gaps
+        mask = torch.rand(b, 1, 1, sk, generator=g) > 0.2
+        mask[0, ..., sk // 3:] = False
+        mask[1, ..., : sk // 2] = False
+    elif kind == "keys_heads":
+        mask = torch.rand(b, hq, 1, sk, generator=g) > 0.4
+    elif kind == "bool":
+        mask = torch.rand(b, 1, sq, sk, generator=g) > 0.3
+        mask[1, 0, 3] = False
+    elif kind == "add":
+        mask = torch.randn(sq, sk, generator=g).bfloat16()
+        mask[2, 1:9] = float("-inf")
+        mask[1, 4:] = torch.finfo(torch.bfloat16).min
+        mask[0] = torch.finfo(torch.bfloat16).min
+        do[:, :, 0] = 0
+        mask[4] = float("-inf")
+    qr, kr, vr = (t.float().clone().requires_grad_(True) for t in (q, k, v))
+    mr = mask.float() if kind == "add" else mask
+    o_ref = R.local_attention(qr, kr, vr, causal=causal, sequence_offset=offset, attention_mask=mr, dropout_p=p,
+                              dropout_seed=77)
+    o_ref.backward(do.float())
+    if kind == "keys":
+        hidden = ~mask[:, :, 0, :, None].expand(b, hkv, sk, d)
+        k, v = k.masked_fill(hidden, float("nan")), v.masked_fill(hidden, float("nan"))
+    if kind == "keys" and sk > 16384:  # per score: 0 x NaN is NaN, as in the reference's products
+        k, v = k.nan_to_num(0.0), v.nan_to_num(0.0)
+    qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    o = Fn.masked_attention(qd, kd, vd, None if mask is None else mask.cuda(), causal=causal,
+                            sequence_offset=offset, dropout_p=p, seed=77)
+    o.backward(do.cuda())
+    ulp = 2.0 ** -9
+    for name, got, exp, bound in (("o", o, o_ref, 1.02 * ulp), ("dv", vd.grad, vr.grad, 1.02 * ulp),
+                                  ("dq", qd.grad, qr.grad, 2 * ulp), ("dk", kd.grad, kr.grad, 2 * ulp)):
+        assert torch.isfinite(got).all(), name
+        if float(exp.detach().abs().max()) < 1e-6:
+            # one visible key per query: dS = dO . V - delta vanishes but for the
+            # rounding of the O that delta is formed from
+            ds = ulp * float((do.float() * o_ref.detach()).abs().sum(-1).max())
+            x = max(float(q.float().abs().max()), float(k.float().abs().max()))
+            assert float(got.detach().abs().max()) <= 1.02 * ds * x / d ** 0.5 / (1 - p), name
+        else:
+            assert rel_l2(got, exp) <= bound, (name, rel_l2(got, exp))
