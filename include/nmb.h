@@ -318,6 +318,16 @@ int nmb_gemm_f32(int a_layout, int b_layout, int64_t m, int64_t n, int64_t k, fl
                  const float* a, int64_t lda, const float* b, int64_t ldb, float beta,
                  const float* c, int64_t ldc, float* d, int64_t ldd, hipStream_t stream);
 
+/* The same with the K range split over workgroups where the output alone has
+ * too few tiles to fill the GPU: workspace of nmb_gemm_f32_workspace_bytes
+ * bytes (0: no split), 16-byte aligned, for the fp32 partial products, which
+ * are summed in a fixed order. */
+int nmb_gemm_f32_workspace_bytes(int64_t m, int64_t n, int64_t k, int64_t* bytes);
+int nmb_gemm_f32_split(int a_layout, int b_layout, int64_t m, int64_t n, int64_t k, float alpha,
+                       const float* a, int64_t lda, const float* b, int64_t ldb, float beta,
+                       const float* c, int64_t ldc, float* d, int64_t ldd, void* workspace,
+                       int64_t workspace_bytes, hipStream_t stream);
+
 /* GEMM with the rotary embedding as its epilogue: the Q/K/V projection and
  * RoPE of q and k in one pass (reference models/gpt/attention.py:172-181 with
  * nn/rotary.py:27-38, 55-70; replaces nmb_gemm_bf16 + two nmb_rope_apply).

@@ -73,7 +73,7 @@ def _workspace(nbytes: int, device: torch.device) -> Tensor:
 
 
 # ---------------------------------------------------------------- GEMM
-_GEMM_WS: dict = {}  # (layouts, m, n, k) -> split-K workspace bytes (a pure function of the shape)
+_GEMM_WS: dict = {}  # (layouts or "f32", m, n, k) -> split-K workspace bytes (a pure function of the shape)
 
 
 def _operand_layout(t: Tensor, rows_dim: int) -> tuple[int, int]:
@@ -91,7 +91,7 @@ def mm(a: Tensor, b: Tensor, *, out: Tensor | None = None, c: Tensor | None = No
     """``out = alpha * a @ b + beta * c`` for 2-D tensors (``c`` may be ``out``).
 
     bf16 runs the gfx950 MFMA kernel ``nmb_gemm_bf16``, fp32 (the parity
-    configuration) the fp32-MFMA kernel ``nmb_gemm_f32``; both take any mix of
+    configuration) the fp32-MFMA kernel ``nmb_gemm_f32_split``; both take any mix of
     row/column-major operands.  Other dtypes are a ValueError.
     """
     m, k = a.shape
@@ -181,11 +181,18 @@ def _mm_f32(a: Tensor, b: Tensor, out: Tensor, c: Tensor | None, alpha: float, b
         raise ValueError("gemm: the output must be row-major")
     if beta != 0.0 and (c is None or (c.stride(1) != 1 and c.numel() > 1)):
         raise ValueError("gemm: beta != 0 needs a row-major C")
+    key = ("f32", m, n, k)
+    nbytes = _GEMM_WS.get(key)
+    if nbytes is None:
+        size = _lib.ctypes.c_int64()
+        _lib.call("nmb_gemm_f32_workspace_bytes", m, n, k, _lib.ctypes.byref(size))
+        nbytes = _GEMM_WS[key] = size.value
+    ws = _workspace(nbytes, a.device) if nbytes else None
     _lib.call(
-        "nmb_gemm_f32", la, 1 - lb_rowmajor, m, n, k, float(alpha), a.data_ptr(), lda, b.data_ptr(),
+        "nmb_gemm_f32_split", la, 1 - lb_rowmajor, m, n, k, float(alpha), a.data_ptr(), lda, b.data_ptr(),
         ldb, float(beta), _lib.ptr(c) if beta != 0.0 else None,
         max(c.stride(0), n) if (c is not None and beta != 0.0) else n, out.data_ptr(),
-        max(out.stride(0), n), _lib.stream_of(a),
+        max(out.stride(0), n), _lib.ptr(ws), nbytes, _lib.stream_of(a),
     )
     return out
 
