@@ -20,13 +20,12 @@
 //   GQA reads KV head h / (Hq / Hkv) directly; the dK/dV workgroup of a KV
 //   head loops over its query heads, so no repeat is materialised and no
 //   atomics are used (deterministic).
-// fp32 path: one wavefront per query (or key) row, fp32 FMA, for the fp32
-//   parity configuration.
+// fp32 path: attention_f32.h, on the fp32 matrix core.
 #include <atomic>
 #include <mutex>
 
 #include "attention_common.h"
-#include "attention_generic.h"
+#include "attention_f32.h"
 
 namespace nmb {
 namespace {
@@ -1146,11 +1145,8 @@ int attn_fwd_impl(bool from_lse, const void* q, const void* const* k_blocks,
 #undef NMB_FWD
   } else {
     NMB_REQUIRE_SUPPORTED(!from_lse, "attn_fwd_from_lse: bf16 only");
-    const dim3 grid(static_cast<unsigned>(seq_q), static_cast<unsigned>(q_heads),
-                    static_cast<unsigned>(batch));
-    hipLaunchKernelGGL((nmb::attn_fwd_generic_kernel<float, 0>), grid, dim3(64), 0, stream,
-                       static_cast<const float*>(q), kv, static_cast<float*>(o), lse, p,
-                       static_cast<int>(head_dim), nmb::MaskRef{}, nmb::DropoutParams{0, 0, 1.f});
+    f32_fwd_launch<float>(p, kv, MaskRef{}, DropoutParams{0, 0, 1.f}, 0, false, q, o, lse,
+                          static_cast<int>(head_dim), stream);
   }
   NMB_CHECK_LAUNCH("attn_fwd");
   return NMB_OK;
@@ -1284,32 +1280,9 @@ int attn_bwd_impl(const void* q, const void* const* k_blocks,
       NMB_CHECK_LAUNCH("attn_bwd(dkdv)");
     }
   } else {
-    if (seq_q > 0) {
-      int64_t rows = batch * q_heads * seq_q;
-      int64_t blocks = (rows + 255) / 256;
-      if (blocks > 8192) blocks = 8192;
-      hipLaunchKernelGGL(nmb::attn_delta_kernel<float>, dim3(static_cast<unsigned>(blocks)),
-                         dim3(256), 0, stream, static_cast<const float*>(o),
-                         static_cast<const float*>(dout), delta, p, D);
-      NMB_CHECK_LAUNCH("attn_bwd(delta)");
-    }
-    const float* qp = static_cast<const float*>(q);
-    const float* dp = static_cast<const float*>(dout);
-    if (seq_q > 0) {
-      const dim3 grid(static_cast<unsigned>(seq_q), static_cast<unsigned>(q_heads),
-                      static_cast<unsigned>(batch));
-      hipLaunchKernelGGL((nmb::attn_bwd_dq_generic_kernel<float, 0>), grid, dim3(64), 0, stream, qp, kv,
-                         dp, lse, delta, static_cast<float*>(dq), p, D, nmb::MaskRef{},
-                         nmb::DropoutParams{0, 0, 1.f});
-      NMB_CHECK_LAUNCH("attn_bwd(dq,f32)");
-    }
-    if (seq_k > 0) {
-      const dim3 grid(static_cast<unsigned>(seq_k), static_cast<unsigned>(kv_heads),
-                      static_cast<unsigned>(batch * n_blocks));
-      hipLaunchKernelGGL((nmb::attn_bwd_dkdv_generic_kernel<float, 0>), grid, dim3(64), 0, stream, qp,
-                         kv, dp, lse, delta, p, D, nmb::MaskRef{}, nmb::DropoutParams{0, 0, 1.f});
-      NMB_CHECK_LAUNCH("attn_bwd(dkdv,f32)");
-    }
+    f32_bwd_launch<float>(p, kv, MaskRef{}, DropoutParams{0, 0, 1.f}, 0, false, q, o, dout, lse, delta, dq, D,
+                          stream);
+    NMB_CHECK_LAUNCH("attn_bwd(f32)");
   }
   return NMB_OK;
 }

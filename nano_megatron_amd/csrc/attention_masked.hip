@@ -1,6 +1,6 @@
 // Attention with an explicit mask and / or attention dropout for gfx950:
 // the reference passes attention_mask and dropout_p to SDPA
-// (nn/kernels/torch_backend.py:60-76).  Semantics as attention_generic.h: a
+// (nn/kernels/torch_backend.py:60-76).  Semantics as attention_f32.h: a
 // query row with no visible key gives zeros and lse = -inf, dropout multiplies
 // the normalised probabilities by the dropout_math.h factor of element
 // ((b Hq + h) Sq + i) Sk + j, and l and the lse stay those of the undropped
@@ -33,7 +33,7 @@
 #include <type_traits>
 
 #include "attention_common.h"
-#include "attention_generic.h"
+#include "attention_f32.h"
 
 namespace nmb {
 namespace {
@@ -52,23 +52,6 @@ struct MaskRead {
 __device__ __forceinline__ void split2(float p, bf16& hi, bf16& lo) {
   hi = static_cast<bf16>(p);
   lo = static_cast<bf16>(p - static_cast<float>(hi));
-}
-
-// The keep decisions of elements idx0 .. idx0 + 3 (even: idx0 is even).
-__device__ __forceinline__ void keep4(const DropoutParams& d, uint64_t idx0, bool even, bool (&keep)[4]) {
-  const uint64_t c = idx0 >> 1;
-  const uint64_t z0 = splitmix64(d.seed, c), z1 = splitmix64(d.seed, c + 1);
-  const uint32_t w[4] = {static_cast<uint32_t>(z0), static_cast<uint32_t>(z0 >> 32), static_cast<uint32_t>(z1),
-                         static_cast<uint32_t>(z1 >> 32)};
-  if (even) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) keep[e] = w[e] >= d.threshold;
-  } else {
-    const uint32_t w4 = static_cast<uint32_t>(splitmix64(d.seed, c + 2));
-    const bool odd = idx0 & 1;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) keep[e] = (odd ? (e < 3 ? w[e + 1] : w4) : w[e]) >= d.threshold;
-  }
 }
 
 // Bit key % 64 of word key / 64: key is visible in the boolean mask row at
@@ -675,8 +658,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dkdv_kernel(
 // ---------------------------------------------------------------- dispatch
 // The MFMA kernels take bf16 heads of 64 and 128 whose rows are 16-byte
 // aligned with 64 rows inside one 2 GiB descriptor, and work items that fit
-// one launch; every other call runs the one-row-per-wavefront kernels (at
-// B 8, Hq 16, S 512, D 64 those take 6.7 ms for a forward and backward).
+// one launch; every other call runs the fp32 matrix-core kernels of
+// attention_f32.h.
 bool mfma_shape(const AttnShape& p, int64_t D, int dtype, std::initializer_list<const void*> rows16) {
   if (dtype != NMB_BF16 || (D != 64 && D != 128) || p.Sk == 0) return false;
   for (const void* r : rows16)
@@ -774,8 +757,8 @@ namespace nmb {
 namespace {
 
 // Shape, mask and dropout of the masked entry points: one K/V block at key
-// offset 0; the generic kernels load elements one at a time, so any head_dim
-// <= 128 and any strides (of bf16 or fp32 data) are accepted.  mask_kind 0
+// offset 0; any head_dim <= 128 and any strides (of bf16 or fp32 data) are
+// accepted.  mask_kind 0
 // (no mask) serves attention with dropout alone.
 int masked_setup(AttnShape* p, KVBlocks* kv, MaskRef* mr, DropoutParams* dp, const void* q, const void* k,
                  const void* v, int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
@@ -805,58 +788,6 @@ int masked_setup(AttnShape* p, KVBlocks* kv, MaskRef* mr, DropoutParams* dp, con
   return NMB_OK;
 }
 
-template <typename T>
-void masked_fwd_launch(const AttnShape& p, const KVBlocks& kv, const MaskRef& mr, const DropoutParams& dp,
-                       int kind, const void* q, void* o, float* lse, int D, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(p.Sq), static_cast<unsigned>(p.Hq), static_cast<unsigned>(p.B));
-  const T* qp = static_cast<const T*>(q);
-  T* op = static_cast<T*>(o);
-  if (kind == 0)
-    hipLaunchKernelGGL((attn_fwd_generic_kernel<T, 0>), grid, dim3(64), 0, stream, qp, kv, op, lse, p, D, mr, dp);
-  else if (kind == 1)
-    hipLaunchKernelGGL((attn_fwd_generic_kernel<T, 1>), grid, dim3(64), 0, stream, qp, kv, op, lse, p, D, mr, dp);
-  else
-    hipLaunchKernelGGL((attn_fwd_generic_kernel<T, 2>), grid, dim3(64), 0, stream, qp, kv, op, lse, p, D, mr, dp);
-}
-
-template <typename T>
-void masked_bwd_launch(const AttnShape& p, const KVBlocks& kv, const MaskRef& mr, const DropoutParams& drop,
-                       int kind, const void* q, const void* o, const void* dout, const float* lse, float* delta,
-                       void* dq, int D, hipStream_t stream) {
-  const T* qp = static_cast<const T*>(q);
-  const T* dp = static_cast<const T*>(dout);
-  const int64_t rows = static_cast<int64_t>(p.B) * p.Hq * p.Sq;
-  if (rows > 0) {
-    int64_t blocks = (rows + 255) / 256;
-    if (blocks > 8192) blocks = 8192;
-    hipLaunchKernelGGL(attn_delta_kernel<T>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
-                       static_cast<const T*>(o), dp, delta, p, D);
-    const dim3 grid(static_cast<unsigned>(p.Sq), static_cast<unsigned>(p.Hq), static_cast<unsigned>(p.B));
-    T* dqp = static_cast<T*>(dq);
-    if (kind == 0)
-      hipLaunchKernelGGL((attn_bwd_dq_generic_kernel<T, 0>), grid, dim3(64), 0, stream, qp, kv, dp, lse, delta,
-                         dqp, p, D, mr, drop);
-    else if (kind == 1)
-      hipLaunchKernelGGL((attn_bwd_dq_generic_kernel<T, 1>), grid, dim3(64), 0, stream, qp, kv, dp, lse, delta,
-                         dqp, p, D, mr, drop);
-    else
-      hipLaunchKernelGGL((attn_bwd_dq_generic_kernel<T, 2>), grid, dim3(64), 0, stream, qp, kv, dp, lse, delta,
-                         dqp, p, D, mr, drop);
-  }
-  if (p.Sk > 0 && p.B > 0) {
-    const dim3 grid(static_cast<unsigned>(p.Sk), static_cast<unsigned>(p.Hkv), static_cast<unsigned>(p.B));
-    if (kind == 0)
-      hipLaunchKernelGGL((attn_bwd_dkdv_generic_kernel<T, 0>), grid, dim3(64), 0, stream, qp, kv, dp, lse,
-                         delta, p, D, mr, drop);
-    else if (kind == 1)
-      hipLaunchKernelGGL((attn_bwd_dkdv_generic_kernel<T, 1>), grid, dim3(64), 0, stream, qp, kv, dp, lse,
-                         delta, p, D, mr, drop);
-    else
-      hipLaunchKernelGGL((attn_bwd_dkdv_generic_kernel<T, 2>), grid, dim3(64), 0, stream, qp, kv, dp, lse,
-                         delta, p, D, mr, drop);
-  }
-}
-
 }  // namespace
 }  // namespace nmb
 
@@ -880,9 +811,11 @@ extern "C" int nmb_attn_masked_fwd(const void* q, const void* k, const void* v, 
   if (nmb::mfma_shape(p, head_dim, dtype, {q, k, v, o}))
     nmb::mfma_fwd_launch(p, mr, dp, mask_kind, dropout_p > 0.f, static_cast<int>(head_dim), q, k, v, o, lse, stream);
   else if (dtype == NMB_BF16)
-    nmb::masked_fwd_launch<nmb::bf16>(p, kv, mr, dp, mask_kind, q, o, lse, static_cast<int>(head_dim), stream);
+    nmb::f32_fwd_launch<nmb::bf16>(p, kv, mr, dp, mask_kind, dropout_p > 0.f, q, o, lse, static_cast<int>(head_dim),
+                                   stream);
   else
-    nmb::masked_fwd_launch<float>(p, kv, mr, dp, mask_kind, q, o, lse, static_cast<int>(head_dim), stream);
+    nmb::f32_fwd_launch<float>(p, kv, mr, dp, mask_kind, dropout_p > 0.f, q, o, lse, static_cast<int>(head_dim),
+                               stream);
   NMB_CHECK_LAUNCH("attn_masked_fwd");
   return NMB_OK;
 }
@@ -918,11 +851,11 @@ extern "C" int nmb_attn_masked_bwd(const void* q, const void* k, const void* v, 
     nmb::mfma_bwd_launch(p, mr, dp, mask_kind, dropout_p > 0.f, static_cast<int>(head_dim), q, k, v, o, dout, lse,
                          delta, dq, dk, dv, stream);
   else if (dtype == NMB_BF16)
-    nmb::masked_bwd_launch<nmb::bf16>(p, kv, mr, dp, mask_kind, q, o, dout, lse, delta, dq,
-                                      static_cast<int>(head_dim), stream);
+    nmb::f32_bwd_launch<nmb::bf16>(p, kv, mr, dp, mask_kind, dropout_p > 0.f, q, o, dout, lse, delta, dq,
+                                   static_cast<int>(head_dim), stream);
   else
-    nmb::masked_bwd_launch<float>(p, kv, mr, dp, mask_kind, q, o, dout, lse, delta, dq,
-                                  static_cast<int>(head_dim), stream);
+    nmb::f32_bwd_launch<float>(p, kv, mr, dp, mask_kind, dropout_p > 0.f, q, o, dout, lse, delta, dq,
+                               static_cast<int>(head_dim), stream);
   NMB_CHECK_LAUNCH("attn_masked_bwd");
   return NMB_OK;
 }

@@ -53,4 +53,21 @@ __device__ __forceinline__ float drop_factor(const DropoutParams& d, uint64_t id
   return keep_bits(d.seed, idx) >= d.threshold ? d.scale : 0.f;
 }
 
+// The keep decisions of elements idx0 .. idx0 + 3 (even: idx0 is even).
+__device__ __forceinline__ void keep4(const DropoutParams& d, uint64_t idx0, bool even, bool (&keep)[4]) {
+  const uint64_t c = idx0 >> 1;
+  const uint64_t z0 = splitmix64(d.seed, c), z1 = splitmix64(d.seed, c + 1);
+  const uint32_t w[4] = {static_cast<uint32_t>(z0), static_cast<uint32_t>(z0 >> 32), static_cast<uint32_t>(z1),
+                         static_cast<uint32_t>(z1 >> 32)};
+  if (even) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) keep[e] = w[e] >= d.threshold;
+  } else {
+    const uint32_t w4 = static_cast<uint32_t>(splitmix64(d.seed, c + 2));
+    const bool odd = idx0 & 1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) keep[e] = (odd ? (e < 3 ? w[e + 1] : w4) : w[e]) >= d.threshold;
+  }
+}
+
 }  // namespace nmb
