@@ -436,6 +436,67 @@ int nmb_adamw_step_hyper(const uint64_t* params, const uint64_t* grads, const in
                          float max_norm, float* norm_out, void* workspace, size_t workspace_bytes,
                          hipStream_t stream);
 
+/* ------------------------------------------------------------ transformer block
+ * The launch sequences of one pre-norm block (reference GPTLayer.forward,
+ * models/gpt/layer.py:91-137, and its autograd) on the kernels above, so that
+ * a block is one call forward and two backward:
+ *   n1 = RMSNorm(x); [q|k|v] = n1 Wqkv^T with RoPE on q and k; o, lse = causal
+ *   attention; h = x + o Wo^T; n2 = RMSNorm(h); [g|u] = n2 Wgu^T;
+ *   act = silu(g) * u; y = h + act Wd^T.
+ * Weights row-major and contiguous in the block's dtype: w_in, w_post
+ * [hidden]; w_qkv [(q_heads + 2 kv_heads) head_dim, hidden] (Wq, Wk, Wv rows);
+ * w_o [hidden, q_heads head_dim]; w_gu [2 ffn, hidden] (Wg, then Wu rows);
+ * w_d [hidden, ffn].  RoPE tables and positions as nmb_rope_apply; q_offset is
+ * the causal mask's query offset.  bf16 needs head_dim 64 or 128.  All other
+ * tensors are contiguous: x, n1, h, n2, y, dy, dx [T, hidden] with T = batch x
+ * seq, qkv [T, (q_heads + 2 kv_heads) head_dim], o [T, q_heads head_dim], lse
+ * fp32 [batch, q_heads, seq], gu [T, 2 ffn], act [T, ffn]. */
+typedef struct nmb_block {
+  int64_t batch, seq, hidden, q_heads, kv_heads, head_dim, ffn;
+  int64_t q_offset;
+  const void *w_in, *w_qkv, *w_o, *w_post, *w_gu, *w_d;
+  const float *cos_table, *sin_table;
+  int64_t n_pos;
+  const int32_t* positions;
+  int64_t pos_batch_stride, pos_offset;
+  float eps;
+  int dtype;
+} nmb_block;
+
+/* Workspace of nmb_block_forward / nmb_block_attention and scratch of the two
+ * backward calls, in bytes (both 16-byte aligned). */
+int nmb_block_sizes(const nmb_block* b, int64_t* forward_workspace, int64_t* backward_bytes);
+
+/* From n1: qkv (RoPE applied), o and lse. */
+int nmb_block_attention(const nmb_block* b, const void* n1, void* qkv, void* o, float* lse,
+                        void* workspace, int64_t workspace_bytes, hipStream_t stream);
+
+/* gu, act and y are nullable: without y the sequence stops after [g|u] / act,
+ * without those after n2.  act needs gu in fp32; n2 may alias n1. */
+int nmb_block_forward(const nmb_block* b, const void* x, void* n1, void* qkv, void* o, float* lse,
+                      void* h, void* n2, void* gu, void* act, void* y, void* workspace,
+                      int64_t workspace_bytes, hipStream_t stream);
+
+/* The backward in two calls that share scratch.  The first runs the MLP's, the
+ * post-attention norm's and the out projection's; without gu (nullable) it
+ * forms [g|u] again from n2.  dw_gu, dw_d and (not captured) dw_post may be
+ * written on `side` (equal to stream: one stream); the caller joins it
+ * (nmb_stream_join) before they are read or scratch is freed.  captured:
+ * the queueing order for HIP graphs. */
+int nmb_block_backward_mlp(const nmb_block* b, const void* dy, const void* o, const void* h,
+                           const void* n2, const void* gu, void* dw_o, void* dw_post, void* dw_gu,
+                           void* dw_d, void* scratch, int64_t scratch_bytes, int captured,
+                           hipStream_t stream, hipStream_t side);
+
+/* The second: attention, the QKV projection and the input norm. */
+int nmb_block_backward_attention(const nmb_block* b, const void* x, const void* n1,
+                                 const void* qkv, const void* o, const float* lse, void* dx,
+                                 void* dw_in, void* dw_qkv, void* scratch, int64_t scratch_bytes,
+                                 hipStream_t stream);
+
+/* stream waits for the work queued on other so far. */
+int nmb_stream_join(hipStream_t stream, hipStream_t other);
+
 #ifdef __cplusplus
 }
 #endif

@@ -111,6 +111,12 @@ SIGNATURES: dict[str, list] = {
     "nmb_gemm_bf16_swiglu_bwd": [_i32, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p],
     "nmb_gemm_bf16_gate_up_swiglu_bwd": [_i64, _i64, _i64, _p, _i64, _p, _i64, _i64, _p, _i64, _i32, _p, _i64,
                                          _p, _i64, _p, _i64, _p],
+    "nmb_block_sizes": [_p, _pi64, _pi64],
+    "nmb_block_attention": [_p, _p, _p, _p, _p, _p, _i64, _p],
+    "nmb_block_forward": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _p],
+    "nmb_block_backward_mlp": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i32, _p, _p],
+    "nmb_block_backward_attention": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _p],
+    "nmb_stream_join": [_p, _p],
     "nmb_adamw_workspace_bytes": [_i64, _psz],
     "nmb_adamw_step": [
         _p, _p, _p, _i32, _i64, _p, _p, _p, _i32, _i32, _f64, _f64, _f64, _f64, _f64, _i64, _f32,
@@ -123,6 +129,19 @@ SIGNATURES: dict[str, list] = {
     ],
 }
 _RESTYPES = {"nmb_last_error": ctypes.c_char_p}
+
+
+class Block(ctypes.Structure):
+    """``nmb_block`` of include/nmb.h."""
+
+    _fields_ = [
+        ("batch", _i64), ("seq", _i64), ("hidden", _i64), ("q_heads", _i64), ("kv_heads", _i64),
+        ("head_dim", _i64), ("ffn", _i64), ("q_offset", _i64),
+        ("w_in", _p), ("w_qkv", _p), ("w_o", _p), ("w_post", _p), ("w_gu", _p), ("w_d", _p),
+        ("cos_table", _p), ("sin_table", _p), ("n_pos", _i64), ("positions", _p),
+        ("pos_batch_stride", _i64), ("pos_offset", _i64), ("eps", _f32), ("dtype", _i32),
+    ]
+
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
@@ -165,8 +184,16 @@ def check(status: int, what: str) -> None:
     raise RuntimeError(f"{what}: {message}")
 
 
+_functions: dict = {}  # entry points looked up so far
+
+
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args), name)
+    fn = _functions.get(name)
+    if fn is None:
+        fn = _functions[name] = getattr(load(), name)
+    status = fn(*args)
+    if status:
+        check(status, name)
 
 
 def dtype_code(dtype: torch.dtype) -> int:
@@ -181,7 +208,8 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 def stream_of(t: torch.Tensor) -> int:
     """Handle of torch's current HIP stream on the tensor's device."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the raw handle: a torch.cuda.Stream object around it costs microseconds per launch
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -11,6 +11,8 @@ models/gpt/layer.py:91-137):
     s = silu(n2 Wg^T) * (n2 Wu^T)            nmb_gemm_bf16_swiglu (activation in the epilogue)
     y = h + s Wd^T                           nmb_gemm_bf16 with the residual as C input
 
+enqueued by one call into csrc/block.hip (two for the backward).
+
 ``CheckpointedBlockFunction`` is the full-recompute policy of
 ``activation_checkpoint`` (nn/activation_checkpoint.py:73-100, selected by
 models/gpt/model.py:162-170, 215-233): it saves only the block input x.  Its
@@ -42,6 +44,7 @@ from typing import Any, Callable
 import torch
 from torch import Tensor
 
+from nano_megatron_amd import _lib
 from nano_megatron_amd import functional as Fn
 
 
@@ -56,6 +59,7 @@ class BlockMeta:
     sin: Tensor
     positions: Tensor | None  # int32 [S] or [B,S], or None for rope_offset + arange
     rope_offset: int | None = None  # RoPE position of token 0 without positions (default: sequence_offset)
+    keep: bool = True    # False: no backward will follow (gradients are off), so nothing is kept for one
 
     @property
     def pos_offset(self) -> int:
@@ -63,29 +67,20 @@ class BlockMeta:
 
 
 def _adjacent(ws: tuple[Tensor, ...]) -> bool:
-    """True if the row blocks ws[0], ws[1], ... lie back to back in one storage."""
+    """True if the row blocks ws[0], ws[1], ... lie back to back in memory."""
     w0 = ws[0]
     ptr = w0.data_ptr()
     for w in ws:
-        if (not w.is_contiguous() or w.dtype != w0.dtype or w.device != w0.device
-                or w.shape[1:] != w0.shape[1:] or w.data_ptr() != ptr
-                or w.untyped_storage().data_ptr() != w0.untyped_storage().data_ptr()):
+        if (w.data_ptr() != ptr or not w.is_contiguous() or w.dtype != w0.dtype or w.device != w0.device
+                or w.shape[1:] != w0.shape[1:]):
             return False
         ptr += w.numel() * w.element_size()
     return True
 
 
-def joined(ws: tuple[Tensor, ...]) -> Tensor:
-    """The row-concatenation of ws: an alias when they are adjacent, else a copy."""
-    if _adjacent(ws):
-        rows = sum(w.shape[0] for w in ws)
-        return ws[0].as_strided((rows, *ws[0].shape[1:]), ws[0].stride())
-    return torch.cat(ws)
-
-
 def pack_adjacent(params) -> None:
     """Re-home parameters as adjacent row blocks of one buffer (values and
-    Parameter objects unchanged), so ``joined`` needs no copy."""
+    Parameter objects unchanged), so the fused projections read them in place."""
     ws = tuple(p.data for p in params)
     if _adjacent(ws):
         return
@@ -100,189 +95,182 @@ def pack_adjacent(params) -> None:
             off += n
 
 
-def _qkv_views(qkv: Tensor, b: int, s: int, m: BlockMeta) -> tuple[Tensor, Tensor, Tensor]:
-    """[B*S, (Hq+2Hkv)*D] -> q [B,S,Hq,D], k, v [B,S,Hkv,D] strided views."""
-    qd = m.heads * m.head_dim
-    kd = m.kv_heads * m.head_dim
-    t = qkv.view(b, s, qkv.shape[-1])
-    q = t[:, :, :qd].unflatten(2, (m.heads, m.head_dim))
-    k = t[:, :, qd : qd + kd].unflatten(2, (m.kv_heads, m.head_dim))
-    v = t[:, :, qd + kd :].unflatten(2, (m.kv_heads, m.head_dim))
-    return q, k, v
+def _align(n: int) -> int:
+    return (n + 255) // 256 * 256
 
 
-def _attention_part(n1: Tensor, w: tuple[Tensor, ...], m: BlockMeta, b: int, s: int) -> tuple:
+class _Block:
+    """One call's ``nmb_block``: the weights checked against the block's shape
+    (the C side sees addresses only) and the tensors that must outlive the
+    launches on this stream."""
+
+    __slots__ = ("desc", "ref", "keep", "dtype", "device", "stream", "tokens", "hidden", "qd", "kd", "ffn",
+                 "forward_ws", "backward_bytes")
+
+    def __init__(self, like: Tensor, shape, w: tuple[Tensor, ...], m: BlockMeta) -> None:
+        Fn._require_gpu(like, m.cos, m.sin)
+        b, s, h = shape
+        qd, kd, f = m.heads * m.head_dim, m.kv_heads * m.head_dim, w[6].shape[0]
+        dtype, device = like.dtype, like.device
+        for t, want in zip(w, ((h,), (qd, h), (kd, h), (kd, h), (h, qd), (h,), (f, h), (f, h), (h, f))):
+            if t.shape != want:
+                raise ValueError(f"block: a weight of shape {tuple(t.shape)} where {want} is needed")
+            if t.dtype != dtype or t.device != device:
+                raise ValueError(f"block: a {t.dtype} weight on {t.device} with {dtype} activations on {device}")
+        if not all([t.is_contiguous() for t in w]):
+            w = tuple(t.contiguous() for t in w)
+        w_in, wq, wk, wv, wo, w_post, wg, wu, wd = w
+        # [Wq; Wk; Wv] and [Wg; Wu] as the model packs them, else copies
+        w_qkv = wq if _adjacent((wq, wk, wv)) else torch.cat((wq, wk, wv))
+        w_gu = wg if _adjacent((wg, wu)) else torch.cat((wg, wu))
+        pos, pos_ptr, pos_bstride = m.positions, None, 0
+        if pos is not None:
+            if pos.dtype != torch.int32:
+                raise ValueError("block: positions must be int32")
+            pos_ptr, pos_bstride = pos.data_ptr(), pos.stride(0) if pos.ndim == 2 else 0
+        self.desc = _lib.Block(
+            b, s, h, m.heads, m.kv_heads, m.head_dim, f, m.sequence_offset, w_in.data_ptr(), w_qkv.data_ptr(),
+            wo.data_ptr(), w_post.data_ptr(), w_gu.data_ptr(), wd.data_ptr(), m.cos.data_ptr(), m.sin.data_ptr(),
+            m.cos.shape[0], pos_ptr, pos_bstride, m.pos_offset, m.eps, _lib.dtype_code(dtype))
+        self.ref = _lib.ctypes.byref(self.desc)
+        self.keep = (w, w_qkv, w_gu)
+        self.dtype, self.device, self.stream = dtype, device, _lib.stream_of(like)
+        self.tokens, self.hidden, self.qd, self.kd, self.ffn = b * s, h, qd, kd, f
+        fwd, bwd = _lib.ctypes.c_int64(), _lib.ctypes.c_int64()
+        _lib.call("nmb_block_sizes", self.ref, _lib.ctypes.byref(fwd), _lib.ctypes.byref(bwd))
+        self.forward_ws, self.backward_bytes = fwd.value, bwd.value
+
+    def new(self, cols: int) -> Tensor:
+        return torch.empty(self.tokens, cols, dtype=self.dtype, device=self.device)
+
+    def bytes(self, n: int) -> Tensor:
+        return torch.empty(max(n, 16), dtype=torch.uint8, device=self.device)
+
+
+def _attention_part(n1: Tensor, w: tuple[Tensor, ...], m: BlockMeta, shape) -> tuple:
     """[q|k|v] (RoPE applied), the attention output o [B*S, Hq*D] and its lse
     from the normalised block input n1."""
-    _, wq, wk, wv = w[:4]
-    # Q/K/V projection with RoPE of q and k as the GEMM epilogue
-    qkv = Fn.mm_rope(n1, joined((wq, wk, wv)).t(), seq=s, head_dim=m.head_dim,
-                     rope_cols=(m.heads + m.kv_heads) * m.head_dim, cos=m.cos, sin=m.sin,
-                     pos_offset=m.pos_offset, positions=m.positions)
-    q, k, v = _qkv_views(qkv, b, s, m)
-    o, lse = Fn.attn_fwd_bshd(q, [k], [v], (0,), causal=True, q_offset=m.sequence_offset, scale=None)
-    return qkv, o.view(b * s, m.heads * m.head_dim), lse
-
-
-def _gate_up_part(n2: Tensor, w: tuple[Tensor, ...], *, act: bool, gu: bool) -> tuple:
-    """(s, [g|u]) of the MLP's gate/up product; one GEMM plan whether or not
-    the activation is applied in the epilogue, so [g|u] has the same bits."""
-    return Fn.mm_gate_up(n2, joined((w[6], w[7])), act=act, gu=gu)
+    blk = _Block(n1, shape, w, m)
+    qkv, o = blk.new(blk.qd + 2 * blk.kd), blk.new(blk.qd)
+    lse = torch.empty(shape[0], m.heads, shape[1], dtype=torch.float32, device=blk.device)
+    ws = blk.bytes(blk.forward_ws)
+    _lib.call("nmb_block_attention", blk.ref, n1.data_ptr(), qkv.data_ptr(), o.data_ptr(), lse.data_ptr(),
+              ws.data_ptr(), blk.forward_ws, blk.stream)
+    return qkv, o, lse
 
 
 def block_forward(x: Tensor, w: tuple[Tensor, ...], m: BlockMeta, *, recompute: bool,
                   keep_gu: bool = True, gate_up: bool = True) -> dict:
     """Run the block on x [B,S,H].  With recompute=True stop after [g|u] (no s, no y),
     or after n2 with gate_up=False (the backward then recomputes [g|u] inside its
-    fused gate/up + SwiGLU-backward GEMM).  With keep_gu=False (a forward whose
-    intermediates are dropped) the gate/up GEMM applies the activation in its
-    epilogue and [g|u] is never written."""
-    w_in, wq, wk, wv, wo, w_post, wg, wu, wd = w
+    fused gate/up + SwiGLU-backward GEMM).  With keep_gu=False the gate/up GEMM
+    applies the activation in its epilogue and (bf16) [g|u] is never written."""
+    x = x.contiguous()
     b, s, hdim = x.shape
-    x2 = x.reshape(b * s, hdim)
-    n1 = Fn.rmsnorm_fwd(x2, w_in, m.eps)
-    qkv, o2, lse = _attention_part(n1, w, m, b, s)
-    h = Fn.mm(o2, wo.t(), c=x2, beta=1.0)
-    n2 = Fn.rmsnorm_fwd(h, w_post, m.eps)
-    acts = dict(x2=x2, n1=n1, qkv=qkv, o2=o2, lse=lse, h=h, n2=n2)
-    if recompute and not gate_up:
-        return acts
-    act, gu = _gate_up_part(n2, w, act=not recompute, gu=recompute or keep_gu)
-    if gu is not None:
-        acts["gu"] = gu
-    if recompute:
-        return acts
-    acts["s"] = act
-    acts["y"] = Fn.mm(act, wd.t(), c=h, beta=1.0).view(b, s, hdim)
+    blk = _Block(x, x.shape, w, m)
+    x2 = x.view(b * s, hdim)
+    acts = dict(x2=x2, n1=blk.new(hdim), qkv=blk.new(blk.qd + 2 * blk.kd), o2=blk.new(blk.qd),
+                lse=torch.empty(b, m.heads, s, dtype=torch.float32, device=x.device), h=blk.new(hdim),
+                n2=blk.new(hdim))
+    gu = None
+    if gate_up or not recompute:
+        if recompute or keep_gu or x.dtype == torch.float32:
+            gu = blk.new(2 * blk.ffn)
+        if recompute or keep_gu:
+            acts["gu"] = gu
+        if not recompute:
+            acts["s"] = blk.new(blk.ffn)
+            acts["y"] = torch.empty_like(x)
+    ws = blk.bytes(blk.forward_ws)
+    n1, qkv, o2, lse, h, n2 = [acts[k].data_ptr() for k in ("n1", "qkv", "o2", "lse", "h", "n2")]
+    _lib.call("nmb_block_forward", blk.ref, x2.data_ptr(), n1, qkv, o2, lse, h, n2, _lib.ptr(gu),
+              _lib.ptr(acts.get("s")), _lib.ptr(acts.get("y")), ws.data_ptr(), blk.forward_ws, blk.stream)
     return acts
 
 
+def block_output(x: Tensor, w: tuple[Tensor, ...], m: BlockMeta) -> Tensor:
+    """The block's output alone: its intermediates share one scratch buffer,
+    freed on return.  Same kernels as ``block_forward``, same bits."""
+    x = x.contiguous()
+    b, s, hdim = x.shape
+    blk = _Block(x, x.shape, w, m)
+    t, es = blk.tokens, x.element_size()
+    sizes = (t * hdim * es, t * (blk.qd + 2 * blk.kd) * es, t * blk.qd * es, 4 * t * m.heads, t * hdim * es,
+             0 if x.dtype == torch.bfloat16 else 2 * t * blk.ffn * es, t * blk.ffn * es, blk.forward_ws)
+    at = [0]
+    for n in sizes:
+        at.append(at[-1] + _align(n))
+    scratch = blk.bytes(at[-1])
+    base = scratch.data_ptr()
+    n1, qkv, o, lse, h, gu, act, ws = [base + off for off in at[:-1]]
+    if x.dtype == torch.bfloat16:
+        gu = None
+    y = torch.empty_like(x)
+    _lib.call("nmb_block_forward", blk.ref, x.data_ptr(), n1, qkv, o, lse, h, n1, gu, act, y.data_ptr(), ws,
+              blk.forward_ws, blk.stream)
+    return y
+
+
 _SIDE_STREAMS: dict[int, torch.cuda.Stream] = {}
+# Multiply-adds of the larger MLP weight gradient from which a host-launched
+# backward uses the second stream: its events and waits cost ~60-100 us of host
+# and queue time, which short products do not give back.  One layer, forward and
+# backward, with / without it: 2^32.4 (1,024 tokens of hidden 1024) 517 / 442 us,
+# 2^33.4 542 / 558 us with full recompute and 494 / 458 us without, 2^34.4 781 /
+# 806 us and (hidden 768) 681 / 696 us, 2^35.4 1,139 / 1,171 us, 2^37.5 3,561 /
+# 3,625 us.
+_SIDE_MIN_MACS = 1 << 34
 
 
-class _SideProducts:
-    """Weight-gradient products on a second stream of the device.
-
-    The weight gradients of the block feed nothing else in its backward; on
-    their own stream (default priority, like every stream here) they fill the
-    CUs that the dX chain's launches leave idle (products of 128-176
-    workgroups, split-K tails).  The MLP's two run there; the out-projection's
-    and the QKV projection's stay on the main stream: the first's overlap would
-    fall on the attention backward, whose workgroups it then displaces, the
-    second's on the norm backward only, with the join then holding the next
-    layer's recompute (each measured slower on the side).  Each product waits for the work queued so far
-    on the main stream, its operands are recorded on the side stream (the
-    allocator keeps them until it is done), and ``join`` makes the main stream
-    wait for all of them before the gradients are returned (autograd may read
-    them on the main stream: accumulation, hooks).  Every kernel is
-    deterministic, so the results do not depend on the overlap.  (Letting the
-    products run on under the next layers' backward, joined by a final
-    callback of the backward pass, measured no faster.)
-
-    Where the products are queued depends on how the step is launched, as
-    measured on whole config-3 steps in one process.  Launched from the host,
-    the gate/up weight gradient is queued after the dX product that follows
-    the fused MLP backward (queued before it, it takes that product's CUs and
-    the step is 2.2% slower), and the post-attention norm's dw column sum runs
-    on the side.  Captured in a HIP graph, where every cross-stream wait is a
-    graph edge that costs device time at each replay (~13 us per layer for the
-    wait behind the dX product), the gate/up weight gradient is queued right
-    after the down projection's behind the same wait, and the column sum stays
-    on the main stream: the replayed step is 1.75% faster."""
-
-    def __init__(self, device: torch.device) -> None:
-        self.main = torch.cuda.current_stream(device)
-        side = _SIDE_STREAMS.get(device.index)
-        if side is None:
-            side = _SIDE_STREAMS[device.index] = torch.cuda.Stream(device)
-        self.side = side
-        self.used = False
-
-    def mm(self, a: Tensor, b: Tensor) -> Tensor:
-        self.side.wait_stream(self.main)
-        with torch.cuda.stream(self.side):
-            out = Fn.mm(a, b)
-        a.record_stream(self.side)
-        b.record_stream(self.side)
-        self.used = True
-        return out
-
-    def stream(self) -> torch.cuda.Stream:
-        """The side stream for work the caller enqueues there itself (joined
-        like the products)."""
-        self.used = True
-        return self.side
-
-    def join(self) -> None:
-        if self.used:
-            self.main.wait_stream(self.side)
+def _side_stream(blk: _Block, captured: bool) -> int:
+    """The stream of the MLP's weight gradients: a second one of the device (at
+    default priority, like every stream here) where the products are long enough
+    for the overlap to pay, else the block's own."""
+    if not captured and 2 * blk.tokens * blk.ffn * blk.hidden < _SIDE_MIN_MACS:
+        return blk.stream
+    side = _SIDE_STREAMS.get(blk.device.index)
+    if side is None:
+        side = _SIDE_STREAMS[blk.device.index] = torch.cuda.Stream(blk.device)
+    return side.cuda_stream
 
 
 def block_backward(acts: dict, dy: Tensor, w: tuple[Tensor, ...], m: BlockMeta, shape,
                    prefetch: Callable[[], None] | None = None) -> tuple:
     """Gradients (dx, dw_in, dWq, dWk, dWv, dWo, dw_post, dWg, dWu, dWd) of the
-    block.  ``prefetch`` (the recompute prefetch of a captured step) is called
+    block (csrc/block.hip holds the sequence and which products run on a second
+    stream).  ``prefetch`` (the recompute prefetch of a captured step) is called
     once the out-projection's products are queued, before the attention
-    backward."""
-    w_in, wq, wk, wv, wo, w_post, wg, wu, wd = w
-    b, s, hdim = shape
-    f = wg.shape[0]
-    dy2 = dy.reshape(b * s, hdim)
-    if not dy2.is_contiguous():
-        dy2 = dy2.contiguous()
-    x2, n1, qkv, o2, lse, h, n2 = (acts[k] for k in ("x2", "n1", "qkv", "o2", "lse", "h", "n2"))
-    side = _SideProducts(dy2.device)
-
-    # MLP: y = h + s Wd^T, s = silu(g) * u, [g|u] = n2 [Wg;Wu]^T
-    # ds = dY Wd and the SwiGLU backward in one GEMM (its epilogue); act feeds dWd.
-    # Without a kept [g|u] (a recomputed block) the same kernel first forms
-    # [g|u] for its tile from n2 (same bits), so the product never reaches memory.
-    if "gu" in acts:
-        dgu, act = Fn.mm_swiglu_bwd(dy2, wd, acts["gu"])
-    else:
-        dgu, act = Fn.mm_gate_up_swiglu_bwd(n2, joined((wg, wu)), dy2, wd)
-    dwd = side.mm(dy2.t(), act)
-    if torch.cuda.is_current_stream_capturing():
-        # captured: both MLP weight gradients behind one wait, the column sum
-        # on the main stream (fewer cross-stream edges in the graph)
-        dwgu = side.mm(dgu.t(), n2)
-        dn2 = Fn.mm(dgu, joined((wg, wu)))
-        dh, dw_post = Fn.rmsnorm_bwd(h, w_post, dn2, m.eps, residual_grad=dy2)
-    else:
-        dn2 = Fn.mm(dgu, joined((wg, wu)))
-        dwgu = side.mm(dgu.t(), n2)
-        # the weight gradient's column sum beside the next products (second stream)
-        dh, dw_post = Fn.rmsnorm_bwd(h, w_post, dn2, m.eps, residual_grad=dy2, dw_stream=side.stream())
-
-    # attention: h = x + o Wo^T
-    do2 = Fn.mm(dh, wo)
-    # on the main stream: beside the attention backward it measured slower
-    dwo = Fn.mm(dh.t(), o2)
-    if prefetch is not None:
-        prefetch()
-    q, k, v = _qkv_views(qkv, b, s, m)
-    dqkv = torch.empty_like(qkv)
-    dq, dk, dv = _qkv_views(dqkv, b, s, m)
-    o4 = o2.view(b, s, m.heads, m.head_dim)
-    do4 = do2.view(b, s, m.heads, m.head_dim)
-    # attention backward with the RoPE backward of q and k fused into the dq/dk stores
-    Fn.attn_bwd_rope_bshd(q, k, v, o4, do4, lse, dq, dk, dv, causal=True, q_offset=m.sequence_offset,
-                          scale=None, cos=m.cos, sin=m.sin, pos_offset=m.pos_offset,
-                          positions=m.positions)
-    dn1 = Fn.mm(dqkv, joined((wq, wk, wv)))
-    # on the main stream too: on the side it only overlaps the norm backward,
-    # and the join then holds the next layer's recompute (measured slower)
-    dwqkv = Fn.mm(dqkv.t(), n1)
-    dx, dw_in = Fn.rmsnorm_bwd(x2, w_in, dn1, m.eps, residual_grad=dh)
-    side.join()
-
-    qd = m.heads * m.head_dim
-    kd = m.kv_heads * m.head_dim
-    return (
-        dx.view(b, s, hdim), dw_in,
-        dwqkv[:qd], dwqkv[qd : qd + kd], dwqkv[qd + kd :],
-        dwo, dw_post, dwgu[:f], dwgu[f:], dwd,
-    )
+    backward.  The temporaries and gradients are allocated and freed in this
+    stream's order: the second stream joins it before this function returns or
+    raises."""
+    dy = dy.contiguous()
+    if dy.dtype != acts["x2"].dtype or tuple(dy.shape) != tuple(shape):
+        raise ValueError(f"block: a {dy.dtype} gradient of shape {tuple(dy.shape)} for a "
+                         f"{acts['x2'].dtype} output of shape {tuple(shape)}")
+    blk = _Block(dy, shape, w, m)
+    h, f, qd, kd = blk.hidden, blk.ffn, blk.qd, blk.kd
+    captured = torch.cuda.is_current_stream_capturing()
+    side = _side_stream(blk, captured)
+    new = lambda *sz: torch.empty(sz, dtype=blk.dtype, device=blk.device)  # noqa: E731
+    dx, dw_in, dwqkv, dwo = torch.empty_like(dy), new(h), new(qd + 2 * kd, h), new(h, qd)
+    dw_post, dwgu, dwd = new(h), new(2 * f, h), new(h, f)
+    scratch = blk.bytes(blk.backward_bytes)
+    gu = acts.get("gu")
+    x2, n1, qkv, o2, lse, hh, n2 = (acts[k].data_ptr() for k in ("x2", "n1", "qkv", "o2", "lse", "h", "n2"))
+    try:
+        _lib.call("nmb_block_backward_mlp", blk.ref, dy.data_ptr(), o2, hh, n2, _lib.ptr(gu), dwo.data_ptr(),
+                  dw_post.data_ptr(), dwgu.data_ptr(), dwd.data_ptr(), scratch.data_ptr(), blk.backward_bytes,
+                  1 if captured else 0, blk.stream, side)
+        if prefetch is not None:
+            prefetch()
+        _lib.call("nmb_block_backward_attention", blk.ref, x2, n1, qkv, o2, lse, dx.data_ptr(), dw_in.data_ptr(),
+                  dwqkv.data_ptr(), scratch.data_ptr(), blk.backward_bytes, blk.stream)
+    finally:
+        if side != blk.stream:
+            _lib.call("nmb_stream_join", blk.stream, side)
+    dwq, dwk, dwv = dwqkv.split((qd, kd, kd))
+    dwg, dwu = dwgu.split((f, f))
+    return dx, dw_in, dwq, dwk, dwv, dwo, dw_post, dwg, dwu, dwd
 
 
 _PREFETCH_STREAMS: dict[int, torch.cuda.Stream] = {}
@@ -334,8 +322,7 @@ class CheckpointedBlockFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx: Any, x: Tensor, meta: BlockMeta, offload: bool, *weights: Tensor) -> Tensor:
         x = x.contiguous()
-        with torch.no_grad():
-            acts = block_forward(x, weights, meta, recompute=False, keep_gu=False)
+        y = block_output(x, weights, meta)
         ctx.meta = meta
         ctx.shape = tuple(x.shape)
         ctx.offloaded = None
@@ -352,7 +339,7 @@ class CheckpointedBlockFunction(torch.autograd.Function):
         if not offload and x.is_cuda and torch.cuda.is_current_stream_capturing():
             ctx.prefetch_prev = _LAST_CHECKPOINTED.get(x.device.index)
             _LAST_CHECKPOINTED[x.device.index] = weakref.ref(ctx)
-        return acts["y"]
+        return y
 
     @staticmethod
     def backward(ctx: Any, dy: Tensor):
@@ -408,8 +395,7 @@ class SelectiveBlockFunction(torch.autograd.Function):
                 *weights: Tensor) -> Tensor:
         x = x.contiguous()
         attn_ck, mlp_ck = "attention" in ops, "mlp" in ops
-        with torch.no_grad():
-            acts = block_forward(x, weights, meta, recompute=False, keep_gu=not mlp_ck)
+        acts = block_forward(x, weights, meta, recompute=False, keep_gu=not mlp_ck)
         ctx.meta = meta
         ctx.shape = tuple(x.shape)
         ctx.ops = (attn_ck, mlp_ck)
@@ -445,7 +431,7 @@ class SelectiveBlockFunction(torch.autograd.Function):
         with torch.no_grad():
             if attn_ck:
                 acts["n1"] = ck.pop(0)
-                acts["qkv"], acts["o2"], acts["lse"] = _attention_part(acts["n1"], weights, m, b, s)
+                acts["qkv"], acts["o2"], acts["lse"] = _attention_part(acts["n1"], weights, m, ctx.shape)
             if mlp_ck:
                 # [g|u] is recomputed inside the MLP backward's GEMM
                 acts["n2"] = ck.pop(0)
@@ -458,8 +444,9 @@ class EagerBlockFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx: Any, x: Tensor, meta: BlockMeta, *weights: Tensor) -> Tensor:
-        with torch.no_grad():
-            acts = block_forward(x.contiguous(), weights, meta, recompute=False)
+        if not meta.keep:
+            return block_output(x, weights, meta)
+        acts = block_forward(x, weights, meta, recompute=False)
         ctx.meta = meta
         ctx.shape = tuple(x.shape)
         keys = ("x2", "n1", "qkv", "o2", "lse", "h", "n2", "gu")

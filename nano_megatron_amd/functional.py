@@ -28,7 +28,7 @@ IGNORE_INDEX = -100
 
 def _require_gpu(*tensors: Tensor) -> None:
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise ValueError(
                 "nano_megatron_amd runs its kernels on the GPU only; got a tensor on "
                 f"{t.device} (there is no CPU fallback)"
@@ -79,10 +79,12 @@ _GEMM_WS: dict = {}  # (layouts or "f32", m, n, k) -> split-K workspace bytes (a
 def _operand_layout(t: Tensor, rows_dim: int) -> tuple[int, int]:
     """(layout, ld) of a 2-D operand: 0 if dim 1 is contiguous (ld = stride(0)),
     1 if dim 0 is contiguous (ld = stride(1))."""
-    if t.stride(1) == 1 and (t.shape[0] == 1 or t.stride(0) >= t.shape[1]):
-        return 0, max(t.stride(0), t.shape[1])
-    if t.stride(0) == 1 and (t.shape[1] == 1 or t.stride(1) >= t.shape[0]):
-        return 1, max(t.stride(1), t.shape[0])
+    s0, s1 = t.stride()
+    rows, cols = t.shape
+    if s1 == 1 and (rows == 1 or s0 >= cols):
+        return 0, max(s0, cols)
+    if s0 == 1 and (cols == 1 or s1 >= rows):
+        return 1, max(s1, rows)
     raise ValueError("gemm operands need one contiguous dimension")
 
 
@@ -478,7 +480,8 @@ def _new_bhsd(shape_bhsd: Sequence[int], like: Tensor) -> Tensor:
 def _eff_strides(t: Tensor, dims=(0, 1, 2)) -> tuple[int, ...]:
     """Strides of the given dims with size-1 dims reported as 0 (never multiplied
     by a non-zero index, so any stride is equivalent there)."""
-    return tuple(t.stride(i) if t.shape[i] > 1 else 0 for i in dims)
+    strides, shape = t.stride(), t.shape
+    return tuple([strides[i] if shape[i] > 1 else 0 for i in dims])
 
 
 def _canonical_bhsd(t: Tensor) -> Tensor:

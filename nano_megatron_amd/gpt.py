@@ -404,6 +404,14 @@ class DenseGPTComponents:
 
 
 # ---------------------------------------------------------------- layer / model
+def _no_bias(*modules: nn.Module) -> bool:
+    for m in modules:
+        params = m._parameters  # a registered None is found here without Module.__getattr__
+        if (params["bias"] if "bias" in params else getattr(m, "bias", None)) is not None:
+            return False
+    return True
+
+
 class GPTLayer(nn.Module):
     """Pre-norm attention + SwiGLU block (models/gpt/layer.py:22-137)."""
 
@@ -427,21 +435,19 @@ class GPTLayer(nn.Module):
 
     # -- fused path
     def fusable(self) -> bool:
+        attention, mlp = self.attention, self.mlp
+        norm, post_norm = self.input_norm, self.post_attention_norm
         return (
-            isinstance(self.attention, GPTAttention)
-            and isinstance(self.mlp, GPTMLP)
-            and type(self.input_norm).__name__ == "RMSNorm"
-            and type(self.post_attention_norm).__name__ == "RMSNorm"
+            isinstance(attention, GPTAttention)
+            and isinstance(mlp, GPTMLP)
+            and type(norm).__name__ == "RMSNorm"
+            and type(post_norm).__name__ == "RMSNorm"
             and self.dropout == 0.0
-            and self.attention.dropout == 0.0
+            and attention.dropout == 0.0
             # the fused block's bf16 attention kernels take heads of 64 and 128
-            and (self.attention.head_dim in (64, 128) or self.input_norm.weight.dtype == torch.float32)
-            and all(
-                getattr(m, "bias", None) is None
-                for m in (self.attention.q_proj.linear, self.attention.k_proj.linear,
-                          self.attention.v_proj.linear, self.attention.out_proj,
-                          self.mlp.gate_proj.linear, self.mlp.up_proj.linear, self.mlp.down_proj)
-            )
+            and (attention.head_dim in (64, 128) or norm.weight.dtype == torch.float32)
+            and _no_bias(attention.q_proj.linear, attention.k_proj.linear, attention.v_proj.linear,
+                         attention.out_proj, mlp.gate_proj.linear, mlp.up_proj.linear, mlp.down_proj)
         )
 
     def block_weights(self) -> tuple[Tensor, ...]:
@@ -461,7 +467,7 @@ class GPTLayer(nn.Module):
         return BlockMeta(
             heads=a.num_heads, kv_heads=a.num_kv_heads, head_dim=a.head_dim,
             eps=float(self.input_norm.eps), sequence_offset=int(sequence_offset), cos=tab.cos,
-            sin=tab.sin, positions=plan.positions, rope_offset=plan.offset,
+            sin=tab.sin, positions=plan.positions, rope_offset=plan.offset, keep=torch.is_grad_enabled(),
         )
 
     # -- module path (reference semantics, used by selective checkpointing)
@@ -573,14 +579,20 @@ class GPTModel(nn.Module):
             if owns_lm_head else None
         )
 
-    def _pack_block_weights(self) -> None:
-        """Keep each layer's [Wq; Wk; Wv] and [Wg; Wu] adjacent in memory so the
-        fused projections read them in place (a no-op once packed)."""
+    def _pack_block_weights(self) -> list[tuple[Tensor, ...] | None]:
+        """Each layer's block weights (None: the layer runs module by module),
+        with its [Wq; Wk; Wv] and [Wg; Wu] kept adjacent in memory so the fused
+        projections read them in place (a no-op once packed)."""
+        out: list[tuple[Tensor, ...] | None] = []
         for layer in self.layers:
-            if layer.fusable():
-                a, m = layer.attention, layer.mlp
-                pack_adjacent((a.q_proj.weight, a.k_proj.weight, a.v_proj.weight))
-                pack_adjacent((m.gate_proj.weight, m.up_proj.weight))
+            if not layer.fusable():
+                out.append(None)
+                continue
+            w = layer.block_weights()
+            pack_adjacent(w[1:4])
+            pack_adjacent(w[6:8])
+            out.append(w)
+        return out
 
     def _checkpoint_layer(self, layer: GPTLayer) -> bool:
         """models/gpt/model.py:162-170."""
@@ -633,13 +645,12 @@ class GPTModel(nn.Module):
                 microbatch=microbatch_index, global_token_offset=offset, op="embedding",
             )
 
-        self._pack_block_weights()
+        fused = self._pack_block_weights()
         begin_forward_pass(hidden_states.device)
         mode = getattr(self.activation_checkpoint_config, "mode", "none")
         offload = bool(getattr(self.activation_checkpoint_config, "offload_saved_tensors", False))
-        for layer in self.layers:
-            if layer.fusable():
-                weights = layer.block_weights()
+        for layer, weights in zip(self.layers, fused):
+            if weights is not None:
                 if any(w.dtype != hidden_states.dtype for w in weights):
                     raise ValueError(
                         "the fused block computes in the parameter dtype: parameters "
