@@ -149,6 +149,15 @@ int nmb_attn_fwd_from_lse(const void* q, const void* const* k_blocks, const void
  * for bf16, the softmax LSE in base 2 (both [batch, q_heads, seq_q]). */
 int nmb_attn_bwd_workspace_bytes(int64_t batch, int64_t q_heads, int64_t seq_q, size_t* bytes);
 
+/* The same plus room for the dK/dV partial sums with which the bf16 backward
+ * divides a key tile's queries over several workgroups where there are too few
+ * key tiles to fill the GPU.  nmb_attn_bwd and nmb_attn_bwd_rope do so if their
+ * workspace has this size, and run undivided with the smaller one (the sums
+ * then round in another order). */
+int nmb_attn_bwd_workspace_bytes_split(int64_t batch, int64_t q_heads, int64_t kv_heads,
+                                       int64_t seq_q, int64_t seq_k, int64_t head_dim, int n_blocks,
+                                       int dtype, size_t* bytes);
+
 /* Backward from the saved lse: dq (overwritten), and per block dk, dv
  * (overwritten).  Deterministic: no atomics. */
 int nmb_attn_bwd(const void* q, const void* const* k_blocks, const void* const* v_blocks,

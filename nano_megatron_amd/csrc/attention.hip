@@ -21,6 +21,7 @@
 //   head loops over its query heads, so no repeat is materialised and no
 //   atomics are used (deterministic).
 // fp32 path: attention_f32.h, on the fp32 matrix core.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -674,11 +675,15 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? 2 : 1) void attn_bwd_dq_kernel(
 // of a second tile would not fit beside them).  Loops over the query heads of the GQA group and
 // over the 64-query tiles that can see these keys, with the next Q/dO tile's
 // global reads in flight during the current tile's MFMA work.
-template <int D, bool ROPE, int NW>
+//
+// SPLIT: the query-tile stream of a key tile is divided over `splits`
+// workgroups (item = split-major), whose fp32 dK and dV sums go to `partial`
+// ([split][batch, block, KV head, key][dK | dV][D]) for attn_bwd_reduce_kernel.
+template <int D, bool ROPE, int NW, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(
     const bf16* __restrict__ q, KVBlocks kv, const bf16* __restrict__ dout,
     const float* __restrict__ lse2, const float* __restrict__ delta, AttnShape p, int n_kt,
-    int items, int per_xcd, RopeGrad rg) {
+    int items, int per_xcd, RopeGrad rg, float* __restrict__ partial, int splits) {
   // KT key tiles of 16 per wave, KSTR keys apart
   constexpr int BQ = 64, KT = 128 / (16 * NW), KSTR = 16 * NW, BKW = KSTR * KT, KS = D / 32, DT = D / 16;
   static_assert(BKW == 128, "128 keys per workgroup");
@@ -694,14 +699,15 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel
   __shared__ __attribute__((aligned(1024))) bf16 sD[kStages][Tile::kElems];
   __shared__ __attribute__((aligned(256))) float sStat[kStages][NW][BQ];
 
-  const int w = xcd_item(items, per_xcd);
-  if (w < 0) return;
+  const int item = xcd_item(items, per_xcd);
+  if (item < 0) return;
+  const int w = SPLIT ? item / splits : item;
   // item = ((b * nblk + blk) * Hkv + hk) * n_pairs + pair.  At head dim 64
   // pair j covers key tiles j and n_kt - 1 - j one after the other, so under
   // causal masking every workgroup sees about the same number of query tiles
   // (the middle tile of an odd n_kt is alone); at 128 the registers of a
   // second tile's state do not fit, and a workgroup takes one key tile.
-  constexpr bool kPair = D == 64;
+  constexpr bool kPair = D == 64 && !SPLIT;
   const int n_pairs = kPair ? (n_kt + 1) / 2 : n_kt;
   const int pj = w % n_pairs;
   const int rest = w / n_pairs;
@@ -729,9 +735,15 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel
     return first_q / BQ;
   };
   const int qtb0 = qt_begin_of(0), qtb1 = n_sub == 2 ? qt_begin_of(1) : 0;
-  const int n_iter0 = group * (n_qt - qtb0);
+  // SPLIT: tiles [first, first + total) of the stream, which never wraps to a
+  // second sub-item (n_iter0 past every tile)
+  const int stream = group * (n_qt - qtb0);
+  const int part = SPLIT ? item % splits : 0;
+  const int first = SPLIT ? static_cast<int>(static_cast<int64_t>(part) * stream / splits) : 0;
+  const int n_iter0 = SPLIT ? 0x7fffffff : stream;
   const int n_iter1 = n_sub == 2 ? group * (n_qt - qtb1) : 0;
-  const int total = n_iter0 + n_iter1;
+  const int total = SPLIT ? static_cast<int>(static_cast<int64_t>(part + 1) * stream / splits) - first
+                          : n_iter0 + n_iter1;
 
   const int64_t kv_off = b * p.kv_sb + hk * p.kv_sh;
   const bf16* kb = static_cast<const bf16*>(kv.k[blk]) + kv_off;
@@ -762,6 +774,23 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel
   };
   // lane holds dK[key = kbase + KSTR j + 4 g + e][d = 16 dt + l16]
   auto finish = [&]() {
+    if constexpr (SPLIT) {
+      const int64_t row0 = ((static_cast<int64_t>(part) * p.B + b) * p.nblk + blk) * p.Hkv + hk;
+#pragma unroll
+      for (int j = 0; j < KT; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = kbase + KSTR * j + g * 4 + e;
+          if (key >= p.Sk) continue;
+          float* r = partial + (row0 * p.Sk + key) * (2 * D) + l16;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+            r[dt * 16] = dka[j][dt][e];
+            r[D + dt * 16] = dva[j][dt][e];
+          }
+        }
+      return;
+    }
     if constexpr (ROPE) {
       // d = 16 dt + l16 and d + D/2 are dt and dt + DT/2 (one K/V block: key =
       // token index).  Every cos/sin value is loaded and every output computed
@@ -826,7 +855,7 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel
   // sub-item's tiles qtb0 .. n_qt - 1 of each head of the group in turn, then
   // from stream tile n_iter0 on the second's from qtb1.  The loads and the
   // compute each walk it one tile per step (no division per iteration).
-  const int qt_first = n_iter0 > 0 ? qtb0 : qtb1;
+  const int qt_first = SPLIT ? (total > 0 ? qtb0 + first % (n_qt - qtb0) : 0) : n_iter0 > 0 ? qtb0 : qtb1;
   auto step_qt = [&](int next, int& qt) {  // qt of stream tile next, from that of next - 1
     const bool wrap = next == n_iter0 || qt + 1 == n_qt;
     qt = wrap ? (next < n_iter0 ? qtb0 : qtb1) : qt + 1;
@@ -839,7 +868,7 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel
   ldo.init(p.o_ss, wave, lane);
   const uint32_t q_bytes = static_cast<uint32_t>(((p.Sq - 1) * p.q_ss + D) * 2);
   const uint32_t o_bytes = static_cast<uint32_t>(((p.Sq - 1) * p.o_ss + D) * 2);
-  int l_ih = 0, l_qt = qt_first;  // the next tile to load
+  int l_ih = SPLIT && total > 0 ? first / (n_qt - qtb0) : 0, l_qt = qt_first;  // the next tile to load
   auto issue = [&](int it, int stage) {
     if (it < total) {
       const int h = hk * group + l_ih, q0 = l_qt * BQ;
@@ -1086,6 +1115,66 @@ __global__ __launch_bounds__(64 * NW, D == 64 ? 2 : 1) void attn_bwd_dkdv_kernel
   finish();
 }
 
+// dK and dV of a split stream: the partial sums in split order, then scale,
+// RoPE backward and rounding as the unsplit kernel's stores.  A thread takes
+// four head-dim elements of a row's first half and their partners in the second.
+template <int D, bool ROPE>
+__global__ __launch_bounds__(256) void attn_bwd_reduce_kernel(const float* __restrict__ partial, KVBlocks kv,
+                                                              AttnShape p, int splits, int64_t rows, RopeGrad rg) {
+  constexpr int TPR = D / 8;
+  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t row = idx / TPR;
+  if (row >= rows) return;
+  const int d = 4 * static_cast<int>(idx % TPR);
+  f32x4 k1 = f32x4{0.f, 0.f, 0.f, 0.f}, k2 = k1, v1 = k1, v2 = k1;
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s) {
+    const float* r = partial + (s * rows + row) * (2 * D) + d;
+    k1 += *reinterpret_cast<const f32x4*>(r);
+    k2 += *reinterpret_cast<const f32x4*>(r + D / 2);
+    v1 += *reinterpret_cast<const f32x4*>(r + D);
+    v2 += *reinterpret_cast<const f32x4*>(r + D + D / 2);
+  }
+  const int key = static_cast<int>(row % p.Sk);
+  const int64_t bk = row / p.Sk;
+  const int hk = static_cast<int>(bk % p.Hkv);
+  const int blk = static_cast<int>((bk / p.Hkv) % p.nblk);
+  const int b = static_cast<int>(bk / p.Hkv / p.nblk);
+  const int64_t off = b * p.kv_sb + hk * p.kv_sh + static_cast<int64_t>(key) * p.kv_ss + d;
+  bf16* dk = static_cast<bf16*>(kv.dk[blk]) + off;
+  bf16* dv = static_cast<bf16*>(kv.dv[blk]) + off;
+  bf16x4 ka, kb, va, vb;
+  float cw[4], sw[4];
+  bool bad = false;
+  if constexpr (ROPE) {
+    const int64_t pos = rope_pos(rg, b, key, &bad);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      cw[e] = rg.cos[pos * (D / 2) + d + e];
+      sw[e] = rg.sin[pos * (D / 2) + d + e];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if constexpr (ROPE) {
+      bf16 r1, r2;
+      rope_back(round_as<bf16>(k1[e] * p.scale), round_as<bf16>(k2[e] * p.scale), cw[e], sw[e], bad, r1, r2);
+      ka[e] = r1;
+      kb[e] = r2;
+    } else {
+      ka[e] = static_cast<bf16>(k1[e] * p.scale);
+      kb[e] = static_cast<bf16>(k2[e] * p.scale);
+    }
+    va[e] = static_cast<bf16>(v1[e]);
+    vb[e] = static_cast<bf16>(v2[e]);
+  }
+  // dK and dV rows need no alignment beyond their element's
+  __builtin_memcpy(dk, &ka, 8);
+  __builtin_memcpy(dk + D / 2, &kb, 8);
+  __builtin_memcpy(dv, &va, 8);
+  __builtin_memcpy(dv + D / 2, &vb, 8);
+}
+
 }  // namespace
 }  // namespace nmb
 
@@ -1182,6 +1271,61 @@ extern "C" int nmb_attn_fwd_from_lse(const void* q, const void* const* k_blocks,
                             dtype, stream);
 }
 
+namespace nmb {
+namespace {
+
+// Workgroups that share the query stream of a 128-key tile of the bf16 dK/dV
+// kernel (stream: the 64-query tiles of all its query heads).  Undivided, the
+// kernel lasts as long as the first key tile's stream however few tiles there
+// are (2 x 4 KV heads of 4 query heads, 1537 tokens, D 128: 104 workgroups of
+// up to 100 tiles).  Dividing costs the partial sums' traffic (1 KB or 2 KB per
+// key and split) and the paired key tiles of D 64, so it stops at two (D 128)
+// or three workgroups per slot, at 8 tiles per workgroup (2 where even that
+// leaves most of the GPU idle, 40 where the tiles alone nearly fill it).
+// Measured (whole backward, us, undivided -> divided): the shape above 290 ->
+// 148; D 128, 8 heads x 4096 310 -> 268; 32 q / 8 KV heads x 4 x 2048, D 64 376
+// -> 335; the same heads, 2 x 1000, 171 -> 82; 16 heads x 3000 168 -> 153; 4 x
+// 129 (32 q / 8 KV) 49 -> 35; left undivided: 16 x 16 heads x 512 73 (two: 113),
+// 8 x 1024 (32 q / 8 KV) 216 (three: 222).
+int dkdv_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D, int64_t nblk) {
+  const int64_t items = (Sk + 127) / 128 * Hkv * B * nblk;
+  const int64_t slots = D == 64 ? 512 : 256;  // workgroups in flight
+  if (items == 0 || items >= 2 * slots) return 1;
+  const int64_t target = D == 64 ? 3 * slots : 2 * slots;
+  const int64_t stream = Hq / Hkv * ((Sq + 63) / 64);
+  const int64_t shortest = 8 * items <= slots ? 2 : (D == 64 && items >= slots ? 40 : 8);
+  return static_cast<int>(std::max<int64_t>(
+      1, std::min<int64_t>(std::min((target + items / 2) / items, stream / shortest), 8)));
+}
+
+// bytes of the row statistics, and of the splits' partial sums behind them
+size_t bwd_stat_bytes(int64_t B, int64_t Hq, int64_t Sq) {
+  return 2 * static_cast<size_t>(B * Hq * Sq) * sizeof(float);
+}
+size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+size_t bwd_partial_bytes(int64_t B, int64_t Hkv, int64_t Sk, int64_t D, int64_t nblk, int splits) {
+  return splits > 1 ? static_cast<size_t>(splits) * B * nblk * Hkv * Sk * 2 * D * sizeof(float) : 0;
+}
+
+}  // namespace
+}  // namespace nmb
+
+extern "C" int nmb_attn_bwd_workspace_bytes_split(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
+                                                  int64_t seq_k, int64_t head_dim, int n_blocks, int dtype,
+                                                  size_t* bytes) {
+  NMB_REQUIRE(bytes != nullptr && batch >= 0 && q_heads > 0 && kv_heads > 0 && seq_q >= 0 && seq_k >= 0 &&
+                  head_dim > 0 && n_blocks >= 1,
+              "attn_bwd_workspace_bytes_split: bad args");
+  const size_t stat = nmb::bwd_stat_bytes(batch, q_heads, seq_q);
+  const int splits = dtype == NMB_BF16 && q_heads % kv_heads == 0
+                         ? nmb::dkdv_splits(batch, q_heads, kv_heads, seq_q, seq_k, head_dim, n_blocks)
+                         : 1;
+  *bytes = splits > 1 ? nmb::align256(stat) +
+                            nmb::bwd_partial_bytes(batch, kv_heads, seq_k, head_dim, n_blocks, splits)
+                      : stat;
+  return NMB_OK;
+}
+
 extern "C" int nmb_attn_bwd_workspace_bytes(int64_t batch, int64_t q_heads, int64_t seq_q,
                                             size_t* bytes) {
   NMB_REQUIRE(bytes != nullptr && batch >= 0 && q_heads >= 0 && seq_q >= 0,
@@ -1262,21 +1406,40 @@ int attn_bwd_impl(const void* q, const void* const* k_blocks,
     }
     if (seq_k > 0) {
       const int n_kt = static_cast<int>((seq_k + 127) / 128);  // 128-key tiles, two per workgroup at D 64
-      const int64_t items = static_cast<int64_t>(D == 64 ? (n_kt + 1) / 2 : n_kt) * kv_heads * batch * n_blocks;
+      // split query streams where the caller's workspace has room for the partial sums
+      int splits = dkdv_splits(batch, q_heads, kv_heads, seq_q, seq_k, D, n_blocks);
+      if (!aligned16(workspace) || workspace_bytes < align256(need) + bwd_partial_bytes(batch, kv_heads, seq_k, D, n_blocks, splits)) splits = 1;
+      float* partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + align256(need));
+      const int64_t items = static_cast<int64_t>(D == 64 && splits == 1 ? (n_kt + 1) / 2 : n_kt) * kv_heads * batch *
+                            n_blocks * splits;
       NMB_REQUIRE(items < (int64_t{1} << 30), "attn_bwd: problem too large for one launch");
       int per_xcd;
       unsigned blocks;
       xcd_grid(items, &per_xcd, &blocks);
       const RopeGrad rg = rope != nullptr ? *rope : RopeGrad{};
-#define NMB_DKDV(DD, RR, NW)                                                                            \
-  hipLaunchKernelGGL((nmb::attn_bwd_dkdv_kernel<DD, RR, NW>), dim3(blocks), dim3(64 * NW), 0, stream, qp, \
-                     kv, dp, lse2, delta, p, n_kt, static_cast<int>(items), per_xcd, rg)
-      if (D == 64) {
-        if (rope) NMB_DKDV(64, true, 4); else NMB_DKDV(64, false, 4);
+#define NMB_DKDV(DD, RR, NW, SS)                                                                            \
+  hipLaunchKernelGGL((nmb::attn_bwd_dkdv_kernel<DD, RR, NW, SS>), dim3(blocks), dim3(64 * NW), 0, stream, qp, \
+                     kv, dp, lse2, delta, p, n_kt, static_cast<int>(items), per_xcd, rg, partial, splits)
+#define NMB_REDUCE(DD, RR)                                                                              \
+  hipLaunchKernelGGL((nmb::attn_bwd_reduce_kernel<DD, RR>), dim3(reduce_blocks), dim3(256), 0, stream, partial, \
+                     kv, p, splits, rows, rg)
+      if (splits > 1) {
+        const int64_t rows = batch * n_blocks * kv_heads * seq_k;
+        const unsigned reduce_blocks = static_cast<unsigned>((rows * (D / 8) + 255) / 256);
+        if (D == 64) NMB_DKDV(64, false, 4, true); else NMB_DKDV(128, false, 8, true);
+        NMB_CHECK_LAUNCH("attn_bwd(dkdv)");
+        if (D == 64) {
+          if (rope) NMB_REDUCE(64, true); else NMB_REDUCE(64, false);
+        } else {
+          if (rope) NMB_REDUCE(128, true); else NMB_REDUCE(128, false);
+        }
+      } else if (D == 64) {
+        if (rope) NMB_DKDV(64, true, 4, false); else NMB_DKDV(64, false, 4, false);
       } else {
-        if (rope) NMB_DKDV(128, true, 8); else NMB_DKDV(128, false, 8);
+        if (rope) NMB_DKDV(128, true, 8, false); else NMB_DKDV(128, false, 8, false);
       }
 #undef NMB_DKDV
+#undef NMB_REDUCE
       NMB_CHECK_LAUNCH("attn_bwd(dkdv)");
     }
   } else {
@@ -1423,7 +1586,7 @@ extern "C" int nmb_attn_bwd_noalloc(const void* q, const void* const* k_blocks,
   const int st = scratch_for_stream(stream, &ws);
   if (st != NMB_OK) return st;
   return nmb::attn_bwd_impl(q, k_blocks, v_blocks, k_offsets, n_blocks, o, dout, lse, dq, dk_blocks,
-                            dv_blocks, ws, kNoAllocScratchBytes, batch, q_heads, kv_heads, seq_q,
+                            dv_blocks, ws, need, batch, q_heads, kv_heads, seq_q,
                             seq_k, head_dim, q_strides, kv_strides, o_strides, causal, q_offset,
                             scale, dtype, stream, nullptr);
 }

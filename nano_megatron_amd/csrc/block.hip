@@ -113,7 +113,8 @@ int backward_scratch(const nmb_block* b, const Dims& d, BwdScratch* s) {
     m[5] = std::max(gu, ds);
   }
   size_t attn = 0, norm = 0;
-  NMB_TRY(nmb_attn_bwd_workspace_bytes(b->batch, b->q_heads, b->seq, &attn));
+  NMB_TRY(nmb_attn_bwd_workspace_bytes_split(b->batch, b->q_heads, b->kv_heads, b->seq, b->seq, b->head_dim, 1,
+                                             b->dtype, &attn));
   NMB_TRY(nmb_rmsnorm_bwd_workspace_bytes(d.T, d.H, &norm));
   s->main_bytes = *std::max_element(m, m + 6);
   s->side_bytes = std::max(side[0], side[1]);

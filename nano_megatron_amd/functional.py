@@ -815,7 +815,8 @@ def attn_bwd_bshd(
     if _eff_strides(dq) != _eff_strides(q) or _eff_strides(do) != _eff_strides(o):
         raise ValueError("attention backward: dq must match q's strides and dO must match O's")
     nbytes = _lib.ctypes.c_size_t(0)
-    _lib.call("nmb_attn_bwd_workspace_bytes", b, hq, sq, _lib.ctypes.byref(nbytes))
+    _lib.call("nmb_attn_bwd_workspace_bytes_split", b, hq, hkv, sq, sk, d, len(ks), _lib.dtype_code(q.dtype),
+              _lib.ctypes.byref(nbytes))
     ws = _workspace(nbytes.value, q.device)
     _lib.call(
         "nmb_attn_bwd", q.data_ptr(), _lib.ptr_array(k.data_ptr() for k in ks),
@@ -858,7 +859,8 @@ def attn_bwd_rope_bshd(q: Tensor, k: Tensor, v: Tensor, o: Tensor, do: Tensor, l
         pos_ptr = positions.data_ptr()
         pos_bstride = positions.stride(0) if positions.ndim == 2 else 0
     nbytes = _lib.ctypes.c_size_t(0)
-    _lib.call("nmb_attn_bwd_workspace_bytes", b, hq, s, _lib.ctypes.byref(nbytes))
+    _lib.call("nmb_attn_bwd_workspace_bytes_split", b, hq, hkv, s, s, d, 1, _lib.NMB_BF16,
+              _lib.ctypes.byref(nbytes))
     ws = _workspace(nbytes.value, q.device)
     _lib.call(
         "nmb_attn_bwd_rope", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(),
