@@ -289,8 +289,12 @@ def kernel_rooflines(device, only: str | None = None) -> list[dict]:
         dout = randn(T, H)
         ids = torch.randint(0, V, (T,), device=device, generator=g)
         lm_grad, grad = randn(V, H), torch.empty(V, H, dtype=bf, device=device)
-        return lambda: Fn._lib.call("nmb_embedding_bwd", dout.data_ptr(), ids.data_ptr(), lm_grad.data_ptr(),
-                                    grad.data_ptr(), T, V, H, Fn._lib.NMB_BF16, Fn._lib.stream_of(dout))
+        nbytes = Fn._lib.ctypes.c_int64()
+        Fn._lib.call("nmb_embedding_bwd_workspace_bytes", T, V, Fn._lib.ctypes.byref(nbytes))
+        ws = torch.empty(max(nbytes.value, 16), dtype=torch.uint8, device=device)
+        return lambda: Fn._lib.call("nmb_embedding_bwd_ws", dout.data_ptr(), ids.data_ptr(), lm_grad.data_ptr(),
+                                    grad.data_ptr(), T, V, H, ws.data_ptr(), nbytes.value, Fn._lib.NMB_BF16,
+                                    Fn._lib.stream_of(dout))
 
     # --- MFMA-bound kernels: one input set
     qkv = randn(T, 3 * H)

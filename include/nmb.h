@@ -267,6 +267,13 @@ int nmb_embedding_fwd(const void* table, const int64_t* ids, void* out, int64_t 
 int nmb_embedding_bwd(const void* dout, const int64_t* ids, const void* grad_in, void* grad_out,
                       int64_t n_tokens, int64_t vocab, int64_t hidden, int dtype,
                       hipStream_t stream);
+/* The same bits with the tokens of each part of the table listed first in a
+ * workspace of nmb_embedding_bwd_workspace_bytes bytes, 16-byte aligned
+ * (nmb_embedding_bwd scans every id for every part: for few tokens). */
+int nmb_embedding_bwd_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t* bytes);
+int nmb_embedding_bwd_ws(const void* dout, const int64_t* ids, const void* grad_in, void* grad_out,
+                         int64_t n_tokens, int64_t vocab, int64_t hidden, void* workspace,
+                         int64_t workspace_bytes, int dtype, hipStream_t stream);
 
 /* ------------------------------------------------------------ cross entropy
  * replaces _VocabParallelCrossEntropy.forward/backward at TP=1

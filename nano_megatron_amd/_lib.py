@@ -87,6 +87,8 @@ SIGNATURES: dict[str, list] = {
     "nmb_dropout_add": [_p, _p, _p, _i64, _f32, _u64, _i32, _p],
     "nmb_embedding_fwd": [_p, _p, _p, _i64, _i64, _i64, _i32, _p],
     "nmb_embedding_bwd": [_p, _p, _p, _p, _i64, _i64, _i64, _i32, _p],
+    "nmb_embedding_bwd_workspace_bytes": [_i64, _i64, _pi64],
+    "nmb_embedding_bwd_ws": [_p, _p, _p, _p, _i64, _i64, _i64, _p, _i64, _i32, _p],
     "nmb_ce_fwd": [_p, _i64, _p, _i64, _i64, _i64, _p, _p, _i32, _p],
     "nmb_ce_bwd": [_p, _i64, _p, _i64, _i64, _i64, _p, _p, _i32, _p],
     "nmb_gemm_bf16_workspace_bytes": [_i32, _i32, _i64, _i64, _i64, _pi64],

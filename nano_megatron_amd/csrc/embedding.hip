@@ -8,26 +8,34 @@
 // 125-142), so the backward can take the LM head's table gradient and return
 // the sum, in the order autograd accumulates them: bf16(lm + bf16(rows)).
 //
-// Backward without atomics (deterministic): workgroup (row block, column
-// chunk) owns RV table rows x CH columns.  It takes the token ids in rounds of
-// 2048 (8 consecutive ids per thread, loaded together), lists the tokens whose
-// id falls in its rows in token order (a workgroup prefix sum of each
-// thread's hits), and once the ids are done (or the list is full) adds their
-// gradient chunks, sixteen rows' loads in flight at a time, to fp32
-// accumulators in LDS in list order, then writes its rows once.  Every output-gradient element is read by one workgroup; the ids
-// (8 bytes per token) are read by all of them from L2.
+// Backward without atomics (deterministic: a row's gradients are added in token
+// order in fp32, and rounded once).  A first launch lists, for every 32 to 256
+// table rows and every 8,192 tokens, the tokens whose id falls in the rows, in token
+// order (one workgroup each: 8 ids per thread, a prefix sum of the hits).  In
+// the second each wavefront owns 4 table rows x 256 columns and adds up rows
+// of few tokens by itself, all their gradient rows in flight together; rows of
+// more than 24 tokens are added by their workgroup, 64 gradient rows (32 KB) at
+// a time through LDS.  What bounds it: writing the table gradient, and for a
+// frequent token (6% of the tokens of text, or the padding of a batch) the
+// latency of its stages, since its additions stay in order.
+// Measured, bf16, us (before: one launch whose workgroups each walked every id
+// for their 16 rows and added 16 gradient rows at a time):
+// 8,192 Zipf tokens x 768, vocabulary 50,304: 43 (99); 8,192 x 1024, vocabulary
+// 8,192: uniform 18 (18), Zipf 40 (93); 16,384 x 1024 of which two thirds one
+// padding token: 370 (1,461); 65,536 Zipf x 1024, vocabulary 50,304: 289 (723).
+#include <type_traits>
+
 #include "common.h"
 #include "vec.h"
 
 namespace nmb {
 namespace {
 
-constexpr int RV = 16;        // table rows per workgroup
-constexpr int CH = 1024;      // columns per workgroup (4 per thread)
-constexpr int kPer = 8;       // token ids per thread per round
-constexpr int kRound = 256 * kPer;  // tokens per round
-constexpr int kList = 3072;    // listed tokens held before their rows are added (12 KB of LDS)
-constexpr int kBatch = 16;     // gradient rows loaded together
+constexpr int RV = 4;           // table rows per wavefront, one after the other
+constexpr int CW = 256;         // columns per wavefront (4 per lane)
+constexpr int kSegment = 8192;  // tokens per list
+constexpr int kHot = 24;        // more tokens than this: the row is added by the whole workgroup
+constexpr int kTokens = 1024;   // such a row's tokens held in LDS
 
 template <typename T>
 __global__ __launch_bounds__(256) void embedding_fwd_kernel(const T* __restrict__ table,
@@ -56,161 +64,306 @@ __global__ __launch_bounds__(256) void embedding_fwd_kernel(const T* __restrict_
   }
 }
 
-// 4 consecutive elements of T (8 bytes of bf16, 16 of fp32) as floats
-template <typename T>
-__device__ __forceinline__ void load4(const T* p, float (&v)[4]) {
-  if constexpr (sizeof(T) == 2) {
-    const uint2 raw = *reinterpret_cast<const uint2*>(p);
-    T e[4];
-    __builtin_memcpy(e, &raw, 8);
+// List (segment blockIdx.y, group blockIdx.x): the segment's tokens whose id is
+// in the group's rows, in token order; counts[segment][group].
+__global__ __launch_bounds__(1024) void embedding_list_kernel(const int64_t* __restrict__ ids, int64_t n_tokens,
+                                                              int64_t vocab, int* __restrict__ counts,
+                                                              int* __restrict__ lists, int row_bits) {
+  constexpr int kPer = kSegment / 1024;
+  __shared__ int totals[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t v0 = static_cast<int64_t>(blockIdx.x) << row_bits;
+  const int64_t v1 = min(v0 + (int64_t{1} << row_bits), vocab);
+  const int64_t base = static_cast<int64_t>(blockIdx.y) * kSegment;
+  const int t0 = static_cast<int>(threadIdx.x) * kPer;
+  int64_t id[kPer];
+  int hits = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = to_f32(e[i]);
-  } else {
-    const float4 raw = *reinterpret_cast<const float4*>(p);
-    v[0] = raw.x;
-    v[1] = raw.y;
-    v[2] = raw.z;
-    v[3] = raw.w;
+  for (int j = 0; j < kPer; ++j) id[j] = base + t0 + j < n_tokens ? ids[base + t0 + j] : -1;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) hits += id[j] >= v0 && id[j] < v1;
+  int incl = hits;  // inclusive prefix over the wavefront
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += y;
   }
+  if (lane == 63) totals[wave] = incl;
+  __syncthreads();
+  int pos = incl - hits;
+  for (int w = 0; w < wave; ++w) pos += totals[w];
+  const int64_t list = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+  if (threadIdx.x == 1023) counts[list] = pos + hits;
+  int* out = lists + list * kSegment;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j)
+    if (id[j] >= v0 && id[j] < v1) out[pos++] = (t0 + j) << row_bits | static_cast<int>(id[j] - v0);
 }
 
+// four consecutive elements
 template <typename T>
-__global__ __launch_bounds__(256, 2) void embedding_bwd_kernel(const T* __restrict__ dout,
-                                                               const int64_t* __restrict__ ids,
-                                                               const T* __restrict__ grad_in,
-                                                               T* __restrict__ grad_out,
-                                                               int64_t n_tokens, int64_t vocab,
-                                                               int64_t hidden) {
-  __shared__ float4 acc[RV * CH / 4];  // 64 KB: row r, this thread's 4 columns at [r * CH / 4 + thread]
-  __shared__ int list[kList];          // matching tokens in token order: token * RV + row
-  __shared__ int wave_total[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t row_blocks = (vocab + RV - 1) / RV;
-  const int64_t v0 = (blockIdx.x % row_blocks) * RV;
-  const int64_t c0 = (blockIdx.x / row_blocks) * CH;
-  const int cols = static_cast<int>(min<int64_t>(CH, hidden - c0));
-  const int c = threadIdx.x * 4;  // this thread's 4 columns
-  const int cc = c < cols ? c : 0;  // (a thread past the chunk's columns loads column 0, unused)
-#pragma unroll
-  for (int r = 0; r < RV; ++r) acc[r * (CH / 4) + threadIdx.x] = make_float4(0.f, 0.f, 0.f, 0.f);
+struct Quad;
+template <>
+struct Quad<bf16> {
+  using Raw = uint2;
+};
+template <>
+struct Quad<float> {
+  using Raw = uint4;
+};
 
-  // the tied LM head's rows of this block, loaded first: nothing depends on
-  // them until the end (rows past the table read its last row, not stored)
-  float prior[RV][4];
+template <typename T>
+__device__ __forceinline__ void unpack4(const typename Quad<T>::Raw& raw, float (&v)[4]) {
+  T e[4];
+  __builtin_memcpy(e, &raw, sizeof(e));
 #pragma unroll
-  for (int r = 0; r < RV; ++r) {
-    if (grad_in != nullptr) {
-      load4<T>(grad_in + min(v0 + r, vocab - 1) * hidden + c0 + cc, prior[r]);
-    } else {
+  for (int i = 0; i < 4; ++i) v[i] = to_f32(e[i]);
+}
+
+// LISTS: the tokens come from embedding_list_kernel's lists; else every id is
+// scanned (few tokens, or a caller without a workspace).
+template <typename T, bool LISTS>
+__global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict__ dout,
+                                                            const int64_t* __restrict__ ids,
+                                                            const T* __restrict__ grad_in,
+                                                            T* __restrict__ grad_out, int64_t n_tokens,
+                                                            int64_t vocab, int64_t hidden,
+                                                            const int* __restrict__ counts,
+                                                            const int* __restrict__ lists, int groups, int row_bits,
+                                                            int chunks) {
+  using Raw = typename Quad<T>::Raw;
+  constexpr int kStage = 128 / static_cast<int>(sizeof(T));  // gradient rows per stage of a hot row: 32 KB
+  constexpr int kPer = kStage / 4;                           // of one wavefront
+  __shared__ __attribute__((aligned(16))) T stage[kStage * CW];
+  __shared__ int tok[kTokens];
+  __shared__ int hot_rows[4], hot_state[2];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t w0 = static_cast<int64_t>(blockIdx.x) / chunks * (4 * RV);  // the workgroup's rows
+  const int64_t v0 = w0 + RV * wave;                                        // the wavefront's
+  const int64_t c0 = static_cast<int64_t>(blockIdx.x) % chunks * CW;
+  const bool in = c0 + 4 * lane < hidden;
+  const uint32_t col = in ? 4u * lane : 0u;  // (a lane past the columns loads the first ones, unused)
+  const int rows = static_cast<int>(max<int64_t>(0, min<int64_t>(RV, vocab - v0)));
+  const char* base = reinterpret_cast<const char*>(dout + c0);
+  const int64_t row_bytes = hidden * static_cast<int64_t>(sizeof(T));
+  auto grad_row = [&](int token) {
+    return *reinterpret_cast<const Raw*>(base + token * row_bytes + col * static_cast<uint32_t>(sizeof(T)));
+  };
+  // the embedding's own gradient is rounded to the table dtype before the tied
+  // LM-head gradient is added (autograd adds two gradient tensors)
+  auto finished = [&](float sum, float prior) {
+    const float mine = round_as<T>(sum);
+    return from_f32<T>(grad_in != nullptr ? add_rn(prior, mine) : mine);
+  };
+
+  Raw prior[RV];  // the tied LM head's rows of this wavefront
+  if (grad_in != nullptr) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) prior[r][e] = 0.f;
-    }
+    for (int r = 0; r < RV; ++r)
+      prior[r] = *reinterpret_cast<const Raw*>(grad_in + min<int64_t>(v0 + r, vocab - 1) * hidden + c0 + col);
   }
 
-  // the listed gradient rows, in token order, into the accumulators: all of
-  // a batch's loads in flight together
-  int listed = 0;  // workgroup-uniform
-  auto add_listed = [&]() {
-    if (c < cols) {
-      for (int k0 = 0; k0 < listed; k0 += kBatch) {
-        float v[kBatch][4];
-        int row[kBatch];
+  // Entry k + lane of list s of the group's rows: the row within the group
+  // (negative: none) and its token.
+  const int group = static_cast<int>(w0 >> row_bits);
+  const int64_t g0 = static_cast<int64_t>(group) << row_bits;
+  const int r0 = static_cast<int>(v0 - g0);
+  const int segments = LISTS ? static_cast<int>((n_tokens + kSegment - 1) / kSegment) : 1;
+  auto entries = [&](int s) {
+    return LISTS ? counts[static_cast<int64_t>(s) * groups + group] : static_cast<int>(n_tokens);
+  };
+  auto fetch = [&](int s, int k, int n, int& row, int& token) {
+    row = -1;
+    token = 0;
+    if (k + lane >= n) return;
+    if constexpr (LISTS) {
+      const int e = lists[(static_cast<int64_t>(s) * groups + group) * kSegment + k + lane];
+      row = e & ((1 << row_bits) - 1);
+      token = s * kSegment + (e >> row_bits);
+    } else {
+      const int64_t id = ids[k + lane];
+      if (id >= g0 && id < g0 + (1 << row_bits)) row = static_cast<int>(id - g0);
+      token = k + lane;
+    }
+  };
+
+  // how many tokens each row has
+  int cnt[RV];
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
-          const int e = list[min(k0 + u, listed - 1)];
-          row[u] = e % RV;
-          load4<T>(dout + static_cast<int64_t>(e / RV) * hidden + c0 + c, v[u]);
-        }
+  for (int r = 0; r < RV; ++r) cnt[r] = 0;
+  const int n0 = segments > 0 ? entries(0) : 0;
+  int row0 = -1, token0 = 0;  // the first entries, kept
+  fetch(0, 0, n0, row0, token0);
+  for (int s = 0; s < segments; ++s) {
+    const int n = s == 0 ? n0 : entries(s);
+    for (int k = 0; k < n; k += 64) {
+      int row = row0, token;
+      if (s != 0 || k != 0) fetch(s, k, n, row, token);
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
-          if (k0 + u < listed) {  // (no break: the loaded rows stay in registers)
-            float4& a = acc[row[u] * (CH / 4) + threadIdx.x];
-            float4 t = a;
-            t.x += v[u][0];
-            t.y += v[u][1];
-            t.z += v[u][2];
-            t.w += v[u][3];
-            a = t;
-          }
+      for (int r = 0; r < RV; ++r) cnt[r] += __popcll(__ballot(row == r0 + r));
+    }
+  }
+  int hot = 0;
+  float acc[RV][4];
+#pragma unroll
+  for (int r = 0; r < RV; ++r) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[r][e] = 0.f;
+    if (cnt[r] > kHot) {
+      hot |= 1 << r;
+      cnt[r] = 0;
+    }
+  }
+  auto add = [&](float (&a)[4], const Raw& raw) {
+    float v[4];
+    unpack4<T>(raw, v);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a[e] += v[e];
+  };
+  // the first U tokens of the mask (bit: the lane holding the token), in order
+  auto take = [&](auto width, uint64_t& mask, int token, Raw (&raw)[decltype(width)::value]) {
+    int at = 0;
+#pragma unroll
+    for (int u = 0; u < decltype(width)::value; ++u) {
+      if (mask == 0) break;
+      at = __ffsll(static_cast<unsigned long long>(mask)) - 1;
+      mask &= mask - 1;
+      raw[u] = grad_row(__builtin_amdgcn_readlane(token, at));
+    }
+  };
+  using W4 = std::integral_constant<int, 4>;
+  using W8 = std::integral_constant<int, 8>;
+  // rows of up to kHot tokens, 64 entries at a time: the first four tokens of
+  // every row loaded together
+  int left = (cnt[0] + cnt[1]) + (cnt[2] + cnt[3]);
+  for (int s = 0; s < segments && left > 0; ++s) {
+    const int n = s == 0 ? n0 : entries(s);
+    for (int k = 0; k < n && left > 0; k += 64) {
+      int row = row0, token = token0;
+      if (s != 0 || k != 0) fetch(s, k, n, row, token);
+      uint64_t mask[RV];
+      int n4[RV];
+      Raw raw[RV][4];
+#pragma unroll
+      for (int r = 0; r < RV; ++r) {
+        mask[r] = cnt[r] > 0 ? __ballot(row == r0 + r) : 0;
+        n4[r] = min(4, static_cast<int>(__popcll(mask[r])));
+        left -= static_cast<int>(__popcll(mask[r]));
+        take(W4{}, mask[r], token, raw[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < RV; ++r) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (u < n4[r]) add(acc[r], raw[r][u]);
+        while (mask[r] != 0) {
+          Raw more[8];
+          const int m = min(8, static_cast<int>(__popcll(mask[r])));
+          take(W8{}, mask[r], token, more);
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+            if (u < m) add(acc[r], more[u]);
         }
       }
     }
-    listed = 0;
-  };
-
-  // the ids in rounds of kPer consecutive tokens per thread, the next round's
-  // in flight while this round's are listed; the rows are added once the
-  // list is full or the ids are done, so that their loads are not spread
-  // over the rounds one latency each
-  int64_t id[kPer], next[kPer];
-#pragma unroll
-  for (int j = 0; j < kPer; ++j) next[j] = -1;
-  auto load_ids = [&](int64_t base, int64_t (&dst)[kPer]) {
-    const int64_t t0 = base + threadIdx.x * kPer;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) dst[j] = t0 + j < n_tokens ? ids[t0 + j] : -1;
-  };
-  load_ids(0, id);
-  for (int64_t base = 0; base < n_tokens; base += kRound) {
-    if (listed > kList - kRound) {
-      // a full round may not fit: add what is listed first (every thread is
-      // past the previous round's list writes: second barrier below)
-      add_listed();
-      __syncthreads();  // every thread is done reading the list
-    }
-    const int t_off = static_cast<int>(base) + threadIdx.x * kPer;
-    int hits = 0;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) hits += id[j] >= v0 && id[j] < v0 + RV;
-    // exclusive prefix of the hits over the workgroup (thread order = token order)
-    int incl = hits;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int y = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += y;
-    }
-    if (lane == 63) wave_total[wave] = incl;
-    __syncthreads();  // wave totals ready
-    int pos = listed + incl - hits;
-    for (int w = 0; w < wave; ++w) pos += wave_total[w];
-    const int total = wave_total[0] + wave_total[1] + wave_total[2] + wave_total[3];
-#pragma unroll
-    for (int j = 0; j < kPer; ++j)
-      if (id[j] >= v0 && id[j] < v0 + RV) list[pos++] = (t_off + j) * RV + static_cast<int>(id[j] - v0);
-    listed += total;
-    __syncthreads();  // the round's list entries are visible; wave totals read
-    if (base + kRound < n_tokens) load_ids(base + kRound, next);
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) id[j] = next[j];
   }
-  add_listed();
-  __syncthreads();
-  if (c >= cols) return;
 #pragma unroll
   for (int r = 0; r < RV; ++r) {
-    if (v0 + r >= vocab) break;
-    const int64_t o = (v0 + r) * hidden + c0 + c;
-    const float4 a4 = acc[r * (CH / 4) + threadIdx.x];
-    const float av[4] = {a4.x, a4.y, a4.z, a4.w};
-    float out[4];
+    if (r >= rows || !in || (hot >> r & 1)) continue;
+    float p[4] = {0.f, 0.f, 0.f, 0.f};
+    if (grad_in != nullptr) unpack4<T>(prior[r], p);
+    T out[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      // the embedding's own gradient is rounded to the table dtype before the
-      // tied LM-head gradient is added (autograd adds two gradient tensors)
-      const float mine = round_as<T>(av[e]);
-      out[e] = grad_in != nullptr ? add_rn(prior[r][e], mine) : mine;
-    }
-    if constexpr (sizeof(T) == 2) {
-      T ov[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ov[e] = from_f32<T>(out[e]);
-      uint2 raw;
-      __builtin_memcpy(&raw, ov, 8);
-      *reinterpret_cast<uint2*>(grad_out + o) = raw;
-    } else {
-      *reinterpret_cast<float4*>(grad_out + o) = make_float4(out[0], out[1], out[2], out[3]);
-    }
+    for (int e = 0; e < 4; ++e) out[e] = finished(acc[r][e], p[e]);
+    Raw raw;
+    __builtin_memcpy(&raw, out, sizeof(out));
+    *reinterpret_cast<Raw*>(grad_out + (v0 + r) * hidden + c0 + col) = raw;
   }
+
+  // Rows of many tokens, by the whole workgroup: wavefront 0 gathers their
+  // tokens, all four load a stage of gradient rows into LDS (the next stage's
+  // loads in flight meanwhile), and each thread adds up one column in order.
+  if (lane == 0) hot_rows[wave] = hot;
+  __syncthreads();
+  int todo = hot_rows[0] | hot_rows[1] << RV | hot_rows[2] << (2 * RV) | hot_rows[3] << (3 * RV);
+  while (todo != 0) {
+    const int hr = __ffs(todo) - 1;
+    todo &= todo - 1;
+    const int64_t v = w0 + hr;
+    const int row_in_group = static_cast<int>(v - g0);
+    const int64_t cell = v * hidden + c0 + threadIdx.x;
+    const bool mine = c0 + threadIdx.x < hidden;
+    float sum = 0.f;
+    int s = 0, k = 0;  // wavefront 0's place in the lists
+    for (bool last = false; !last;) {
+      if (wave == 0) {
+        int n = 0;
+        while (s < segments && n <= kTokens - 64) {
+          const int ns = entries(s);
+          for (; k < ns && n <= kTokens - 64; k += 64) {
+            int row, token;
+            fetch(s, k, ns, row, token);
+            const uint64_t mask = __ballot(row == row_in_group);
+            if (row == row_in_group) tok[n + __popcll(mask & ((1ull << lane) - 1))] = token;
+            n += static_cast<int>(__popcll(mask));
+          }
+          if (k >= ns) {
+            ++s;
+            k = 0;
+          }
+        }
+        if (lane == 0) {
+          hot_state[0] = n;
+          hot_state[1] = s >= segments;
+        }
+      }
+      __syncthreads();
+      const int n = hot_state[0];
+      last = hot_state[1] != 0;
+      Raw next[kPer];
+      auto load = [&](int at) {
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) next[j] = grad_row(tok[min(at + wave * kPer + j, n - 1)]);
+      };
+      if (n > 0) load(0);
+      for (int at = 0; at < n; at += kStage) {
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+          *reinterpret_cast<Raw*>(&stage[(wave * kPer + j) * CW + 4 * lane]) = next[j];
+        __syncthreads();
+        if (at + kStage < n) load(at + kStage);
+        const int m = min(kStage, n - at);
+        if (m == kStage) {
+#pragma unroll 16
+          for (int i = 0; i < kStage; ++i) sum += to_f32(stage[i * CW + threadIdx.x]);
+        } else {
+          for (int i = 0; i < m; ++i) sum += to_f32(stage[i * CW + threadIdx.x]);
+        }
+        __syncthreads();
+      }
+    }
+    if (mine) grad_out[cell] = finished(sum, grad_in != nullptr ? to_f32(grad_in[cell]) : 0.f);
+  }
+}
+
+// Rows per list as a power of two: lists as short as 256 of them allow (a
+// wavefront scans its rows' list 64 entries at a time), 32 rows at least; an
+// entry holds a token of 13 bits and a row of at most 18.
+int list_row_bits(int64_t vocab) {
+  int bits = 5;
+  while (bits < 18 && ((vocab - 1) >> bits) + 1 > 256) ++bits;
+  return bits;
+}
+
+// Bytes of the counts (rounded up to 256) and lists of n_tokens ids.  Up to 64
+// tokens every wavefront scans the ids itself (one step) instead of a launch
+// for the lists (30 tokens: 5.2 us).
+int64_t list_bytes(int64_t n_tokens, int64_t vocab) {
+  if (n_tokens <= 64) return 0;
+  const int bits = list_row_bits(vocab);
+  const int64_t lists = (n_tokens + kSegment - 1) / kSegment * (((vocab - 1) >> bits) + 1);
+  return (lists * 4 + 255) / 256 * 256 + lists * kSegment * 4;
 }
 
 template <typename T>
@@ -233,15 +386,18 @@ int fwd_impl(const void* table, const int64_t* ids, void* out, int64_t n_tokens,
 
 template <typename T>
 int bwd_impl(const void* dout, const int64_t* ids, const void* grad_in, void* grad_out,
-             int64_t n_tokens, int64_t vocab, int64_t hidden, hipStream_t stream) {
+             int64_t n_tokens, int64_t vocab, int64_t hidden, void* workspace, int64_t workspace_bytes,
+             hipStream_t stream) {
   NMB_REQUIRE_SUPPORTED(hidden % 4 == 0, "embedding_bwd: hidden (%lld) must be a multiple of 4",
                         (long long)hidden);
-  const int64_t blocks = ((vocab + RV - 1) / RV) * ((hidden + CH - 1) / CH);
-  NMB_REQUIRE(blocks < (int64_t{1} << 31), "embedding_bwd: table too large");
-  // the token list holds token * RV + row in 32 bits
+  const int64_t chunks = (hidden + CW - 1) / CW;
+  const int64_t blocks = (vocab + 4 * RV - 1) / (4 * RV) * chunks;
+  const int row_bits = list_row_bits(vocab);
+  const int64_t groups = ((vocab - 1) >> row_bits) + 1;
+  NMB_REQUIRE(blocks < (int64_t{1} << 31) && chunks < (int64_t{1} << 31), "embedding_bwd: table too large");
   NMB_REQUIRE_SUPPORTED(n_tokens < (int64_t{1} << 27), "embedding_bwd: %lld tokens exceed the supported 2^27",
                         (long long)n_tokens);
-  // rows of 4 elements are read as one 8-byte (bf16) or 16-byte (fp32) access
+  // rows of 4 elements: one alignment for every dtype's accesses
   const uintptr_t align = 4 * sizeof(T) - 1;
   NMB_REQUIRE((reinterpret_cast<uintptr_t>(dout) & align) == 0 &&
                   (reinterpret_cast<uintptr_t>(grad_out) & align) == 0 &&
@@ -249,11 +405,42 @@ int bwd_impl(const void* dout, const int64_t* ids, const void* grad_in, void* gr
               "embedding_bwd: dout, grad_in and grad_out must be aligned to %d bytes",
               static_cast<int>(align + 1));
   if (blocks == 0) return NMB_OK;
-  hipLaunchKernelGGL((embedding_bwd_kernel<T>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                     stream, static_cast<const T*>(dout), ids, static_cast<const T*>(grad_in),
-                     static_cast<T*>(grad_out), n_tokens, vocab, hidden);
+  const int64_t bytes = workspace != nullptr ? list_bytes(n_tokens, vocab) : 0;
+  int* counts = nullptr;
+  int* lists = nullptr;
+  if (bytes > 0) {
+    NMB_REQUIRE(workspace_bytes >= bytes, "embedding_bwd: workspace of %lld bytes is smaller than the %lld required",
+                (long long)workspace_bytes, (long long)bytes);
+    const int64_t segments = (n_tokens + kSegment - 1) / kSegment;
+    counts = static_cast<int*>(workspace);
+    lists = counts + (segments * groups * 4 + 255) / 256 * 64;
+    hipLaunchKernelGGL(embedding_list_kernel, dim3(static_cast<unsigned>(groups), static_cast<unsigned>(segments)),
+                       dim3(1024), 0, stream, ids, n_tokens, vocab, counts, lists, row_bits);
+    NMB_CHECK_LAUNCH("embedding_bwd(lists)");
+    hipLaunchKernelGGL((embedding_bwd_kernel<T, true>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
+                       static_cast<const T*>(dout), ids, static_cast<const T*>(grad_in), static_cast<T*>(grad_out),
+                       n_tokens, vocab, hidden, counts, lists, static_cast<int>(groups), row_bits,
+                       static_cast<int>(chunks));
+  } else {
+    hipLaunchKernelGGL((embedding_bwd_kernel<T, false>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
+                       static_cast<const T*>(dout), ids, static_cast<const T*>(grad_in), static_cast<T*>(grad_out),
+                       n_tokens, vocab, hidden, counts, lists, static_cast<int>(groups), row_bits,
+                       static_cast<int>(chunks));
+  }
   NMB_CHECK_LAUNCH("embedding_bwd");
   return NMB_OK;
+}
+
+int bwd(const void* dout, const int64_t* ids, const void* grad_in, void* grad_out, int64_t n_tokens, int64_t vocab,
+        int64_t hidden, void* workspace, int64_t workspace_bytes, int dtype, hipStream_t stream) {
+  NMB_REQUIRE(dout != nullptr && ids != nullptr && grad_out != nullptr, "embedding_bwd: null argument");
+  NMB_REQUIRE(n_tokens >= 0 && vocab > 0 && hidden > 0, "embedding_bwd: invalid shape");
+  if (dtype == NMB_BF16)
+    return bwd_impl<bf16>(dout, ids, grad_in, grad_out, n_tokens, vocab, hidden, workspace, workspace_bytes, stream);
+  if (dtype == NMB_F32)
+    return bwd_impl<float>(dout, ids, grad_in, grad_out, n_tokens, vocab, hidden, workspace, workspace_bytes, stream);
+  NMB_REQUIRE_SUPPORTED(false, "embedding_bwd: unsupported dtype %d", dtype);
+  return NMB_EUNSUPPORTED;
 }
 
 }  // namespace
@@ -272,12 +459,17 @@ extern "C" int nmb_embedding_fwd(const void* table, const int64_t* ids, void* ou
 extern "C" int nmb_embedding_bwd(const void* dout, const int64_t* ids, const void* grad_in,
                                  void* grad_out, int64_t n_tokens, int64_t vocab, int64_t hidden,
                                  int dtype, hipStream_t stream) {
-  NMB_REQUIRE(dout != nullptr && ids != nullptr && grad_out != nullptr, "embedding_bwd: null argument");
-  NMB_REQUIRE(n_tokens >= 0 && vocab > 0 && hidden > 0, "embedding_bwd: invalid shape");
-  if (dtype == NMB_BF16)
-    return nmb::bwd_impl<nmb::bf16>(dout, ids, grad_in, grad_out, n_tokens, vocab, hidden, stream);
-  if (dtype == NMB_F32)
-    return nmb::bwd_impl<float>(dout, ids, grad_in, grad_out, n_tokens, vocab, hidden, stream);
-  NMB_REQUIRE_SUPPORTED(false, "embedding_bwd: unsupported dtype %d", dtype);
-  return NMB_EUNSUPPORTED;
+  return nmb::bwd(dout, ids, grad_in, grad_out, n_tokens, vocab, hidden, nullptr, 0, dtype, stream);
+}
+
+extern "C" int nmb_embedding_bwd_workspace_bytes(int64_t n_tokens, int64_t vocab, int64_t* bytes) {
+  NMB_REQUIRE(bytes != nullptr && n_tokens >= 0 && vocab > 0, "embedding_bwd_workspace_bytes: bad args");
+  *bytes = nmb::list_bytes(n_tokens, vocab);
+  return NMB_OK;
+}
+
+extern "C" int nmb_embedding_bwd_ws(const void* dout, const int64_t* ids, const void* grad_in, void* grad_out,
+                                    int64_t n_tokens, int64_t vocab, int64_t hidden, void* workspace,
+                                    int64_t workspace_bytes, int dtype, hipStream_t stream) {
+  return nmb::bwd(dout, ids, grad_in, grad_out, n_tokens, vocab, hidden, workspace, workspace_bytes, dtype, stream);
 }

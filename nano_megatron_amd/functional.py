@@ -1196,8 +1196,12 @@ class EmbeddingFunction(torch.autograd.Function):
         if ctx.tie is not None:
             grad_in, ctx.tie.grad = ctx.tie.grad, None
         grad = torch.empty(vocab, hidden, dtype=dtype, device=dout.device)
-        _lib.call("nmb_embedding_bwd", dout.data_ptr(), ids.data_ptr(), _lib.ptr(grad_in), grad.data_ptr(),
-                  ids.numel(), vocab, hidden, _lib.dtype_code(dtype), _lib.stream_of(dout))
+        nbytes = _lib.ctypes.c_int64()
+        _lib.call("nmb_embedding_bwd_workspace_bytes", ids.numel(), vocab, _lib.ctypes.byref(nbytes))
+        ws = _workspace(nbytes.value, dout.device)
+        _lib.call("nmb_embedding_bwd_ws", dout.data_ptr(), ids.data_ptr(), _lib.ptr(grad_in), grad.data_ptr(),
+                  ids.numel(), vocab, hidden, ws.data_ptr(), nbytes.value, _lib.dtype_code(dtype),
+                  _lib.stream_of(dout))
         return grad, None, None
 
 

@@ -1,0 +1,47 @@
+"""The embedding backward through its token lists, at the edges of lists, row
+groups and column chunks."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import nano_megatron_amd.functional as Fn
+from nano_megatron_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tokens,vocab,hidden", [(1, 1, 8), (64, 512, 128), (65, 17, 136), (8192, 513, 256),
+                                                 (8193, 1025, 120), (20000, 3000, 64), (600, 50257, 264)])
+@pytest.mark.parametrize("tied", [False, True])
+def test_listed_tokens_are_added_in_order(dtype, tokens, vocab, hidden, tied) -> None:
+    """A hot id over half the tokens (runs of more than a 64-entry step), ids
+    outside the table, rows without tokens: every row equals the sequential fp32
+    sum in token order, rounded, plus the tied gradient, bit for bit; so does
+    the entry without lists."""
+    g = torch.Generator(device="cuda").manual_seed(tokens + vocab)
+    ids = torch.randint(0, vocab, (tokens,), generator=g, device="cuda")
+    ids[torch.rand(tokens, generator=g, device="cuda") < 0.5] = vocab // 2
+    if tokens > 8:
+        ids[3], ids[5] = -1, vocab
+    dout = torch.randn(tokens, hidden, generator=g, device="cuda").to(dtype)
+    lm = torch.randn(vocab, hidden, generator=g, device="cuda").to(dtype) if tied else None
+    tie = Fn.TiedGrad()
+    tie.grad = lm
+    table = torch.zeros(vocab, hidden, dtype=dtype, device="cuda", requires_grad=True)
+    (got,) = torch.autograd.grad(Fn.embedding(table, ids, tie), table, dout)
+    plain = torch.empty_like(got)
+    _lib.call("nmb_embedding_bwd", dout.data_ptr(), ids.data_ptr(), _lib.ptr(lm), plain.data_ptr(), tokens, vocab,
+              hidden, _lib.dtype_code(dtype), _lib.stream_of(dout))
+    assert torch.equal(got, plain)
+    host, rows = ids.cpu().numpy(), dout.float().cpu().numpy()
+    exp = np.zeros((vocab, hidden), np.float32)
+    for v in np.unique(host[(host >= 0) & (host < vocab)]):
+        exp[v] = np.add.accumulate(rows[host == v], axis=0, dtype=np.float32)[-1]
+    exp = torch.from_numpy(exp).to(dtype)
+    if tied:
+        exp = (exp.float() + lm.cpu().float()).to(dtype)
+    assert torch.equal(got.cpu(), exp)
