@@ -480,7 +480,7 @@ typedef struct nmb_block {
 } nmb_block;
 
 /* Workspace of nmb_block_forward / nmb_block_attention and scratch of the two
- * backward calls, in bytes (both 16-byte aligned). */
+ * backward calls, in bytes (both 16-byte aligned); either may be null. */
 int nmb_block_sizes(const nmb_block* b, int64_t* forward_workspace, int64_t* backward_bytes);
 
 /* From n1: qkv (RoPE applied), o and lse. */

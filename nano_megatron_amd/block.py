@@ -104,8 +104,7 @@ class _Block:
     (the C side sees addresses only) and the tensors that must outlive the
     launches on this stream."""
 
-    __slots__ = ("desc", "ref", "keep", "dtype", "device", "stream", "tokens", "hidden", "qd", "kd", "ffn",
-                 "forward_ws", "backward_bytes")
+    __slots__ = ("desc", "ref", "keep", "dtype", "device", "stream", "tokens", "hidden", "qd", "kd", "ffn")
 
     def __init__(self, like: Tensor, shape, w: tuple[Tensor, ...], m: BlockMeta) -> None:
         Fn._require_gpu(like, m.cos, m.sin)
@@ -136,9 +135,16 @@ class _Block:
         self.keep = (w, w_qkv, w_gu)
         self.dtype, self.device, self.stream = dtype, device, _lib.stream_of(like)
         self.tokens, self.hidden, self.qd, self.kd, self.ffn = b * s, h, qd, kd, f
-        fwd, bwd = _lib.ctypes.c_int64(), _lib.ctypes.c_int64()
-        _lib.call("nmb_block_sizes", self.ref, _lib.ctypes.byref(fwd), _lib.ctypes.byref(bwd))
-        self.forward_ws, self.backward_bytes = fwd.value, bwd.value
+
+    def forward_ws(self) -> int:
+        size = _lib.ctypes.c_int64()
+        _lib.call("nmb_block_sizes", self.ref, _lib.ctypes.byref(size), None)
+        return size.value
+
+    def backward_bytes(self) -> int:
+        size = _lib.ctypes.c_int64()
+        _lib.call("nmb_block_sizes", self.ref, None, _lib.ctypes.byref(size))
+        return size.value
 
     def new(self, cols: int) -> Tensor:
         return torch.empty(self.tokens, cols, dtype=self.dtype, device=self.device)
@@ -153,9 +159,10 @@ def _attention_part(n1: Tensor, w: tuple[Tensor, ...], m: BlockMeta, shape) -> t
     blk = _Block(n1, shape, w, m)
     qkv, o = blk.new(blk.qd + 2 * blk.kd), blk.new(blk.qd)
     lse = torch.empty(shape[0], m.heads, shape[1], dtype=torch.float32, device=blk.device)
-    ws = blk.bytes(blk.forward_ws)
+    ws_bytes = blk.forward_ws()
+    ws = blk.bytes(ws_bytes)
     _lib.call("nmb_block_attention", blk.ref, n1.data_ptr(), qkv.data_ptr(), o.data_ptr(), lse.data_ptr(),
-              ws.data_ptr(), blk.forward_ws, blk.stream)
+              ws.data_ptr(), ws_bytes, blk.stream)
     return qkv, o, lse
 
 
@@ -181,10 +188,11 @@ def block_forward(x: Tensor, w: tuple[Tensor, ...], m: BlockMeta, *, recompute: 
         if not recompute:
             acts["s"] = blk.new(blk.ffn)
             acts["y"] = torch.empty_like(x)
-    ws = blk.bytes(blk.forward_ws)
+    ws_bytes = blk.forward_ws()
+    ws = blk.bytes(ws_bytes)
     n1, qkv, o2, lse, h, n2 = [acts[k].data_ptr() for k in ("n1", "qkv", "o2", "lse", "h", "n2")]
     _lib.call("nmb_block_forward", blk.ref, x2.data_ptr(), n1, qkv, o2, lse, h, n2, _lib.ptr(gu),
-              _lib.ptr(acts.get("s")), _lib.ptr(acts.get("y")), ws.data_ptr(), blk.forward_ws, blk.stream)
+              _lib.ptr(acts.get("s")), _lib.ptr(acts.get("y")), ws.data_ptr(), ws_bytes, blk.stream)
     return acts
 
 
@@ -194,9 +202,9 @@ def block_output(x: Tensor, w: tuple[Tensor, ...], m: BlockMeta) -> Tensor:
     x = x.contiguous()
     b, s, hdim = x.shape
     blk = _Block(x, x.shape, w, m)
-    t, es = blk.tokens, x.element_size()
+    t, es, ws_bytes = blk.tokens, x.element_size(), blk.forward_ws()
     sizes = (t * hdim * es, t * (blk.qd + 2 * blk.kd) * es, t * blk.qd * es, 4 * t * m.heads, t * hdim * es,
-             0 if x.dtype == torch.bfloat16 else 2 * t * blk.ffn * es, t * blk.ffn * es, blk.forward_ws)
+             0 if x.dtype == torch.bfloat16 else 2 * t * blk.ffn * es, t * blk.ffn * es, ws_bytes)
     at = [0]
     for n in sizes:
         at.append(at[-1] + _align(n))
@@ -207,7 +215,7 @@ def block_output(x: Tensor, w: tuple[Tensor, ...], m: BlockMeta) -> Tensor:
         gu = None
     y = torch.empty_like(x)
     _lib.call("nmb_block_forward", blk.ref, x.data_ptr(), n1, qkv, o, lse, h, n1, gu, act, y.data_ptr(), ws,
-              blk.forward_ws, blk.stream)
+              ws_bytes, blk.stream)
     return y
 
 
@@ -254,17 +262,18 @@ def block_backward(acts: dict, dy: Tensor, w: tuple[Tensor, ...], m: BlockMeta, 
     new = lambda *sz: torch.empty(sz, dtype=blk.dtype, device=blk.device)  # noqa: E731
     dx, dw_in, dwqkv, dwo = torch.empty_like(dy), new(h), new(qd + 2 * kd, h), new(h, qd)
     dw_post, dwgu, dwd = new(h), new(2 * f, h), new(h, f)
-    scratch = blk.bytes(blk.backward_bytes)
+    nbytes = blk.backward_bytes()
+    scratch = blk.bytes(nbytes)
     gu = acts.get("gu")
     x2, n1, qkv, o2, lse, hh, n2 = (acts[k].data_ptr() for k in ("x2", "n1", "qkv", "o2", "lse", "h", "n2"))
     try:
         _lib.call("nmb_block_backward_mlp", blk.ref, dy.data_ptr(), o2, hh, n2, _lib.ptr(gu), dwo.data_ptr(),
-                  dw_post.data_ptr(), dwgu.data_ptr(), dwd.data_ptr(), scratch.data_ptr(), blk.backward_bytes,
+                  dw_post.data_ptr(), dwgu.data_ptr(), dwd.data_ptr(), scratch.data_ptr(), nbytes,
                   1 if captured else 0, blk.stream, side)
         if prefetch is not None:
             prefetch()
         _lib.call("nmb_block_backward_attention", blk.ref, x2, n1, qkv, o2, lse, dx.data_ptr(), dw_in.data_ptr(),
-                  dwqkv.data_ptr(), scratch.data_ptr(), blk.backward_bytes, blk.stream)
+                  dwqkv.data_ptr(), scratch.data_ptr(), nbytes, blk.stream)
     finally:
         if side != blk.stream:
             _lib.call("nmb_stream_join", blk.stream, side)

@@ -169,11 +169,12 @@ char* at(void* p, int64_t bytes) { return static_cast<char*>(p) + bytes; }
 extern "C" int nmb_block_sizes(const nmb_block* b, int64_t* forward_workspace, int64_t* backward_bytes) {
   Dims d;
   NMB_TRY(block_dims(b, &d));
-  NMB_REQUIRE(forward_workspace != nullptr && backward_bytes != nullptr, "block_sizes: null output");
-  BwdScratch s;
-  NMB_TRY(forward_ws(d, forward_workspace));
-  NMB_TRY(backward_scratch(b, d, &s));
-  *backward_bytes = s.total;
+  if (forward_workspace != nullptr) NMB_TRY(forward_ws(d, forward_workspace));
+  if (backward_bytes != nullptr) {
+    BwdScratch s;
+    NMB_TRY(backward_scratch(b, d, &s));
+    *backward_bytes = s.total;
+  }
   return NMB_OK;
 }
 

@@ -1098,19 +1098,99 @@ struct Plan {
   double time;    // the estimate the plan was chosen by (seconds)
 };
 
-// Configuration and K split for an M x N x K product on 256 CUs.  Products
-// with both operands M/N-contiguous (the weight gradients) or too few output
-// tiles for the CUs use the two-workgroups-per-CU configurations with a K
-// split; the others the one-workgroup configurations.  Among those, the
-// least estimated time = rounds of workgroups over the CUs x tile time + the
-// fp32 partials written and read back (~5 TB/s).
 // Columns of one wavefront's share of a configuration's tile.
 constexpr int wave_cols(const Config& c) { return c.nw == 4 ? c.tbn / 2 : (c.tbn == 256 ? c.tbn / 4 : c.tbn / 2); }
 
+// Estimated time (us) of configuration c with the K range in `splits` parts of
+// kps: a launch's fixed time, plus rounds of workgroups x their K depth (a
+// round of the two-workgroups-per-CU configurations that leaves one per CU runs
+// at the single rate), plus the output's stores, plus for a K split the second
+// launch and the fp32 partials written and read back.  The constants are a
+// least-squares fit to 3,900 timings of every configuration and split over 170
+// shapes (50 to 8,192 tokens of hidden 768 to 2048 and the LM head's, all three
+// layouts; 8% rms): the choice it makes is 0.7% slower than the best of them on
+// average (worst 16%), against 5.5% (50%) for the rule it replaces, which split
+// K whenever tiles were fewer than CUs and gave the one-workgroup
+// configurations no K split (3000 x 2048 x 5632 NT 107 -> 82 us, 2048 x 768 x
+// 50304 NN 210 -> 174, 4096 x 1024 x 2736 NT 49 -> 38, 2127 x 1024 x 1024 NT 25
+// -> 17, 11264 x 2048 x 8192 TN 419 -> 359).
+double plan_time(int c, int64_t m, int64_t n, int64_t kps, int64_t splits, bool a_kc, bool b_kc) {
+  struct Cost {
+    double fixed, round;   // us per launch, per round after the first
+    double k[3], k_two[3]; // us per unit of k: NT, NN, TN; with two workgroups per CU
+  };
+  constexpr Cost kCost[] = {
+      {6.8, 1.5, {0.0197, 0.0193, 0.0194}, {0, 0, 0}},
+      {6.1, 0.9, {0.0117, 0.0129, 0.0150}, {0, 0, 0}},
+      {5.6, 0.2, {0.0099, 0.0102, 0.0111}, {0.0159, 0.0135, 0.0136}},
+      {6.5, 0.3, {0.0157, 0.0190, 0.0194}, {0.0235, 0.0213, 0.0221}},
+  };
+  const Config& cf = kConfigs[c];
+  const Cost& q = kCost[c];
+  const int layout = !a_kc ? 2 : (b_kc ? 0 : 1);
+  const int64_t items = ((m + cf.tbm - 1) / cf.tbm) * ((n + cf.tbn - 1) / cf.tbn) * splits;
+  const double depth = static_cast<double>(kps);
+  double t = q.fixed;
+  if (cf.nw == 8) {
+    const int64_t rounds = (items + 255) / 256;
+    t += rounds * depth * q.k[layout] + (rounds - 1) * q.round;
+  } else {
+    const int64_t full = items / 512, rest = items % 512;
+    t += full * depth * q.k_two[layout] + (full > 0 ? (full - 1) * q.round : 0.0);
+    if (rest > 0) t += depth * (rest > 256 ? q.k_two[layout] : q.k[layout]) + (full > 0 ? q.round : 0.0);
+  }
+  const double out = static_cast<double>(m) * n;
+  t += out * 2 / 4.3e6;
+  if (splits > 1) t += 3.0 + 0.22 * splits + splits * out * 8 / 7.2e6;
+  return t;
+}
+
+// Configuration and K split of a plain product: the least estimated time.  The
+// partials of a split stay within 80 MB, where they still pass through the
+// Infinity Cache (a 2-way split of 11264 x 2048 x 8192, 184 MB, took 423 us
+// against 359 unsplit).
+Plan plan_plain(int64_t m, int64_t n, int64_t k, bool a_kc, bool b_kc) {
+  // a pure function of its arguments, asked twice per product (workspace and
+  // launch) and ~1 us each: the last ones of this thread are kept
+  struct Known {
+    int64_t m = -1, n, k;
+    int layout;
+    Plan plan;
+  };
+  constexpr int kKnown = 64;
+  static thread_local Known known[kKnown];
+  const int layout = (a_kc ? 2 : 0) + (b_kc ? 1 : 0);
+  Known& slot = known[static_cast<uint64_t>(m * 31 + n * 7 + k * 3 + layout) % kKnown];
+  if (slot.m == m && slot.n == n && slot.k == k && slot.layout == layout) return slot.plan;
+  Plan best{2, 1, 0, 0.0};
+  bool any = false;
+  for (int c = 0; c < static_cast<int>(sizeof(kConfigs) / sizeof(kConfigs[0])); ++c) {
+    const int bkt = kConfigs[c].bkt;
+    const int64_t kt = std::max<int64_t>((k + bkt - 1) / bkt, 1);  // K tiles
+    for (int64_t s = 1; s <= 16; ++s) {
+      const int64_t tps = (kt + s - 1) / s;  // K tiles per split
+      if ((kt + tps - 1) / tps != s) continue;
+      if (s > 1 && (tps * bkt < 96 || s * m * n * 4 > (int64_t{80} << 20))) break;
+      const double t = plan_time(c, m, n, tps * bkt, s, a_kc, b_kc) * 1e-6;
+      if (!any || t < best.time * 0.999) {
+        any = true;
+        best = Plan{c, static_cast<int>(s), static_cast<int>(tps * bkt), t};
+      }
+    }
+  }
+  slot = Known{m, n, k, layout, best};
+  return best;
+}
+
+// Configuration for a product with an epilogue that takes whole sums (RoPE on
+// heads of rope_head_dim, or whole_k), never split along K: too few output
+// tiles for the CUs use the two-workgroups-per-CU configurations, the others
+// the one-workgroup ones; among those, the least estimated time = rounds of
+// workgroups over the CUs x tile time.  Any other product: plan_plain.
 Plan plan_for(int64_t m, int64_t n, int64_t k, bool a_kc, bool b_kc, int rope_head_dim = 0,
               bool whole_k = false) {
+  if (rope_head_dim == 0 && !whole_k) return plan_plain(m, n, k, a_kc, b_kc);
   constexpr int64_t kCUs = 256;
-  constexpr double kBytesPerS = 5e12;
   const int64_t big_tiles = ((m + 255) / 256) * ((n + 127) / 128);
   const bool small = (!a_kc && !b_kc) || big_tiles < kCUs;
   Plan best{small ? 2 : 1, 1, 0, 0.0};
@@ -1120,46 +1200,17 @@ Plan plan_for(int64_t m, int64_t n, int64_t k, bool a_kc, bool b_kc, int rope_he
   for (int pass = 0; pass < 2 && best_t < 0; ++pass) {
     for (int c = 0; c < static_cast<int>(sizeof(kConfigs) / sizeof(kConfigs[0])); ++c) {
       const Config& cf = kConfigs[c];
-      // the RoPE epilogue needs whole heads per wavefront and no K split
       if (pass == 0 && (cf.nw == 4) != small) continue;
-      if (rope_head_dim > 0 && wave_cols(cf) % rope_head_dim != 0) continue;
+      if (rope_head_dim > 0 && wave_cols(cf) % rope_head_dim != 0) continue;  // whole heads per wavefront
       if (pass == 1 && rope_head_dim == 0) continue;
       const int64_t slots = cf.nw == 4 ? 2 * kCUs : kCUs;
       const int64_t tiles = ((m + cf.tbm - 1) / cf.tbm) * ((n + cf.tbn - 1) / cf.tbn);
       const int64_t kt = std::max<int64_t>((k + cf.bkt - 1) / cf.bkt, 1);  // K tiles
-      for (int64_t s = 1; s <= (small && rope_head_dim == 0 && !whole_k ? 16 : 1); ++s) {
-        const int64_t tps = (kt + s - 1) / s;  // K tiles per split
-        const int64_t splits = (kt + tps - 1) / tps;
-        if (splits != s || (s > 1 && tps * cf.bkt < 512)) continue;
-        const int64_t rounds = (tiles * splits + slots - 1) / slots;
-        double t = static_cast<double>(rounds) * 2.0 * cf.tbm * cf.tbn * (tps * cf.bkt) / cf.rate;
-        if (splits > 1) t += static_cast<double>(splits) * m * n * 8 / kBytesPerS;
-        if (best_t < 0 || t < best_t * 0.999) {
-          best_t = t;
-          best = Plan{c, static_cast<int>(splits), static_cast<int>(tps * cf.bkt), t};
-        }
-      }
-    }
-  }
-  // Weight gradients (both operands M/N-contiguous, long K): also the 256 x 256
-  // configuration in a single round of workgroups, each split at least 1024
-  // deep; its per-workgroup rate on this layout was measured at ~5.8e12 FLOP/s
-  // (the 16-tile-row 32-deep tiles of the other family read twice the LDS
-  // bytes per MFMA through the transposing reads).
-  if (!a_kc && !b_kc && rope_head_dim == 0 && !whole_k) {
-    constexpr double kRateMN = 5.8e12;
-    const Config& cf = kConfigs[0];
-    const int64_t tiles = ((m + cf.tbm - 1) / cf.tbm) * ((n + cf.tbn - 1) / cf.tbn);
-    const int64_t kt = std::max<int64_t>((k + cf.bkt - 1) / cf.bkt, 1);
-    for (int64_t s = 1; s <= 16; ++s) {
-      const int64_t tps = (kt + s - 1) / s;
-      const int64_t splits = (kt + tps - 1) / tps;
-      if (splits != s || tiles * splits > kCUs || (s > 1 && tps * cf.bkt < 1024)) continue;
-      double t = 2.0 * cf.tbm * cf.tbn * (tps * cf.bkt) / kRateMN;
-      if (splits > 1) t += static_cast<double>(splits) * m * n * 8 / kBytesPerS;
-      if (t < best_t * 0.999) {
+      const int64_t rounds = (tiles + slots - 1) / slots;
+      const double t = static_cast<double>(rounds) * 2.0 * cf.tbm * cf.tbn * (kt * cf.bkt) / cf.rate;
+      if (best_t < 0 || t < best_t * 0.999) {
         best_t = t;
-        best = Plan{0, static_cast<int>(splits), static_cast<int>(tps * cf.bkt), t};
+        best = Plan{c, 1, static_cast<int>(kt * cf.bkt), t};
       }
     }
   }
