@@ -28,9 +28,11 @@
 // Row, column and k tails: the loads of invalid chunks get an offset past the
 // buffer's num_records, which the hardware returns as zeros.
 //
-// LDS holds S = 2-4 K-tile stages (as many as fit the workgroup's share);
-// after the barrier that publishes tile kt, the loads of tile kt + S - 1 go
-// into the stage everyone has finished reading (one barrier per K tile).
+// LDS holds S = 2-4 K-tile stages (as many as fit the workgroup's share), with
+// one barrier per K tile: in the 128-row tiles the loads of tile kt + S - 1 go
+// into the stage freed by the last tile after the barrier that publishes tile
+// kt; in the 256-row ones the barrier stands between a tile's two 32-deep
+// steps and the loads of tile kt + S follow it (see k_loop).
 // Each MFMA computes a D^T tile (B fragment as the A operand), so a lane ends
 // up with four consecutive columns of one output row; the epilogues stage the
 // tile through LDS and store whole rows.  Blocks are mapped so that the tiles
@@ -42,6 +44,7 @@
 // (deterministic) and applies alpha, beta and the bf16 rounding (or writes
 // fp32, for nmb_gemm_bf16_f32out).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "lds_dma.h"
@@ -132,19 +135,10 @@ struct Loader {
     }
   }
 
-  // loads K tile [k0, k0 + BKT) (zeros at and past k_end) into the LDS tile
-  __device__ __forceinline__ void issue(const bf16* tile, int k0, int k_end, int wave) const {
-    const uint32_t koff = static_cast<uint32_t>(k0) * kstride;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const bool ok = off[j] != kOOB && k0 + kin[j] < k_end;
-      load_lds16(rsrc, tile + 512 * (wave * kPer + j), ok ? off[j] + koff : kOOB);
-    }
-  }
-  // The same with scalar arithmetic only for a whole K tile: m0 is the LDS
-  // byte address of this wave's first 1 KB of the tile (uniform) and the K
-  // advance rides in the instruction's scalar offset; a partial last K tile
-  // zeroes its chunks past k_end per lane.
+  // Loads K tile [k0, k0 + BKT) (zeros at and past k_end) with scalar arithmetic
+  // only for a whole K tile: m0 is the LDS byte address of this wave's first
+  // 1 KB of the tile (uniform) and the K advance rides in the instruction's
+  // scalar offset; a partial last K tile zeroes its chunks past k_end per lane.
   __device__ __forceinline__ void issue_s(uint32_t m0, int k0, int k_end) const {
     const uint32_t koff = static_cast<uint32_t>(k0) * kstride;
     if (k0 + BKT <= k_end) {
@@ -157,6 +151,14 @@ struct Loader {
         load_lds16s(rsrc, m0 + 1024u * j, ok ? off[j] : kOOB, koff);
       }
     }
+  }
+  // Load j of issue_s alone, any K tile (past k_end: zeros), without a branch.
+  // The scalar offset stays inside the matrix: the hardware takes it off
+  // num_records before the range check of the lane's offset.
+  __device__ __forceinline__ void issue_one(int j, uint32_t m0, int k0, int k_end) const {
+    const bool ok = off[j] != kOOB && k0 + kin[j] < k_end;
+    const uint32_t koff = k0 < k_end ? static_cast<uint32_t>(k0) * kstride : 0u;
+    load_lds16s(rsrc, m0 + 1024u * j, ok ? off[j] : kOOB, koff);
   }
 };
 
@@ -259,6 +261,14 @@ __device__ __forceinline__ const bf16* at_byte(const void* base, uint32_t off) {
   return reinterpret_cast<const bf16*>(reinterpret_cast<const char*>(base) + off);
 }
 
+// This wave's LDS reads have completed and its loads but the latest `later`
+// have landed; then the workgroup's barrier.  One asm statement, so that no LDS
+// read moves between the wait and the barrier.
+template <int later>
+__device__ __forceinline__ void wait_tiles() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(later) : "memory");
+}
+
 // The K loop of one tile: acc[i][j] += the wave's 16 x 16 MFMA tiles of
 // op(A) op(B) over [k_begin, k_end), the operands streamed through the S LDS
 // stages (at sA + Map::a(stage), sB + Map::b(stage)) by the loaders (the
@@ -268,7 +278,7 @@ __device__ __forceinline__ const bf16* at_byte(const void* base, uint32_t off) {
 // after the barrier.  Returns with every load of the loop complete; the other
 // waves may still read the last stage.
 template <int TBM, int TBN, int NW, int BKT, bool A_KC, bool B_KC, int TM, int TN,
-          class Map = LinearStages<TBM, TBN, BKT>, class Hook = NoHook>
+          class Map = LinearStages<TBM, TBN, BKT>, class Hook = NoHook, bool PIPE = BKT == 64>
 __device__ __forceinline__ void k_loop(const Loader<TBM, A_KC, BKT, NW>& la,
                                        const Loader<TBN, B_KC, BKT, NW>& lb, bf16 (*sA)[TBM * BKT],
                                        bf16 (*sB)[TBN * BKT], f32x4 (&acc)[TM][TN], int wm, int wn,
@@ -281,81 +291,157 @@ __device__ __forceinline__ void k_loop(const Loader<TBM, A_KC, BKT, NW>& la,
   fra.init(wm, lane);
   frb.init(wn, lane);
 
-  // S - 1 K tiles in flight.  Each K tile kt: wait until this wave's loads of
-  // tile kt have landed (those of later tiles may stay in flight), barrier
-  // (everyone's have; everyone is done with the stage read last iteration),
-  // all fragment reads, the loads of tile kt + S - 1 into that freed stage,
-  // then the MFMAs.
-  constexpr int kLoads = Loader<TBM, A_KC, BKT, NW>::kPer + Loader<TBN, B_KC, BKT, NW>::kPer;
+  constexpr int kLoadsA = Loader<TBM, A_KC, BKT, NW>::kPer;
+  constexpr int kLoads = kLoadsA + Loader<TBN, B_KC, BKT, NW>::kPer;
   const int nk = (k_end - k_begin + BKT - 1) / BKT;
-  // scalar load issue (fewer VALU instructions in the loop): 1-4% faster on
-  // the 256 x 128 and 128-row tiles, 2-4% slower on 256 x 256 (measured)
-  constexpr bool kScalarIssue = !(TBM == 256 && TBN == 256);
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const uint32_t a_lds = lds_offset(&sA[0][0]) + 1024u * wave_u * Loader<TBM, A_KC, BKT, NW>::kPer;
   const uint32_t b_lds = lds_offset(&sB[0][0]) + 1024u * wave_u * Loader<TBN, B_KC, BKT, NW>::kPer;
   auto issue = [&](int kt) {
     const int st = kt % S;
-    if constexpr (kScalarIssue) {
-      la.issue_s(a_lds + Map::a(st), k_begin + kt * BKT, k_end);
-      lb.issue_s(b_lds + Map::b(st), k_begin + kt * BKT, k_end);
-    } else {
-      la.issue(at_byte(&sA[0][0], Map::a(st)), k_begin + kt * BKT, k_end, wave);
-      lb.issue(at_byte(&sB[0][0], Map::b(st)), k_begin + kt * BKT, k_end, wave);
-    }
+    la.issue_s(a_lds + Map::a(st), k_begin + kt * BKT, k_end);
+    lb.issue_s(b_lds + Map::b(st), k_begin + kt * BKT, k_end);
   };
+  if constexpr (PIPE) {
+    // S K tiles in flight and the fragments of the next 32-deep step always
+    // being read while the MFMAs of this one run, across the K tiles too: with
+    // the second step's fragments in registers a K tile's stage is free, so the
+    // one barrier per K tile stands between the two steps, the loads of tile
+    // kt + S go out behind it, one after every few MFMAs, and a tile has a
+    // whole iteration to arrive.  (Reading both steps after the barrier left
+    // the MFMAs waiting for the first step's reads in every K tile and the fill
+    // half an iteration: a K tile took 1.5 us against 0.85 us of MFMAs.  With
+    // the loads all right behind the barrier, or the reads placed by scheduling
+    // hints, 1-4% slower.)  Loads past the last K tile are issued as well, out
+    // of range (zeros into a stage nobody reads), so that the waits are constant
+    // and the loop has no branch; with a hook, whose loads own the other stages
+    // by then, they are not.  Measured on 256 x 256 tiles, before -> after in one
+    // run: 8192^3 NT 925 -> 822 us, 2048 x 50304 x 1536 NT 360 -> 320, 2048 x
+    // 768 x 50304 NN in 8 K splits 180 -> 159, 50304 x 768 x 2048 TN 178 -> 164,
+    // 8192 x 11264 x 2048 NT 318 -> 309, 8192 x 2048 x 5632 NT 146 -> 142; on
+    // the 256 x 128 tiles (whose 8 fragment reads per 16 MFMAs bound them by
+    // LDS) 0-9%; the fused gate/up backward below 8192 x 5632 x 2048 607 -> 575.
+    constexpr bool kTail = std::is_same_v<Hook, NoHook>;
+    static_assert(KSTEPS == 2 && (kTail || S == 2), "two steps; a hook's loads follow the last wait");
+    auto read_a = [&](int st, int i, int k) { return fra.get(at_byte(&sA[0][0], Map::a(st)), i, k); };
+    auto read_b = [&](int st, int j, int k) { return frb.get(at_byte(&sB[0][0], Map::b(st)), j, k); };
+    bf16x8 fa0[TM], fb0[TN], fa1[TM], fb1[TN];
 #pragma unroll
-  for (int p = 0; p < S - 1; ++p)
-    if (p >= pre && p < nk) issue(p);
-  for (int kt = 0; kt < nk; ++kt) {
-    // tiles issued after tile kt: min(nk - 1, kt + S - 2) - kt
-    const int after = min(nk - 1, kt + S - 2) - kt;
-    if (after >= 2) wait_vmcnt<2 * kLoads>();
-    else if (after == 1) wait_vmcnt<kLoads>();
-    else wait_vmcnt<0>();
-    lds_barrier();
-    hook(kt, nk);
-    const int st = kt % S;
-    const bf16* ta = at_byte(&sA[0][0], Map::a(st));
-    const bf16* tb = at_byte(&sB[0][0], Map::b(st));
-    bf16x8 fa[KSTEPS][TM], fb[KSTEPS][TN];
+    for (int p = 0; p < S; ++p)
+      if (p >= pre && p < nk) issue(p);
+    if (nk >= S) wait_tiles<(S - 1) * kLoads>();
+    else wait_tiles<0>();
+    hook(0, nk);
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
+    for (int j = 0; j < TN; ++j) fb0[j] = read_b(0, j, 0);
 #pragma unroll
-      for (int j = 0; j < TN; ++j) fb[ks][j] = frb.get(tb, j, 32 * ks);
+    for (int i = 0; i < TM; ++i) fa0[i] = read_a(0, i, 0);
+    for (int kt = 0; kt + 1 < nk; ++kt) {
+      const int st = kt % S;
 #pragma unroll
-      for (int i = 0; i < TM; ++i) fa[ks][i] = fra.get(ta, i, 32 * ks);
-    }
-    if constexpr (KSTEPS == 2) {
-      // The wave issues in order and a full LDS queue stalls it, MFMAs
-      // included: let the step-0 MFMAs start after the step-0 reads and put one
-      // step-1 read between every two of them (scheduling hints only).
+      for (int j = 0; j < TN; ++j) fb1[j] = read_b(st, j, 32);
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < TM; ++i) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb[0][j], fa[0][i], acc[i][j]);
-      constexpr int R = TM + TN;
-      __builtin_amdgcn_sched_group_barrier(0x100, R, 0);  // step-0 LDS reads
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // two MFMAs
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one step-1 LDS read
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb0[j], fa0[i], acc[i][j]);
+        fa1[i] = read_a(st, i, 32);
       }
-      if constexpr (TM * TN > 2 * R) __builtin_amdgcn_sched_group_barrier(0x008, TM * TN - 2 * R, 0);
-      if (kt + S - 1 < nk) issue(kt + S - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      wait_tiles<(S - 2) * kLoads>();
+      hook(kt + 1, nk);
+      const int sn = (kt + 1) % S, k0 = k_begin + (kt + S) * BKT;
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int j = 0; j < TN; ++j) fb0[j] = read_b(sn, j, 0);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb[1][j], fa[1][i], acc[i][j]);
-    } else {
-      if (kt + S - 1 < nk) issue(kt + S - 1);
+      for (int i = 0; i < TM; ++i) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb1[j], fa1[i], acc[i][j]);
+        fa0[i] = read_a(sn, i, 0);
+        if (kTail || kt + S < nk) {
+          // this row's share of the loads (stage (kt + S) % S)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb[0][j], fa[0][i], acc[i][j]);
+          for (int l = 0; l < kLoads; ++l) {
+            if (l * TM / kLoads == i) {
+              if (l < kLoadsA) la.issue_one(l, a_lds + Map::a(st), k0, k_end);
+              else lb.issue_one(l - kLoadsA, b_lds + Map::b(st), k0, k_end);
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int sl = (nk - 1) % S;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) fb1[j] = read_b(sl, j, 32);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) fa1[i] = read_a(sl, i, 32);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb0[j], fa0[i], acc[i][j]);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb1[j], fa1[i], acc[i][j]);
+    if constexpr (kTail) wait_vmcnt<0>();  // the loads past the end, before the stages are used again
+  } else {
+    // S - 1 K tiles in flight.  Each K tile kt: wait until this wave's loads of
+    // tile kt have landed (those of later tiles may stay in flight), barrier
+    // (everyone's have; everyone is done with the stage read last iteration),
+    // all fragment reads, the loads of tile kt + S - 1 into that freed stage,
+    // then the MFMAs.
+#pragma unroll
+    for (int p = 0; p < S - 1; ++p)
+      if (p >= pre && p < nk) issue(p);
+    for (int kt = 0; kt < nk; ++kt) {
+      // tiles issued after tile kt: min(nk - 1, kt + S - 2) - kt
+      const int after = min(nk - 1, kt + S - 2) - kt;
+      if (after >= 2) wait_vmcnt<2 * kLoads>();
+      else if (after == 1) wait_vmcnt<kLoads>();
+      else wait_vmcnt<0>();
+      lds_barrier();
+      hook(kt, nk);
+      const int st = kt % S;
+      const bf16* ta = at_byte(&sA[0][0], Map::a(st));
+      const bf16* tb = at_byte(&sB[0][0], Map::b(st));
+      bf16x8 fa[KSTEPS][TM], fb[KSTEPS][TN];
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fb[ks][j] = frb.get(tb, j, 32 * ks);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fa[ks][i] = fra.get(ta, i, 32 * ks);
+      }
+      if constexpr (KSTEPS == 2) {
+        // The wave issues in order and a full LDS queue stalls it, MFMAs
+        // included: let the step-0 MFMAs start after the step-0 reads and put one
+        // step-1 read between every two of them (scheduling hints only).
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb[0][j], fa[0][i], acc[i][j]);
+        constexpr int R = TM + TN;
+        __builtin_amdgcn_sched_group_barrier(0x100, R, 0);  // step-0 LDS reads
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // two MFMAs
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one step-1 LDS read
+        }
+        if constexpr (TM * TN > 2 * R) __builtin_amdgcn_sched_group_barrier(0x008, TM * TN - 2 * R, 0);
+        if (kt + S - 1 < nk) issue(kt + S - 1);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb[1][j], fa[1][i], acc[i][j]);
+      } else {
+        if (kt + S - 1 < nk) issue(kt + S - 1);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(fb[0][j], fa[0][i], acc[i][j]);
+      }
     }
   }
-
 }
 
 // One workgroup's work: item L of the launch (XCD-ordered as below), on the
@@ -990,7 +1076,9 @@ __global__ __launch_bounds__(512, 1) void gemm_gu_swb_kernel(GemmArgs g1, GemmAr
     Loader<TBM, true, BKT, NW> la;
     Loader<TB2, B2_KC, BKT, NW> lb;
     init2(la, lb, lane);
-    k_loop<TBM, TB2, NW, BKT, true, B2_KC, TM, TN2, GuSwbPhase2Stages>(
+    // not pipelined: g and u fill the registers its second set of fragments needs
+    // (3-6% slower with it, spills)
+    k_loop<TBM, TB2, NW, BKT, true, B2_KC, TM, TN2, GuSwbPhase2Stages, NoHook, false>(
         la, lb, reinterpret_cast<bf16(*)[TBM * BKT]>(smem), reinterpret_cast<bf16(*)[TB2 * BKT]>(smem),
         acc2, wm, wc * WN2, 0, g2.K, wave, lane, pre2);
   }
@@ -1108,20 +1196,21 @@ constexpr int wave_cols(const Config& c) { return c.nw == 4 ? c.tbn / 2 : (c.tbn
 // launch and the fp32 partials written and read back.  The constants are a
 // least-squares fit to 3,900 timings of every configuration and split over 170
 // shapes (50 to 8,192 tokens of hidden 768 to 2048 and the LM head's, all three
-// layouts; 8% rms): the choice it makes is 0.7% slower than the best of them on
-// average (worst 16%), against 5.5% (50%) for the rule it replaces, which split
+// layouts; 8% rms): the choice it makes is 0.6% slower than the best of them on
+// average (worst 12%), against 5.5% (50%) for the rule it replaces, which split
 // K whenever tiles were fewer than CUs and gave the one-workgroup
-// configurations no K split (3000 x 2048 x 5632 NT 107 -> 82 us, 2048 x 768 x
-// 50304 NN 210 -> 174, 4096 x 1024 x 2736 NT 49 -> 38, 2127 x 1024 x 1024 NT 25
-// -> 17, 11264 x 2048 x 8192 TN 419 -> 359).
+// configurations no K split (timed before the 256-row tiles' K loop was
+// pipelined: 3000 x 2048 x 5632 NT 107 -> 82 us, 2048 x 768 x 50304 NN 210 ->
+// 174, 4096 x 1024 x 2736 NT 49 -> 38, 2127 x 1024 x 1024 NT 25 -> 17, 11264 x
+// 2048 x 8192 TN 419 -> 359).
 double plan_time(int c, int64_t m, int64_t n, int64_t kps, int64_t splits, bool a_kc, bool b_kc) {
   struct Cost {
     double fixed, round;   // us per launch, per round after the first
     double k[3], k_two[3]; // us per unit of k: NT, NN, TN; with two workgroups per CU
   };
   constexpr Cost kCost[] = {
-      {6.8, 1.5, {0.0197, 0.0193, 0.0194}, {0, 0, 0}},
-      {6.1, 0.9, {0.0117, 0.0129, 0.0150}, {0, 0, 0}},
+      {7.0, 1.8, {0.0179, 0.0181, 0.0186}, {0, 0, 0}},
+      {6.1, 1.2, {0.0111, 0.0122, 0.0141}, {0, 0, 0}},
       {5.6, 0.2, {0.0099, 0.0102, 0.0111}, {0.0159, 0.0135, 0.0136}},
       {6.5, 0.3, {0.0157, 0.0190, 0.0194}, {0.0235, 0.0213, 0.0221}},
   };
