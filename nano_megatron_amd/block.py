@@ -136,6 +136,24 @@ class _Block:
         self.dtype, self.device, self.stream = dtype, device, _lib.stream_of(like)
         self.tokens, self.hidden, self.qd, self.kd, self.ffn = b * s, h, qd, kd, f
 
+    def checked(self, acts: dict, shape, m: BlockMeta) -> dict:
+        """The activations a backward reads, contiguous: saved-tensor hooks may
+        have given back others (the C side sees addresses only)."""
+        h, n = self.hidden, self.tokens
+        wants = dict(x2=(n, h), n1=(n, h), qkv=(n, self.qd + 2 * self.kd), o2=(n, self.qd),
+                     lse=(shape[0], m.heads, shape[1]), h=(n, h), n2=(n, h), gu=(n, 2 * self.ffn))
+        out = {}
+        for name, want in wants.items():
+            t = acts.get(name)
+            if t is None and name == "gu":
+                continue
+            dtype = torch.float32 if name == "lse" else self.dtype
+            if t.shape != want or t.dtype != dtype or t.device != self.device:
+                raise ValueError(f"block: {name} saved as a {t.dtype} tensor of shape {tuple(t.shape)} on {t.device} "
+                                 f"where {dtype} of shape {want} on {self.device} is needed")
+            out[name] = t if t.is_contiguous() else t.contiguous()
+        return out
+
     def forward_ws(self) -> int:
         size = _lib.ctypes.c_int64()
         _lib.call("nmb_block_sizes", self.ref, _lib.ctypes.byref(size), None)
@@ -157,6 +175,9 @@ def _attention_part(n1: Tensor, w: tuple[Tensor, ...], m: BlockMeta, shape) -> t
     """[q|k|v] (RoPE applied), the attention output o [B*S, Hq*D] and its lse
     from the normalised block input n1."""
     blk = _Block(n1, shape, w, m)
+    if n1.shape != (blk.tokens, blk.hidden):
+        raise ValueError(f"block: n1 saved with shape {tuple(n1.shape)}")
+    n1 = n1.contiguous()
     qkv, o = blk.new(blk.qd + 2 * blk.kd), blk.new(blk.qd)
     lse = torch.empty(shape[0], m.heads, shape[1], dtype=torch.float32, device=blk.device)
     ws_bytes = blk.forward_ws()
@@ -257,6 +278,7 @@ def block_backward(acts: dict, dy: Tensor, w: tuple[Tensor, ...], m: BlockMeta, 
                          f"{acts['x2'].dtype} output of shape {tuple(shape)}")
     blk = _Block(dy, shape, w, m)
     h, f, qd, kd = blk.hidden, blk.ffn, blk.qd, blk.kd
+    acts = blk.checked(acts, shape, m)
     captured = torch.cuda.is_current_stream_capturing()
     side = _side_stream(blk, captured)
     new = lambda *sz: torch.empty(sz, dtype=blk.dtype, device=blk.device)  # noqa: E731
