@@ -9,7 +9,8 @@
 //
 // Configurations (a plan per shape picks one): 256 x 256 or 256 x 128 output
 // tiles of 8 wavefronts, one workgroup per CU, 64-deep K tiles; 128 x 128 or
-// 128 x 256 tiles of 4 wavefronts, two workgroups per CU, 32-deep K tiles.
+// 128 x 256 tiles of 4 wavefronts, two workgroups per CU, 32-deep K tiles; for
+// few rows 64 x 64 tiles of 4 wavefronts, two workgroups per CU, 64-deep K tiles.
 // Every one runs two wavefronts per SIMD: one wavefront per SIMD leaves the
 // MFMA unit idle through every LDS and barrier wait, and with the compiler's
 // accumulator allocation issues MFMAs at ~60% of the peak rate.
@@ -448,14 +449,15 @@ __device__ __forceinline__ void k_loop(const Loader<TBM, A_KC, BKT, NW>& la,
 // operand stages sA and sB in LDS.
 //
 // TBM x TBN output tile, NW wavefronts (4: 2 x 2, two workgroups per CU;
-// 8: 2 x 4 or 4 x 2, one workgroup per CU), BKT-deep K tiles.  RD > 0: RoPE
+// 8: 2 x 4 or 4 x 2, one workgroup per CU; 64-column tiles: 4 x 1), BKT-deep
+// K tiles.  RD > 0: RoPE
 // epilogue on heads of RD.  SWI: B is [2F, K] (gate rows, then up rows), N = F,
 // and D = swiglu(gate product, up product).
 template <int TBM, int TBN, int NW, int BKT, bool A_KC, bool B_KC, int RD, bool SWI, bool SWB>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int L,
                                           bf16 (*sA)[TBM * BKT],
                                           bf16 (*sB)[TBN * BKT]) {
-  constexpr int WAVES_N = NW == 4 ? 2 : (TBN == 256 ? 4 : 2);
+  constexpr int WAVES_N = NW == 4 ? (TBN == 64 ? 1 : 2) : (TBN == 256 ? 4 : 2);
   constexpr int WAVES_M = NW / WAVES_N;
   constexpr int WM = TBM / WAVES_M, WN = TBN / WAVES_N;  // wave tile
   constexpr int TM = WM / 16, TN = WN / 16;              // 16 x 16 MFMA tiles per wave
@@ -748,10 +750,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int L,
   // products with no residual add run up to 4.5% faster (bit-identical).
   constexpr int RPA = (S * TBM * BKT) / TBN;  // tile rows that fit in sA, the rest in sB
   static_assert(RPA + S * BKT >= TBM, "the bf16 tile fits in the operand stages");
-  static_assert(TBN % 128 == 0, "16-byte slots of a tile row, swizzled by 4 row bits");
+  static_assert(TBN % 128 == 0 || TBN == 64, "16-byte slots of a tile row, swizzled by 4 (3) row bits");
   auto tile_at = [&](int r, int c) -> bf16* {  // tile element (r, c), c a multiple of 4
     bf16* rp = r < RPA ? &sA[0][0] + r * TBN : &sB[0][0] + (r - RPA) * TBN;
-    return rp + 8 * ((c >> 3) ^ (r & 15)) + (c & 4);
+    return rp + 8 * ((c >> 3) ^ (r & (TBN == 64 ? 7 : 15))) + (c & 4);
   };
   __syncthreads();  // every wave is done with the operand stages
   if constexpr (RD > 0) {
@@ -1177,7 +1179,22 @@ constexpr Config kConfigs[] = {
     {256, 128, 8, 64, 3.0e12},
     {128, 128, 4, 32, 1.6e12},  // two workgroups per CU
     {128, 256, 4, 32, 1.7e12},
+    {64, 64, 4, 64, 0.6e12},  // K-contiguous operands only; see kSmall
 };
+
+// The 64 x 64 tiles, for the products of few tokens (K-contiguous operands: the
+// forward's).  What bounds those is how fast the weights reach the CUs, a chain
+// of loads per workgroup: 128 x 128 tiles of 193 x 3072 x 1024 occupy 48 of the
+// 256 CUs with twice the bytes each, and with a K split a second launch adds up
+// the partials.  Four times the workgroups with 48 KB of K tiles on the way each
+// (a wavefront takes 16 rows x 64 columns: a whole head of 64 for RoPE, 32 gate
+// and 32 up columns for SwiGLU).  Weights from HBM, 128 x 128 tiles -> these:
+// 193 x 3072 x 1024 with RoPE 17.6 -> 8.6 us, 193 x 5472 x 1024 with SwiGLU
+// 15.8 -> 10.6, 193 x 1024 x 1024 13.9 (4 K splits) -> 6.6 (unsplit), 193 x 1024
+// x 2736 14 -> 10.8, 5 x 2048 x 11264 with SwiGLU 24.7 -> 15.1; past two rounds
+// of workgroups the larger tiles' fewer operand reads win (1024 x 5472 x 1024
+// with SwiGLU 23.9 against 27.3, 2127 x 2048 x 2048 27.9 against 35.6).
+constexpr int kSmall = 4;
 
 struct Plan {
   int config;     // index into kConfigs
@@ -1187,7 +1204,7 @@ struct Plan {
 };
 
 // Columns of one wavefront's share of a configuration's tile.
-constexpr int wave_cols(const Config& c) { return c.nw == 4 ? c.tbn / 2 : (c.tbn == 256 ? c.tbn / 4 : c.tbn / 2); }
+constexpr int wave_cols(const Config& c) { return c.tbn == 64 ? 64 : c.nw == 4 ? c.tbn / 2 : (c.tbn == 256 ? c.tbn / 4 : c.tbn / 2); }
 
 // Estimated time (us) of configuration c with the K range in `splits` parts of
 // kps: a launch's fixed time, plus rounds of workgroups x their K depth (a
@@ -1202,7 +1219,8 @@ constexpr int wave_cols(const Config& c) { return c.nw == 4 ? c.tbn / 2 : (c.tbn
 // configurations no K split (timed before the 256-row tiles' K loop was
 // pipelined: 3000 x 2048 x 5632 NT 107 -> 82 us, 2048 x 768 x 50304 NN 210 ->
 // 174, 4096 x 1024 x 2736 NT 49 -> 38, 2127 x 1024 x 1024 NT 25 -> 17, 11264 x
-// 2048 x 8192 TN 419 -> 359).
+// 2048 x 8192 TN 419 -> 359).  The 64 x 64 tiles' constants are from 560 more
+// (5 to 2,127 tokens, NT, K splits of 1 to 12, weights from HBM).
 double plan_time(int c, int64_t m, int64_t n, int64_t kps, int64_t splits, bool a_kc, bool b_kc) {
   struct Cost {
     double fixed, round;   // us per launch, per round after the first
@@ -1213,6 +1231,7 @@ double plan_time(int c, int64_t m, int64_t n, int64_t kps, int64_t splits, bool 
       {6.1, 1.2, {0.0111, 0.0122, 0.0141}, {0, 0, 0}},
       {5.6, 0.2, {0.0099, 0.0102, 0.0111}, {0.0159, 0.0135, 0.0136}},
       {6.5, 0.3, {0.0157, 0.0190, 0.0194}, {0.0235, 0.0213, 0.0221}},
+      {2.9, 0.2, {0.0039, 0, 0}, {0.0075, 0, 0}},
   };
   const Config& cf = kConfigs[c];
   const Cost& q = kCost[c];
@@ -1254,6 +1273,7 @@ Plan plan_plain(int64_t m, int64_t n, int64_t k, bool a_kc, bool b_kc) {
   Plan best{2, 1, 0, 0.0};
   bool any = false;
   for (int c = 0; c < static_cast<int>(sizeof(kConfigs) / sizeof(kConfigs[0])); ++c) {
+    if (c == kSmall && !(a_kc && b_kc)) continue;
     const int bkt = kConfigs[c].bkt;
     const int64_t kt = std::max<int64_t>((k + bkt - 1) / bkt, 1);  // K tiles
     for (int64_t s = 1; s <= 16; ++s) {
@@ -1275,7 +1295,9 @@ Plan plan_plain(int64_t m, int64_t n, int64_t k, bool a_kc, bool b_kc) {
 // heads of rope_head_dim, or whole_k), never split along K: too few output
 // tiles for the CUs use the two-workgroups-per-CU configurations, the others
 // the one-workgroup ones; among those, the least estimated time = rounds of
-// workgroups over the CUs x tile time.  Any other product: plan_plain.
+// workgroups over the CUs x tile time.  Where that is a two-workgroups-per-CU
+// one, the 64 x 64 tiles replace it if plan_time rates them faster (heads of 64
+// at most: a wavefront has 64 columns).  Any other product: plan_plain.
 Plan plan_for(int64_t m, int64_t n, int64_t k, bool a_kc, bool b_kc, int rope_head_dim = 0,
               bool whole_k = false) {
   if (rope_head_dim == 0 && !whole_k) return plan_plain(m, n, k, a_kc, b_kc);
@@ -1289,7 +1311,7 @@ Plan plan_for(int64_t m, int64_t n, int64_t k, bool a_kc, bool b_kc, int rope_he
   for (int pass = 0; pass < 2 && best_t < 0; ++pass) {
     for (int c = 0; c < static_cast<int>(sizeof(kConfigs) / sizeof(kConfigs[0])); ++c) {
       const Config& cf = kConfigs[c];
-      if (pass == 0 && (cf.nw == 4) != small) continue;
+      if (c == kSmall || (pass == 0 && (cf.nw == 4) != small)) continue;
       if (rope_head_dim > 0 && wave_cols(cf) % rope_head_dim != 0) continue;  // whole heads per wavefront
       if (pass == 1 && rope_head_dim == 0) continue;
       const int64_t slots = cf.nw == 4 ? 2 * kCUs : kCUs;
@@ -1302,6 +1324,11 @@ Plan plan_for(int64_t m, int64_t n, int64_t k, bool a_kc, bool b_kc, int rope_he
         best = Plan{c, 1, static_cast<int>(kt * cf.bkt), t};
       }
     }
+  }
+  if (a_kc && b_kc && small && rope_head_dim != 128) {
+    const int64_t kps = std::max<int64_t>((k + 63) / 64, 1) * 64;
+    if (plan_time(kSmall, m, n, kps, 1, true, true) < plan_time(best.config, m, n, best.kps, 1, true, true))
+      best = Plan{kSmall, 1, static_cast<int>(kps), best.time};
   }
   return best;
 }
@@ -1337,6 +1364,8 @@ int launch(GemmArgs g, hipStream_t stream) {
   return NMB_OK;
 }
 
+int launch_small(const GemmArgs& g, hipStream_t s) { return launch<64, 64, 4, 64, true, true>(g, s); }
+
 template <int TBM, int TBN, int NW, int BKT>
 int dispatch_layout(bool a_kc, bool b_kc, const GemmArgs& g, hipStream_t s) {
   if (a_kc && b_kc) return launch<TBM, TBN, NW, BKT, true, true>(g, s);
@@ -1352,6 +1381,7 @@ int dispatch_rope(int config, bool b_kc, const GemmArgs& g, hipStream_t s) {
       case 0: return b_kc ? launch<256, 256, 8, 64, true, true, RD>(g, s) : launch<256, 256, 8, 64, true, false, RD>(g, s);
       case 1: return b_kc ? launch<256, 128, 8, 64, true, true, RD>(g, s) : launch<256, 128, 8, 64, true, false, RD>(g, s);
       case 2: return b_kc ? launch<128, 128, 4, 32, true, true, RD>(g, s) : launch<128, 128, 4, 32, true, false, RD>(g, s);
+      case kSmall: return launch<64, 64, 4, 64, true, true, RD>(g, s);
       default: break;
     }
   }
@@ -1383,6 +1413,7 @@ int dispatch_swiglu_bwd(int config, bool b_kc, const GemmArgs& g, hipStream_t s)
                         : launch<256, 128, 8, 64, true, false, 0, false, true>(g, s);
     case 2: return b_kc ? launch<128, 128, 4, 32, true, true, 0, false, true>(g, s)
                         : launch<128, 128, 4, 32, true, false, 0, false, true>(g, s);
+    case kSmall: return launch<64, 64, 4, 64, true, true, 0, false, true>(g, s);
     default: return b_kc ? launch<128, 256, 4, 32, true, true, 0, false, true>(g, s)
                          : launch<128, 256, 4, 32, true, false, 0, false, true>(g, s);
   }
@@ -1393,6 +1424,7 @@ int dispatch_swiglu(int config, const GemmArgs& g, hipStream_t s) {
     case 0: return launch<256, 256, 8, 64, true, true, 0, true>(g, s);
     case 1: return launch<256, 128, 8, 64, true, true, 0, true>(g, s);
     case 2: return launch<128, 128, 4, 32, true, true, 0, true>(g, s);
+    case kSmall: return launch<64, 64, 4, 64, true, true, 0, true>(g, s);
     default: return launch<128, 256, 4, 32, true, true, 0, true>(g, s);
   }
 }
@@ -1489,6 +1521,7 @@ extern "C" int nmb_gemm_bf16(int a_layout, int b_layout, int64_t m, int64_t n, i
     case 0: return nmb::dispatch_layout<256, 256, 8, 64>(a_kc, b_kc, g, stream);
     case 1: return nmb::dispatch_layout<256, 128, 8, 64>(a_kc, b_kc, g, stream);
     case 2: return nmb::dispatch_layout<128, 128, 4, 32>(a_kc, b_kc, g, stream);
+    case nmb::kSmall: return nmb::launch_small(g, stream);
     default: return nmb::dispatch_layout<128, 256, 4, 32>(a_kc, b_kc, g, stream);
   }
 }
@@ -1517,6 +1550,7 @@ extern "C" int nmb_gemm_bf16_f32out(int a_layout, int b_layout, int64_t m, int64
     case 0: return nmb::dispatch_layout<256, 256, 8, 64>(a_kc, b_kc, g, stream);
     case 1: return nmb::dispatch_layout<256, 128, 8, 64>(a_kc, b_kc, g, stream);
     case 2: return nmb::dispatch_layout<128, 128, 4, 32>(a_kc, b_kc, g, stream);
+    case nmb::kSmall: return nmb::launch_small(g, stream);
     default: return nmb::dispatch_layout<128, 256, 4, 32>(a_kc, b_kc, g, stream);
   }
 }
@@ -1564,7 +1598,7 @@ extern "C" int nmb_gemm_bf16_rope(int b_layout, int64_t m, int64_t n, int64_t k,
   };
   nmb::Plan p = nmb::plan_for(m, n, k, true, b_kc, static_cast<int>(head_dim));
   int64_t n_rope = n;
-  if (rope_cols > 0 && rope_cols < n) {
+  if (rope_cols > 0 && rope_cols < n && p.config != nmb::kSmall) {
     // The columns past rope_cols (v) need no rotation: as a plain product of
     // their own they can take a tile shape that fills the CUs in whole rounds
     // where the full width cannot (8192 x 3072: 1.5 rounds of 256 x 256 tiles
@@ -1586,6 +1620,7 @@ extern "C" int nmb_gemm_bf16_rope(int b_layout, int64_t m, int64_t n, int64_t k,
         case 0: st2 = nmb::dispatch_layout<256, 256, 8, 64>(true, b_kc, gv, stream); break;
         case 1: st2 = nmb::dispatch_layout<256, 128, 8, 64>(true, b_kc, gv, stream); break;
         case 2: st2 = nmb::dispatch_layout<128, 128, 4, 32>(true, b_kc, gv, stream); break;
+        case nmb::kSmall: st2 = nmb::launch_small(gv, stream); break;
         default: st2 = nmb::dispatch_layout<128, 256, 4, 32>(true, b_kc, gv, stream); break;
       }
       if (st2 != NMB_OK) return st2;

@@ -16,8 +16,8 @@ pytestmark = pytest.mark.gpu
 SHAPES = [  # (m, n, k, split?): M and N off the tiles, K off the K tile and the split
     (1003, 2056, 5640, True),   # 256 x 128, split
     (2001, 2056, 11272, True),  # 256 x 256, split
-    (193, 1032, 1000, True),    # 128 x 128, split
-    (50, 1024, 2744, True),
+    (193, 1032, 1000, False),   # NT: 64 x 64; the others: 128 x 128, split
+    (50, 1024, 2744, True),     # NT: 64 x 64, split
     (2127, 1032, 1032, False),  # 128 x 128, one workgroup per CU
     (5501, 1024, 2744, False),  # 256 x 128
     (2056, 4104, 2056, False),  # 256 x 256
