@@ -1205,12 +1205,23 @@ int attn_fwd_impl(bool from_lse, const void* q, const void* const* k_blocks,
     // the forward addresses a K/V block through a 32-bit buffer offset
     NMB_REQUIRE_SUPPORTED(seq_k == 0 || ((seq_k - 1) * kv_strides[1] + head_dim) * 2 < (int64_t{1} << 31),
                           "attn_fwd: a K/V block spans more than 2 GiB");
-    // queries per workgroup: NWV waves x TQ column tiles of 16.  D 64: 8 waves x 4
+    // queries per workgroup: NWV waves x TQ column tiles of 16.  Few queries (below):
+    // 4 x 1.  Else D 64: 8 waves x 4
     // for 512 .. 1023 queries, 4 x 2 (three workgroups per CU) from 1024, else
     // 4 x 4; D 128: 8 x 2 (two waves per SIMD)
+    // Where workgroups of 64 queries (one column tile per wave, 4 waves) all run
+    // at once, three per CU at D 64 and one at D 128, they replace the larger
+    // ones, which then leave CUs idle and put a chain of two or four column tiles
+    // on every wave.  Causal forward, us, larger -> 64 queries (same bits): 16
+    // heads of 64 x 193 tokens 11.1 -> 7.0, 2 x 16 x 512 23.7 -> 12.0, 16 x 1023
+    // 46.0 -> 20.5, 3 x 12 x 709 25.0 -> 17.2, 16 x 3000 69 -> 58; 8 heads of 128
+    // x 193 14.3 -> 10.2, 8 x 2000 77 -> 56, but in two rounds (2 x 16 x 1024) 44
+    // -> 54, and one tile of queries (8 x 40) 5.6 -> 6.0.
+    const int64_t items64 = (seq_q + 63) / 64 * q_heads * batch;
+    const bool few = head_dim == 64 ? items64 <= 768 : seq_q > 64 && items64 <= 256;
     const bool long_seq = head_dim == 64 && seq_q >= 1024;
-    const int nwv = (head_dim == 64 && seq_q >= 512 && !long_seq) || head_dim == 128 ? 8 : 4;
-    const int bq = 16 * nwv * (head_dim == 64 && !long_seq ? 4 : 2);
+    const int nwv = !few && ((head_dim == 64 && seq_q >= 512 && !long_seq) || head_dim == 128) ? 8 : 4;
+    const int bq = few ? 64 : 16 * nwv * (head_dim == 64 && !long_seq ? 4 : 2);
     const int n_qt = static_cast<int>((seq_q + bq - 1) / bq);
     const int64_t items = static_cast<int64_t>(n_qt) * q_heads * batch;
     NMB_REQUIRE(items < (int64_t{1} << 30), "attn_fwd: problem too large for one launch");
@@ -1222,7 +1233,13 @@ int attn_fwd_impl(bool from_lse, const void* q, const void* const* k_blocks,
 #define NMB_FWD(DD, TT, NW, FF)                                                                        \
   hipLaunchKernelGGL((nmb::attn_fwd_kernel<DD, TT, NW, FF>), dim3(blocks), dim3(64 * NW), 0, stream, qp, kv, \
                      op, lse, p, n_qt, static_cast<int>(items), per_xcd)
-    if (head_dim == 64 && nwv == 8) {
+    if (few) {
+      if (head_dim == 64) {
+        if (from_lse) NMB_FWD(64, 1, 4, true); else NMB_FWD(64, 1, 4, false);
+      } else {
+        if (from_lse) NMB_FWD(128, 1, 4, true); else NMB_FWD(128, 1, 4, false);
+      }
+    } else if (head_dim == 64 && nwv == 8) {
       if (from_lse) NMB_FWD(64, 4, 8, true); else NMB_FWD(64, 4, 8, false);
     } else if (long_seq) {
       if (from_lse) NMB_FWD(64, 2, 4, true); else NMB_FWD(64, 2, 4, false);
