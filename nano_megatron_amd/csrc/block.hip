@@ -4,9 +4,9 @@
 // caller one call forward and two backward.  Driven one C call per kernel from
 // Python, every launch cost about 29 us of host time and short sequences waited
 // for the host: a smoke-configuration step (4 fp32 layers, 4 x 128 tokens) took
-// 4.44 ms against 1.4 ms of kernels (now 1.92 ms), the logits of a 193-token
-// prefix through 24 layers of hidden 1024 4.69 ms (now 2.02 ms), one layer of
-// hidden 768 on 3 x 709 tokens forward and backward 0.87 ms (now 0.41 ms).
+// 4.44 ms against 1.4 ms of kernels (1.92 ms so), the logits of a 193-token
+// prefix through 24 layers of hidden 1024 4.69 ms (2.02 ms so), one layer of
+// hidden 768 on 3 x 709 tokens forward and backward 0.87 ms (0.41 ms so).
 //
 // Weight gradients on a second stream: the block's weight gradients feed
 // nothing else in its backward, and beside the dX chain they fill the CUs that
