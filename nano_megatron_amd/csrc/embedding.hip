@@ -182,8 +182,8 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict_
       row = e & ((1 << row_bits) - 1);
       token = s * kSegment + (e >> row_bits);
     } else {
-      const int64_t id = ids[k + lane];
-      if (id >= g0 && id < g0 + (1 << row_bits)) row = static_cast<int>(id - g0);
+      const int64_t id = ids[k + lane];  // (the last group's rows may end past the table)
+      if (id >= g0 && id < min<int64_t>(g0 + (1 << row_bits), vocab)) row = static_cast<int>(id - g0);
       token = k + lane;
     }
   };

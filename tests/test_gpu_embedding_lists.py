@@ -45,3 +45,29 @@ def test_listed_tokens_are_added_in_order(dtype, tokens, vocab, hidden, tied) ->
     if tied:
         exp = (exp.float() + lm.cpu().float()).to(dtype)
     assert torch.equal(got.cpu(), exp)
+
+
+@pytest.mark.parametrize("entry,tokens", [("nmb_embedding_bwd_ws", 64), ("nmb_embedding_bwd_ws", 300),
+                                          ("nmb_embedding_bwd", 30), ("nmb_embedding_bwd", 300)])
+@pytest.mark.parametrize("vocab", [17, 8190, 50257])
+def test_repeated_ids_past_the_table_write_nothing(entry, tokens, vocab) -> None:
+    """More than 24 tokens of one id (the rows a whole workgroup adds up) at and
+    past a table that ends inside a workgroup's 16 rows: the rows behind the
+    table gradient stay as they were, and the table's are the other tokens'."""
+    hidden, band = 64, 32
+    g = torch.Generator(device="cuda").manual_seed(vocab + tokens)
+    ids = torch.full((tokens,), vocab, device="cuda")
+    ids[::10] = vocab + 1
+    ids[0], ids[-1] = vocab - 1, vocab - 1
+    assert int((ids == vocab).sum()) > 24
+    dout = torch.randn(tokens, hidden, generator=g, device="cuda")
+    out = torch.full((vocab + band, hidden), 7.0, device="cuda")
+    nbytes = _lib.ctypes.c_int64()
+    _lib.call("nmb_embedding_bwd_workspace_bytes", tokens, vocab, _lib.ctypes.byref(nbytes))
+    ws = torch.empty(max(nbytes.value, 16), dtype=torch.uint8, device="cuda")
+    extra = (ws.data_ptr(), nbytes.value) if entry.endswith("_ws") else ()
+    _lib.call(entry, dout.data_ptr(), ids.data_ptr(), None, out.data_ptr(), tokens, vocab, hidden, *extra,
+              _lib.dtype_code(torch.float32), _lib.stream_of(dout))
+    assert (out[vocab:] == 7.0).all()
+    assert (out[: vocab - 1] == 0).all()
+    assert torch.equal(out[vocab - 1], dout[0] + dout[-1])
