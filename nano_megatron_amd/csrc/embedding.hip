@@ -344,6 +344,9 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict_
       }
     }
     if (mine) grad_out[cell] = finished(sum, grad_in != nullptr ? to_f32(grad_in[cell]) : 0.f);
+    // a last gather that found nothing passed no barrier since hot_state was
+    // read, and wavefront 0 writes it again for the next row
+    __syncthreads();
   }
 }
 

@@ -71,3 +71,25 @@ def test_repeated_ids_past_the_table_write_nothing(entry, tokens, vocab) -> None
     assert (out[vocab:] == 7.0).all()
     assert (out[: vocab - 1] == 0).all()
     assert torch.equal(out[vocab - 1], dout[0] + dout[-1])
+
+
+@pytest.mark.parametrize("first", [961, 970, 1024])
+def test_frequent_rows_whose_last_gather_is_empty(first) -> None:
+    """A row's tokens are gathered up to 1,024 at a time and a gather stops past
+    960: with 961 to 1,024 tokens, all in the first 8,192, the second gather of
+    the row finds nothing.  Seven more frequent rows of the same 16 follow."""
+    tokens, vocab, hidden = 2 * 8192, 64, 264
+    g = torch.Generator(device="cuda").manual_seed(first)
+    ids = torch.full((tokens,), vocab - 1, device="cuda")
+    ids[:first] = 16
+    for i, n in enumerate((40, 100, 970, 1000, 1500, 65, 30)):
+        at = 1100 + 1600 * i
+        ids[at: at + n] = 18 + 2 * i
+    dout = torch.randn(tokens, hidden, generator=g, device="cuda")
+    table = torch.zeros(vocab, hidden, device="cuda", requires_grad=True)
+    (got,) = torch.autograd.grad(Fn.embedding(table, ids, None), table, dout)
+    host, rows = ids.cpu().numpy(), dout.cpu().numpy()
+    exp = np.zeros((vocab, hidden), np.float32)
+    for v in np.unique(host):
+        exp[v] = np.add.accumulate(rows[host == v], axis=0, dtype=np.float32)[-1]
+    assert np.array_equal(got.cpu().numpy(), exp)
