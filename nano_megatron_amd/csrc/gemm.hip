@@ -324,6 +324,7 @@ __device__ __forceinline__ void k_loop(const Loader<TBM, A_KC, BKT, NW>& la,
     // LDS) 0-9%; the fused gate/up backward below 8192 x 5632 x 2048 607 -> 575.
     constexpr bool kTail = std::is_same_v<Hook, NoHook>;
     static_assert(KSTEPS == 2 && (kTail || S == 2), "two steps; a hook's loads follow the last wait");
+    if (nk <= 0) return;  // K = 0: no stage was filled, acc stays as it is
     auto read_a = [&](int st, int i, int k) { return fra.get(at_byte(&sA[0][0], Map::a(st)), i, k); };
     auto read_b = [&](int st, int j, int k) { return frb.get(at_byte(&sB[0][0], Map::b(st)), j, k); };
     bf16x8 fa0[TM], fb0[TN], fa1[TM], fb1[TN];

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import nano_megatron_amd.functional as Fn
+from nano_megatron_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +50,59 @@ def test_gate_up_swiglu_backward_k_tiles(k1, k2) -> None:
     for _ in range(3):
         out = Fn.mm_gate_up_swiglu_bwd(x, wgu, dy, wd)
         assert torch.equal(out[0], exp[0]) and torch.equal(out[1], exp[1])
+
+
+@pytest.mark.parametrize("m,n", [(40, 72), (296, 3000), (4096, 4096)])
+@pytest.mark.parametrize("la,lb", [(0, 0), (0, 1), (1, 1)])
+def test_no_k_gives_beta_c(m, n, la, lb) -> None:
+    """K = 0: the product is zero, D = beta C, on every tile shape (the C entry
+    points take it; a product of NaN runs first, whose values LDS may still hold)."""
+    stream = torch.cuda.current_stream().cuda_stream
+    nan = torch.full((512, 512), float("nan"), device="cuda", dtype=torch.bfloat16)
+    c = torch.randn(m, n, device="cuda").bfloat16()
+    a, b = torch.ones(m, 8, device="cuda").bfloat16(), torch.ones(n, 8, device="cuda").bfloat16()
+    lda, ldb = (8 if la == 0 else m), (8 if lb == 0 else n)
+    for beta in (0.0, 1.0):
+        Fn.mm(nan, nan.t())
+        d = torch.full_like(c, 5.0)
+        _lib.call("nmb_gemm_bf16", la, lb, m, n, 0, 1.0, a.data_ptr(), lda, b.data_ptr(), ldb, beta,
+                  c.data_ptr() if beta else None, n, d.data_ptr(), n, None, 0, stream)
+        assert torch.equal(d, c * beta)
+        d32 = torch.full((m, n), 3.0, device="cuda")
+        _lib.call("nmb_gemm_bf16_f32out", la, lb, m, n, 0, 1.0, a.data_ptr(), lda, b.data_ptr(), ldb, beta,
+                  d32.data_ptr(), n, None, 0, stream)
+        assert (d32 == 3.0 * beta).all()
+
+
+@pytest.mark.parametrize("m,f", [(40, 72), (512, 4096)])
+def test_no_k_in_the_fused_products(m, f) -> None:
+    """K = 0 with the RoPE, SwiGLU and SwiGLU backward epilogues: zero products."""
+    stream = torch.cuda.current_stream().cuda_stream
+    bf = dict(device="cuda", dtype=torch.bfloat16)
+    nan = torch.full((512, 512), float("nan"), **bf)
+    x, w = torch.ones(m, 8, **bf), torch.ones(2 * f, 8, **bf)
+    ang = torch.rand(m, 32, device="cuda")
+    cos, sin = ang.cos(), ang.sin()
+    Fn.mm(nan, nan.t())
+    d = torch.full((m, 128), 5.0, **bf)
+    _lib.call("nmb_gemm_bf16_rope", 0, m, 128, 0, x.data_ptr(), 8, w.data_ptr(), 8, d.data_ptr(), 128,
+              cos.data_ptr(), sin.data_ptr(), m, None, 0, 0, m, 64, 64, stream)
+    assert (d == 0).all()
+    act, gu = torch.full((m, f), 5.0, **bf), torch.full((m, 2 * f), 5.0, **bf)
+    Fn.mm(nan, nan.t())
+    _lib.call("nmb_gemm_bf16_swiglu", m, f, 0, x.data_ptr(), 8, w.data_ptr(), 8, act.data_ptr(), f, gu.data_ptr(),
+              2 * f, stream)
+    assert (act == 0).all() and (gu == 0).all()
+    gu = torch.randn(m, 2 * f, device="cuda").bfloat16()
+    for lb, ldb in ((0, 8), (1, f)):
+        dgu = torch.full_like(gu, 5.0)
+        Fn.mm(nan, nan.t())
+        _lib.call("nmb_gemm_bf16_swiglu_bwd", lb, m, f, 0, x.data_ptr(), 8, w.data_ptr(), ldb, gu.data_ptr(), 2 * f,
+                  dgu.data_ptr(), 2 * f, act.data_ptr(), f, stream)
+        assert (dgu == 0).all() and torch.equal(act, Fn.swiglu_fwd(gu[:, :f], gu[:, f:]))
+        # the fused pair: no gate / up product (K1 = 0) before a ds of 8 x 1
+        dy, wd = torch.ones(m, 8, **bf), torch.ones(f * 8, **bf)
+        Fn.mm(nan, nan.t())
+        _lib.call("nmb_gemm_bf16_gate_up_swiglu_bwd", m, f, 0, x.data_ptr(), 8, w.data_ptr(), 8, 8, dy.data_ptr(), 8,
+                  lb, wd.data_ptr(), ldb, dgu.data_ptr(), 2 * f, act.data_ptr(), f, stream)
+        assert (dgu == 0).all() and (act == 0).all()
