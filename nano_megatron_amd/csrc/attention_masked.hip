@@ -12,16 +12,18 @@
 // the other side per step, streamed into LDS by direct loads.  Everything the
 // one-row-per-wavefront kernels held in fp32 stays so: the scores, the row sum
 // and the probabilities; a probability (and a dS) enters its product as the
-// sum of two bf16 values (its rounding and the rounding of the rest, 2^-17 of
-// it at most left out), so those products run twice.  What bounds them: at
-// B 8, Hq 16, S 512, D 64 (one pass, forward and backward, 15 GFLOP counted
-// once, 67 MB) the exponentials, mask selects and splits on the VALU and the
-// latency of each 64-row step, not the matrix cores; 64 queries (keys) per
-// workgroup give 1,024 workgroups there and three per CU.  Measured there with
-// a padding mask: forward 30 us, dQ 36 us, dK/dV 46 us (one wavefront per row:
-// 1,939, 2,279 and 2,506 us); with dropout 0.1 at Hq 12 32, 37 and 54 us
-// (1,823, 2,124 and 2,423 us).  Errors against 64 bits are those of the fp32
-// kernels to four digits (rel. L2 0.0016 to 0.0023, the outputs' own rounding).
+// sum of three bf16 values that hold its fp32 bits, so those products run
+// three times.  What bounds them: at B 8, Hq 16, S 512, D 64 (one pass, forward
+// and backward, 15 GFLOP counted once, 67 MB) the exponentials, mask selects
+// and splits on the VALU and the latency of each 64-row step, not the matrix
+// cores; 64 queries (keys) per workgroup give 1,024 workgroups there and three
+// per CU.  Measured there with a padding mask: forward 34 us, dQ 39 us, dK/dV
+// 53 us (one wavefront per row: 1,939, 2,279 and 2,506 us); with dropout 0.1 at
+// Hq 12 36, 41 and 62 us (1,823, 2,124 and 2,423 us).  With two bf16 terms (up
+// to 2^-17 of a probability left out) they took 31, 35 and 46 us, and the
+// errors of O and dV against 64 bits grew by 5e-7 and 1e-6 of themselves (the
+// outputs' own rounding is 1.7e-3); with three they are within 1e-8 of the
+// fp32 kernels' over 30 shapes.
 //
 // Boolean masks that are the same for every query (a padding mask) are read
 // once per workgroup into one bit per key in LDS: key tiles without a visible
@@ -48,10 +50,15 @@ struct MaskRead {
   int vec4;
 };
 
-// p = hi + lo up to 2^-17 |p|
-__device__ __forceinline__ void split2(float p, bf16& hi, bf16& lo) {
-  hi = static_cast<bf16>(p);
-  lo = static_cast<bf16>(p - static_cast<float>(hi));
+// p as three bf16 terms, to its fp32 bits (each rounding leaves a rest of fewer
+// bits, the last at most 2^-25 |p|)
+constexpr int kTerms = 3;
+__device__ __forceinline__ void split(float p, bf16x8 (&t)[kTerms], int i) {
+#pragma unroll
+  for (int k = 0; k < kTerms; ++k) {
+    t[k][i] = static_cast<bf16>(p);
+    p -= static_cast<float>(t[k][i]);
+  }
 }
 
 // Bit key % 64 of word key / 64: key is visible in the boolean mask row at
@@ -270,7 +277,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_fwd_kernel(
       for (int dt = 0; dt < DT; ++dt) acc[dt] *= alpha;
     }
     const float mc = m == -__builtin_inff() ? 0.f : m;  // no visible key yet: P = 0
-    bf16x8 ph[2], pl[2];
+    bf16x8 pt[2][kTerms];
 #pragma unroll
     for (int mk = 0; mk < 4; ++mk) {
       bool keep[4] = {true, true, true, true};
@@ -280,10 +287,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_fwd_kernel(
         float pv = fast_exp2((s[mk][e] - mc) * kLog2e);
         l += pv;
         if constexpr (DROP) pv = keep[e] ? pv : 0.f;  // the factor 1 / (1 - p) at the end
-        bf16 hi, lo;
-        split2(pv, hi, lo);
-        ph[mk >> 1][4 * (mk & 1) + e] = hi;
-        pl[mk >> 1][4 * (mk & 1) + e] = lo;
+        split(pv, pt[mk >> 1], 4 * (mk & 1) + e);
       }
     }
 #pragma unroll
@@ -291,8 +295,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_fwd_kernel(
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
         const bf16x8 vv = Tile::col8(tv, 32 * s2, dt * 16, l16, g);
-        acc[dt] = mfma16(vv, pl[s2], acc[dt]);
-        acc[dt] = mfma16(vv, ph[s2], acc[dt]);
+#pragma unroll
+        for (int t = kTerms - 1; t >= 0; --t) acc[dt] = mfma16(vv, pt[s2][t], acc[dt]);
       }
   }
   wait_vmcnt<0>();  // no load may still write this workgroup's LDS when it ends
@@ -393,7 +397,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dq_kernel(
     if constexpr (MK == kKeyMask) bits = sBits[kt] >> (4 * g);
     kt = tiles.from(kt + 1);
     const int lim = mask_limit(p, 0, k0, p.q_offset + qi);
-    bf16x8 sh[2], sl[2];
+    bf16x8 st[2][kTerms];
 #pragma unroll
     for (int mk = 0; mk < 4; ++mk) {
       f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f}, t = s;
@@ -411,10 +415,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dq_kernel(
         float dz = t[e];
         if constexpr (DROP) dz = keep[e] ? dz * dp.scale : 0.f;
         const float ds = x == -__builtin_inff() ? 0.f : pv * (dz - dl);
-        bf16 hi, lo;
-        split2(ds, hi, lo);
-        sh[mk >> 1][4 * (mk & 1) + e] = hi;
-        sl[mk >> 1][4 * (mk & 1) + e] = lo;
+        split(ds, st[mk >> 1], 4 * (mk & 1) + e);
       }
     }
 #pragma unroll
@@ -422,8 +423,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dq_kernel(
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
         const bf16x8 kk = Tile::col8(tk, 32 * s2, dt * 16, l16, g);
-        acc[dt] = mfma16(kk, sl[s2], acc[dt]);
-        acc[dt] = mfma16(kk, sh[s2], acc[dt]);
+#pragma unroll
+        for (int t = kTerms - 1; t >= 0; --t) acc[dt] = mfma16(kk, st[s2][t], acc[dt]);
       }
   }
   wait_vmcnt<0>();  // no load may still write this workgroup's LDS when it ends
@@ -566,7 +567,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dkdv_kernel(
     const uint64_t pbase = (static_cast<uint64_t>(b) * p.Hq + h) * p.Sq + q0;
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
-      bf16x8 ph, pl, sh, sl;
+      bf16x8 pt[kTerms], st[kTerms];
 #pragma unroll
       for (int m2 = 0; m2 < 2; ++m2) {
         const int mq = 2 * s2 + m2;
@@ -620,23 +621,19 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dkdv_kernel(
           const float ds = off ? 0.f : pv * (dz - sDl[ql]);
           if constexpr (DROP) pv = keep[e] ? pv * dp.scale : 0.f;
           pv = off ? 0.f : pv;
-          bf16 hi, lo;
-          split2(pv, hi, lo);
-          ph[4 * m2 + e] = hi;
-          pl[4 * m2 + e] = lo;
-          split2(ds, hi, lo);
-          sh[4 * m2 + e] = hi;
-          sl[4 * m2 + e] = lo;
+          split(pv, pt, 4 * m2 + e);
+          split(ds, st, 4 * m2 + e);
         }
       }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const bf16x8 bd = Tile::col8(td, 32 * s2, dt * 16, l16, g);
         const bf16x8 bq = Tile::col8(tq, 32 * s2, dt * 16, l16, g);
-        dva[dt] = mfma16(pl, bd, dva[dt]);
-        dka[dt] = mfma16(sl, bq, dka[dt]);
-        dva[dt] = mfma16(ph, bd, dva[dt]);
-        dka[dt] = mfma16(sh, bq, dka[dt]);
+#pragma unroll
+        for (int t = kTerms - 1; t >= 0; --t) {
+          dva[dt] = mfma16(pt[t], bd, dva[dt]);
+          dka[dt] = mfma16(st[t], bq, dka[dt]);
+        }
       }
     }
   }

@@ -86,3 +86,46 @@ def test_masked_mfma_attention_matches_oracle(kind, causal, offset, hq, hkv, sq,
             assert float(got.detach().abs().max()) <= 1.02 * ds * x / d ** 0.5 / (1 - p), name
         else:
             assert rel_l2(got, exp) <= bound, (name, rel_l2(got, exp))
+
+
+@pytest.mark.parametrize("kind", ["keys", "bool", "add"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_probabilities_keep_their_fp32_bits(kind, d) -> None:
+    """Pairs of keys whose scores differ by 2^-12 and whose values are opposite,
+    and such pairs of queries: every sum is of differences of 2^-12 of its
+    terms, so that two bf16 terms per probability (2^-18 of it in error, 2^-19.5
+    in the mean) would show as 2^-7.5 of the results.  The dots are exact in
+    fp32 (multiples of 2^-12 below 2^8); a probability within 2^-22 gives 2^-10
+    of a result beside its rounding, 2^-9; dQ and dK also see delta from the
+    rounded O: twice that."""
+    g = torch.Generator().manual_seed(3)
+    b, h, n = 1, 2, 96
+
+    def grid(*shape):  # multiples of 1/8 up to 1.5
+        return (torch.randint(-12, 13, shape, generator=g) / 8).double()
+
+    def pairs(x, col):
+        x = x.repeat_interleave(2, 2)
+        x[..., col] = 0
+        x[:, :, 1::2, col] = 2.0 ** -9
+        return x
+
+    q, k = grid(b, h, n, d), grid(b, h, n, d)
+    q[..., 0], k[..., 1] = 1.5, 1.5
+    k[:, :, ::2, 1] = -1.5
+    q, k = pairs(q, 1), pairs(k, 0)
+    v, do = (torch.randn(b, h, n, d, generator=g).bfloat16().double().repeat_interleave(2, 2) for _ in range(2))
+    v[:, :, 1::2], do[:, :, 1::2] = -v[:, :, 1::2], -do[:, :, 1::2]
+    for t in (q, k):
+        assert torch.equal(t, t.bfloat16().double())
+    ref = [t.clone().requires_grad_() for t in (q, k, v)]
+    o_ref = torch.softmax(ref[0] @ ref[1].transpose(2, 3) / 8, -1) @ ref[2]
+    grads = torch.autograd.grad(o_ref, ref, do)
+    mask = {"keys": torch.ones(b, 1, 1, 2 * n, dtype=torch.bool), "bool": torch.ones(2 * n, 2 * n, dtype=torch.bool),
+            "add": torch.zeros(2 * n, 2 * n, dtype=torch.bfloat16)}[kind]
+    dev = [t.bfloat16().cuda().requires_grad_() for t in (q, k, v)]
+    o = Fn.masked_attention(*dev, mask.cuda(), causal=False, scale=0.125)
+    got = (o, *torch.autograd.grad(o, dev, do.bfloat16().cuda()))
+    ulp = 2.0 ** -9
+    for name, a, e, bound in zip(("o", "dq", "dk", "dv"), got, (o_ref, *grads), (1.5, 3, 3, 1.5)):
+        assert rel_l2(a, e) <= bound * ulp, (name, rel_l2(a, e) / ulp)
