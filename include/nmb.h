@@ -220,9 +220,10 @@ int nmb_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o
  * that of the undropped softmax, and the backward, given the same seed,
  * regenerates the mask.  The mask cannot equal torch's Philox stream, so
  * dropout matches the reference in distribution, not bit for bit.  bf16 or
- * fp32, head_dim <= 128, any strides; computed in fp32 one query row per
- * wavefront (a parity path: no configuration of the reference uses a mask
- * or attention dropout).  Backward workspace: nmb_attn_bwd_workspace_bytes
+ * fp32, head_dim <= 128, any strides; scores, probabilities and sums in fp32
+ * (bf16 heads of 64 and 128 with aligned rows on the bf16 matrix cores, the
+ * probabilities as three bf16 terms; the rest on the fp32 matrix cores).
+ * Keys hidden from a query may hold NaN or infinity.  Backward workspace: nmb_attn_bwd_workspace_bytes
  * (only its first half, the delta rows, is used). */
 int nmb_attn_masked_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                         int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,

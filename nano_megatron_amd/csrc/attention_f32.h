@@ -29,16 +29,10 @@
 // wavefront per row took 97, 123 (and 18 for delta) and 84 us.
 #pragma once
 
-#include "attention_common.h"
-#include "dropout_math.h"
+#include "attention_rows.h"
 
 namespace nmb {
 namespace {
-
-struct MaskRef {
-  const void* p;
-  int64_t sb, sh, sq, sk;  // element strides of [batch, q_heads, seq_q, seq_k] (0: broadcast)
-};
 
 __device__ __forceinline__ f32x4 mfma_f32x4(float a, float b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -121,7 +115,8 @@ __device__ __forceinline__ float score(float s, float scale, const MaskRef& mr, 
 }
 
 // A row (of 4 g + e) hidden from all 16 columns may hold anything: its column
-// operand becomes zeros, so that no 0 x NaN reaches a sum.
+// operand becomes zeros, so that the padding of a batch does not bring 0 x NaN
+// to the sums (rows hidden from some of the columns may: attention_rows.h).
 template <int DM>
 __device__ __forceinline__ void drop_hidden(const bool (&hidden)[4], int g, float (&v)[4][DM / 16]) {
 #pragma unroll
@@ -164,6 +159,8 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(const T* __restrict__
   constexpr int DT = DM / 16;
   __shared__ __attribute__((aligned(16))) WaveSums<DM> sums;
   __shared__ float sM[4][16], sL[4][16];
+  __shared__ uint32_t sBad;  // rows with a NaN
+  if (threadIdx.x == 0) sBad = 0;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, g = lane >> 4;
   const int q0 = 16 * (static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x));  // heavy tiles first
@@ -261,10 +258,25 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(const T* __restrict__
       lt += f * sL[w][r];
       v += f * sums.v[w][r][d];
     }
+    if (v != v) atomicOr(&sBad, 1u << r);
     if (d < D)
       o[b * p.o_sb + static_cast<int64_t>(q0 + r) * p.o_ss + h * p.o_sh + d] =
           from_f32<T>(v * (lt > 0.f ? 1.f / lt : 0.f));
     if (d == 0) lse[row + q0 + r] = lt > 0.f ? mx + logf(lt) : -__builtin_inff();
+  }
+  __syncthreads();
+  for (uint32_t bad = sBad; bad != 0; bad &= bad - 1) {  // NaN: see attention_rows.h
+    const int i = q0 + __ffs(bad) - 1;
+    if ((i & 3) != wave) continue;
+    const RowMask rm = row_mask(p, mr, dp, b, h);
+    float rmax = -__builtin_inff(), rl = 0.f, ra[2] = {0.f, 0.f};
+    for (int blk = 0; blk < p.nblk; ++blk)
+      row_fwd<T, MK, DROP>(q + b * p.q_sb + static_cast<int64_t>(i) * p.q_ss + h * p.q_sh,
+                           static_cast<const T*>(kv.k[blk]) + b * p.kv_sb + hk * p.kv_sh,
+                           static_cast<const T*>(kv.v[blk]) + b * p.kv_sb + hk * p.kv_sh, kv.koff[blk], i, p, D, rm,
+                           lane, rmax, rl, ra);
+    row_store(o + b * p.o_sb + static_cast<int64_t>(i) * p.o_ss + h * p.o_sh, ra, rl > 0.f ? 1.f / rl : 0.f, D, lane);
+    if (lane == 0) lse[row + i] = rl > 0.f ? rmax + logf(rl) : -__builtin_inff();
   }
 }
 
@@ -278,6 +290,8 @@ __global__ __launch_bounds__(256) void attn_f32_dq_kernel(const T* __restrict__ 
                                                           MaskRef mr, DropoutParams dp) {
   constexpr int DT = DM / 16;
   __shared__ __attribute__((aligned(16))) WaveSums<DM> sums;
+  __shared__ uint32_t sBad;  // rows with a NaN
+  if (threadIdx.x == 0) sBad = 0;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, g = lane >> 4;
   const int q0 = 16 * (static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x));
@@ -359,7 +373,23 @@ __global__ __launch_bounds__(256) void attn_f32_dq_kernel(const T* __restrict__ 
     const int r = i / DM, d = i % DM;
     if (q0 + r >= p.Sq || d >= D) continue;
     const float v = (sums.v[0][r][d] + sums.v[1][r][d]) + (sums.v[2][r][d] + sums.v[3][r][d]);
+    if (v != v) atomicOr(&sBad, 1u << r);
     dq[b * p.q_sb + static_cast<int64_t>(q0 + r) * p.q_ss + h * p.q_sh + d] = from_f32<T>(v * p.scale);
+  }
+  __syncthreads();
+  for (uint32_t bad = sBad; bad != 0; bad &= bad - 1) {  // NaN: see attention_rows.h
+    const int r = __ffs(bad) - 1, i = q0 + r;
+    if ((i & 3) != wave) continue;
+    const RowMask rm = row_mask(p, mr, dp, b, h);
+    const int64_t q_off = b * p.q_sb + static_cast<int64_t>(i) * p.q_ss + h * p.q_sh;
+    const float row_delta = __shfl(dl, r, 64);
+    float ra[2] = {0.f, 0.f};
+    for (int blk = 0; blk < p.nblk; ++blk)
+      row_dq<T, MK, DROP>(q + q_off, dout + b * p.o_sb + static_cast<int64_t>(i) * p.o_ss + h * p.o_sh,
+                          static_cast<const T*>(kv.k[blk]) + b * p.kv_sb + hk * p.kv_sh,
+                          static_cast<const T*>(kv.v[blk]) + b * p.kv_sb + hk * p.kv_sh, kv.koff[blk], i,
+                          lse[row + i], row_delta, p, D, rm, lane, ra);
+    row_store(dq + q_off, ra, p.scale, D, lane);
   }
 }
 
@@ -373,6 +403,8 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const T* __restrict_
                                                             int vec, MaskRef mr, DropoutParams dp) {
   constexpr int DT = DM / 16;
   __shared__ __attribute__((aligned(16))) WaveSums<DM> sums;
+  __shared__ uint32_t sBad;  // keys with a NaN
+  if (threadIdx.x == 0) sBad = 0;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, g = lane >> 4;
   const int j0 = 16 * static_cast<int>(blockIdx.x), hk = blockIdx.y;
@@ -478,9 +510,25 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const T* __restrict_
       const int r = i / DM, d = i % DM;
       if (j0 + r >= p.Sk || d >= D) continue;
       const float v = (sums.v[0][r][d] + sums.v[1][r][d]) + (sums.v[2][r][d] + sums.v[3][r][d]);
+      if (v != v) atomicOr(&sBad, 1u << r);
       outs[w][static_cast<int64_t>(j0 + r) * p.kv_ss + d] = from_f32<T>(w == 0 ? v * p.scale : v);
     }
     __syncthreads();
+  }
+  for (uint32_t bad = sBad; bad != 0; bad &= bad - 1) {  // NaN: see attention_rows.h
+    const int j = j0 + __ffs(bad) - 1;
+    if ((j & 3) != wave) continue;
+    const int64_t off = static_cast<int64_t>(j) * p.kv_ss;
+    float rk[2] = {0.f, 0.f}, rv[2] = {0.f, 0.f};
+    for (int h = hk * group; h < (hk + 1) * group; ++h) {
+      const int64_t row = (static_cast<int64_t>(b) * p.Hq + h) * p.Sq;
+      row_dkdv<T, MK, DROP>(static_cast<const T*>(kv.k[blk]) + kv_off + off,
+                            static_cast<const T*>(kv.v[blk]) + kv_off + off, q + b * p.q_sb + h * p.q_sh,
+                            dout + b * p.o_sb + h * p.o_sh, lse + row, delta + row, koff, j, p, D,
+                            row_mask(p, mr, dp, b, h), lane, rk, rv);
+    }
+    row_store(outs[0] + off, rk, p.scale, D, lane);
+    row_store(outs[1] + off, rv, 1.f, D, lane);
   }
 }
 

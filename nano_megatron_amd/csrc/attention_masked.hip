@@ -17,9 +17,9 @@
 // and backward, 15 GFLOP counted once, 67 MB) the exponentials, mask selects
 // and splits on the VALU and the latency of each 64-row step, not the matrix
 // cores; 64 queries (keys) per workgroup give 1,024 workgroups there and three
-// per CU.  Measured there with a padding mask: forward 34 us, dQ 39 us, dK/dV
-// 53 us (one wavefront per row: 1,939, 2,279 and 2,506 us); with dropout 0.1 at
-// Hq 12 36, 41 and 62 us (1,823, 2,124 and 2,423 us).  With two bf16 terms (up
+// per CU.  Measured there with a padding mask: forward 35 us, dQ 39 us, dK/dV
+// 54 us (one wavefront per row: 1,939, 2,279 and 2,506 us); with dropout 0.1 at
+// Hq 12 36, 40 and 63 us (1,823, 2,124 and 2,423 us).  With two bf16 terms (up
 // to 2^-17 of a probability left out) they took 31, 35 and 46 us, and the
 // errors of O and dV against 64 bits grew by 5e-7 and 1e-6 of themselves (the
 // outputs' own rounding is 1.7e-3); with three they are within 1e-8 of the
@@ -29,7 +29,8 @@
 // once per workgroup into one bit per key in LDS: key tiles without a visible
 // key are skipped, and masked keys' rows are loaded as zeros.  Other masks are
 // read from global memory per score, four at a time where their layout
-// allows.
+// allows.  A row whose result is NaN, as hidden keys that hold NaN or infinity
+// make it, is run again by attention_rows.h.
 #include <algorithm>
 #include <initializer_list>
 #include <type_traits>
@@ -178,6 +179,22 @@ __device__ __forceinline__ void issue_none(const void* any, bf16* a, bf16* b, in
   for (int j = 0; j < TS::P; ++j) load_lds16(rz, b + 512 * (wave * TS::P + j), kOOB);
 }
 
+// attention_rows.h's kind of a mask kind
+template <int MK>
+constexpr int row_kind = MK == kNoMask ? 0 : (MK == kAddMask ? 2 : 1);
+
+// The wave's rows l16 with a NaN among their accumulators (lanes with `in`),
+// which attention_rows.h runs again.
+template <int DT>
+__device__ __forceinline__ uint32_t nan_rows(const f32x4 (&acc)[DT], bool in) {
+  bool nan = false;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) nan = nan || acc[dt][e] != acc[dt][e];
+  return rows_of(__ballot(nan && in));
+}
+
 // three stages (48 KB, three workgroups per CU) at D 64, two (64 KB, two per
 // CU) at D 128
 template <int D>
@@ -301,17 +318,27 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_fwd_kernel(
   }
   wait_vmcnt<0>();  // no load may still write this workgroup's LDS when it ends
   l = xor32_sum(xor16_sum(l));
-  if (qi >= p.Sq) return;
-  const float inv = (l > 0.f ? 1.f / l : 0.f) * (DROP ? dp.scale : 1.f);
-  bf16* orow = o + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(qi) * p.o_ss;
+  uint32_t bad = nan_rows<DT>(acc, qi < p.Sq);
+  if (qi < p.Sq && !(bad >> l16 & 1)) {
+    const float inv = (l > 0.f ? 1.f / l : 0.f) * (DROP ? dp.scale : 1.f);
+    bf16* orow = o + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(qi) * p.o_ss;
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
-    bf16x4 wv;
+    for (int dt = 0; dt < DT; ++dt) {
+      bf16x4 wv;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) wv[e] = static_cast<bf16>(acc[dt][e] * inv);
-    *reinterpret_cast<bf16x4*>(orow + dt * 16 + g * 4) = wv;
+      for (int e = 0; e < 4; ++e) wv[e] = static_cast<bf16>(acc[dt][e] * inv);
+      *reinterpret_cast<bf16x4*>(orow + dt * 16 + g * 4) = wv;
+    }
+    if (g == 0) lse[static_cast<int64_t>(bh) * p.Sq + qi] = l > 0.f ? m + logf(l) : -__builtin_inff();
   }
-  if (g == 0) lse[static_cast<int64_t>(bh) * p.Sq + qi] = l > 0.f ? m + logf(l) : -__builtin_inff();
+  for (; bad != 0; bad &= bad - 1) {
+    const int i = qt * BQ + 16 * wave + __ffs(bad) - 1;
+    float rmax = -__builtin_inff(), rl = 0.f, ra[2] = {0.f, 0.f};
+    row_fwd<bf16, row_kind<MK>, DROP>(q + b * p.q_sb + h * p.q_sh + static_cast<int64_t>(i) * p.q_ss, kb, vb, 0, i, p,
+                                      D, row_mask(p, mr.r, dp, b, h), lane, rmax, rl, ra);
+    row_store(o + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(i) * p.o_ss, ra, rl > 0.f ? 1.f / rl : 0.f, D, lane);
+    if (lane == 0) lse[static_cast<int64_t>(bh) * p.Sq + i] = rl > 0.f ? rmax + logf(rl) : -__builtin_inff();
+  }
 }
 
 // ---------------------------------------------------------------- dQ
@@ -428,13 +455,25 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dq_kernel(
       }
   }
   wait_vmcnt<0>();  // no load may still write this workgroup's LDS when it ends
-  if (qi >= p.Sq) return;
+  uint32_t bad = nan_rows<DT>(acc, qi < p.Sq);
+  if (qi < p.Sq && !(bad >> l16 & 1)) {
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
-    bf16x4 wv;
+    for (int dt = 0; dt < DT; ++dt) {
+      bf16x4 wv;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) wv[e] = static_cast<bf16>(acc[dt][e] * p.scale);
-    *reinterpret_cast<bf16x4*>(dq + q_row + dt * 16 + g * 4) = wv;
+      for (int e = 0; e < 4; ++e) wv[e] = static_cast<bf16>(acc[dt][e] * p.scale);
+      *reinterpret_cast<bf16x4*>(dq + q_row + dt * 16 + g * 4) = wv;
+    }
+  }
+  for (; bad != 0; bad &= bad - 1) {
+    const int r = __ffs(bad) - 1, i = qt * BQ + 16 * wave + r;
+    const float row_delta = __shfl(dl, r, 64);
+    const int64_t q_off = b * p.q_sb + h * p.q_sh + static_cast<int64_t>(i) * p.q_ss;
+    float ra[2] = {0.f, 0.f};
+    row_dq<bf16, row_kind<MK>, DROP>(q + q_off, dout + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(i) * p.o_ss, kb,
+                                     vb, 0, i, lse[static_cast<int64_t>(bh) * p.Sq + i], row_delta, p, D,
+                                     row_mask(p, mr.r, dp, b, h), lane, ra);
+    row_store(dq + q_off, ra, p.scale, D, lane);
   }
 }
 
@@ -639,16 +678,42 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dkdv_kernel(
   }
   wait_vmcnt<0>();  // no load may still write this workgroup's LDS when it ends
   // lane holds dK[key = kbase + 4 g + e][d = 16 dt + l16]
+  uint32_t bad = 0;  // keys with a NaN
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    bool nan = false;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) nan = nan || dka[dt][e] != dka[dt][e] || dva[dt][e] != dva[dt][e];
+    const uint64_t lanes = __ballot(nan);
+#pragma unroll
+    for (int gg = 0; gg < 4; ++gg)
+      if ((lanes >> (16 * gg)) & 0xffff) bad |= 1u << (4 * gg + e);
+  }
+  const int64_t kv_off = b * p.kv_sb + hk * p.kv_sh;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int kr = kbase + 4 * g + e;
-    if (kr >= p.Sk) continue;
-    const int64_t r = b * p.kv_sb + hk * p.kv_sh + static_cast<int64_t>(kr) * p.kv_ss;
+    if (kr >= p.Sk || (bad >> (4 * g + e) & 1)) continue;
+    const int64_t r = kv_off + static_cast<int64_t>(kr) * p.kv_ss;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       dk[r + dt * 16 + l16] = static_cast<bf16>(dka[dt][e] * p.scale);
       dv[r + dt * 16 + l16] = static_cast<bf16>(dva[dt][e]);
     }
+  }
+  for (; bad != 0; bad &= bad - 1) {
+    const int j = kbase + __ffs(bad) - 1;
+    if (j >= p.Sk) break;
+    const int64_t r = kv_off + static_cast<int64_t>(j) * p.kv_ss;
+    float rk[2] = {0.f, 0.f}, rv[2] = {0.f, 0.f};
+    for (int h = hk * group; h < (hk + 1) * group; ++h) {
+      const int64_t row = (static_cast<int64_t>(b) * p.Hq + h) * p.Sq;
+      row_dkdv<bf16, row_kind<MK>, DROP>(k + r, v + r, q + b * p.q_sb + h * p.q_sh, dout + b * p.o_sb + h * p.o_sh,
+                                         lse + row, delta + row, 0, j, p, D, row_mask(p, mr.r, dp, b, h), lane, rk,
+                                         rv);
+    }
+    row_store(dk + r, rk, p.scale, D, lane);
+    row_store(dv + r, rv, 1.f, D, lane);
   }
 }
 

@@ -6,6 +6,8 @@ and dropout over even and odd key counts."""
 
 from __future__ import annotations
 
+import math
+
 import pytest
 import torch
 
@@ -68,8 +70,6 @@ def test_masked_mfma_attention_matches_oracle(kind, causal, offset, hq, hkv, sq,
     if kind == "keys":
         hidden = ~mask[:, :, 0, :, None].expand(b, hkv, sk, d)
         k, v = k.masked_fill(hidden, float("nan")), v.masked_fill(hidden, float("nan"))
-    if kind == "keys" and sk > 16384:  # per score: 0 x NaN is NaN, as in the reference's products
-        k, v = k.nan_to_num(0.0), v.nan_to_num(0.0)
     qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
     o = Fn.masked_attention(qd, kd, vd, None if mask is None else mask.cuda(), causal=causal,
                             sequence_offset=offset, dropout_p=p, seed=77)
@@ -129,3 +129,74 @@ def test_probabilities_keep_their_fp32_bits(kind, d) -> None:
     ulp = 2.0 ** -9
     for name, a, e, bound in zip(("o", "dq", "dk", "dv"), got, (o_ref, *grads), (1.5, 3, 3, 1.5)):
         assert rel_l2(a, e) <= bound * ulp, (name, rel_l2(a, e) / ulp)
+
+
+HIDDEN = [
+    # (dtype, mask, causal, offset, sq, sk, d, p, keys and queries that hold NaN or infinity)
+    ("bf16", "none", True, 0, 130, 130, 64, 0.1, [70, 129], []),  # seen by the last queries only
+    ("bf16", "none", True, 5, 1, 40, 128, 0.1, list(range(6, 40)), []),  # one query before keys never written
+    ("bf16", "bool", True, 0, 100, 100, 64, 0.0, [3, 64, 90], [7]),
+    ("bf16", "bool", False, 0, 70, 131, 128, 0.2, [130], [0, 69]),
+    ("bf16", "add", False, 0, 66, 96, 64, 0.0, [0, 50], [65]),
+    ("bf16", "keys", True, 0, 65, 65, 64, 0.0, [20], [64]),
+    ("bf16", "bool", True, 0, 40, 50, 80, 0.0, [3, 17], [7]),
+    ("fp32", None, True, 0, 40, 40, 64, 0.0, [20, 39], []),
+    ("fp32", None, True, 5, 1, 16, 100, 0.0, list(range(6, 16)), []),
+    ("fp32", "none", True, 0, 33, 33, 128, 0.3, [17], [2, 32]),
+    ("fp32", "bool", False, 0, 30, 50, 20, 0.0, [3, 40], [29]),
+    ("fp32", "add", False, 0, 30, 50, 64, 0.2, [3, 40], [0]),
+]
+
+
+@pytest.mark.parametrize("dtype,kind,causal,offset,sq,sk,d,p,bad_keys,bad_queries", HIDDEN)
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_hidden_rows_may_hold_anything(dtype, kind, causal, offset, sq, sk, d, p, bad_keys, bad_queries, value) -> None:
+    """Keys hidden from a query, and queries without a finite score, are not read
+    for it: every other query's results and every gradient are those of finite
+    data (the bounds of the tests above; fp32: 64 roundings), with the keys
+    masked from all queries, from some, or by causality alone."""
+    dt, (b, hq, hkv) = (torch.bfloat16 if dtype == "bf16" else torch.float32), (2, 4, 2)
+    g = torch.Generator().manual_seed(sq + sk + d)
+    q, do = (torch.randn(b, hq, sq, d, generator=g).to(dt) for _ in range(2))
+    k, v = (torch.randn(b, hkv, sk, d, generator=g).to(dt) for _ in range(2))
+    see = torch.ones(b, 1, sq, sk, dtype=torch.bool)
+    mask = None
+    if kind == "keys":
+        mask = torch.rand(b, 1, 1, sk, generator=g) > 0.2
+        mask[..., bad_keys] = False
+        see = mask.expand_as(see)
+    elif kind in ("bool", "add"):
+        see = torch.rand(b, 1, sq, sk, generator=g) > 0.3
+        see[..., bad_keys[1:]] = False  # the first one is hidden from some queries
+        mask = see if kind == "bool" else torch.randn(b, 1, sq, sk, generator=g).masked_fill(~see, -math.inf).to(dt)
+    if causal:
+        see = see & (torch.arange(sk)[None] <= offset + torch.arange(sq)[:, None])
+    lost = see[..., bad_keys].any(-1).expand(b, hq, sq).clone()  # queries whose result is NaN
+    lost[..., bad_queries] = True
+    ref = [t.double().requires_grad_() for t in (q, k, v)]
+    kr, vr = (t.repeat_interleave(hq // hkv, 1) for t in ref[1:])
+    s = ref[0] @ kr.transpose(2, 3) / math.sqrt(d)
+    s = (s + mask.double() if kind == "add" else s).masked_fill(~see, -math.inf)
+    pr = torch.softmax(s, -1).nan_to_num(0.0)
+    if p:
+        pr = pr * R.dropout_keep(9, tuple(s.shape), p) / (1 - p)
+    o_ref = pr @ vr
+    grads = torch.autograd.grad(o_ref, ref, do.double().masked_fill(lost[..., None], 0.0))
+    k[:, :, bad_keys], v[:, :, bad_keys] = value, -value
+    q[:, :, bad_queries], do[:, :, bad_queries] = value, value
+    dev = [t.cuda().requires_grad_() for t in (q, k, v)]
+    if kind is None:
+        o = Fn.attention(*dev, causal=causal, sequence_offset=offset)
+    else:
+        o = Fn.masked_attention(*dev, None if mask is None else mask.cuda(), causal=causal, sequence_offset=offset,
+                                dropout_p=p, seed=9)
+    got = torch.autograd.grad(o, dev, do.cuda())
+    if math.isnan(value):
+        assert torch.isnan(o.cpu()[lost & see.any(-1)]).all()
+    ulp = 2.0 ** -9
+    bounds = (1.02 * ulp, 2 * ulp, 2 * ulp, 1.02 * ulp) if dtype == "bf16" else (64 * 2.0 ** -24,) * 4
+    keep = ~lost
+    pairs = [("o", o.cpu()[keep], o_ref[keep])] + list(zip(("dq", "dk", "dv"), got, grads))
+    for (name, a, e), bound in zip(pairs, bounds):
+        assert torch.isfinite(a).all(), name
+        assert rel_l2(a, e) <= bound if float(e.detach().abs().max()) > 1e-6 else float(a.abs().max()) < 1e-2, name
