@@ -224,7 +224,9 @@ int nmb_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o
  * (bf16 heads of 64 and 128 with aligned rows on the bf16 matrix cores, the
  * probabilities as three bf16 terms; the rest on the fp32 matrix cores).
  * Keys hidden from a query may hold NaN or infinity.  Backward workspace: nmb_attn_bwd_workspace_bytes
- * (only its first half, the delta rows, is used). */
+ * (its first half the delta rows, its second, with an additive mask, the rows'
+ * normalisers; with the first half alone dK and dV of a row masked throughout
+ * by the type's lowest value are those of probabilities of 1). */
 int nmb_attn_masked_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                         int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
                         int64_t seq_k, int64_t head_dim, const int64_t* q_strides,

@@ -1460,8 +1460,8 @@ int attn_bwd_impl(const void* q, const void* const* k_blocks,
       NMB_CHECK_LAUNCH("attn_bwd(dkdv)");
     }
   } else {
-    f32_bwd_launch<float>(p, kv, MaskRef{}, DropoutParams{0, 0, 1.f}, 0, false, q, o, dout, lse, delta, dq, D,
-                          stream);
+    f32_bwd_launch<float>(p, kv, MaskRef{}, DropoutParams{0, 0, 1.f}, 0, false, q, o, dout, lse, delta, nullptr,
+                          dq, D, stream);
     NMB_CHECK_LAUNCH("attn_bwd(f32)");
   }
   return NMB_OK;

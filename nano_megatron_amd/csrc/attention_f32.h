@@ -282,15 +282,21 @@ __global__ __launch_bounds__(256) void attn_f32_fwd_kernel(const T* __restrict__
 
 // dQ, and delta = rowsum(dO o O) for the dK/dV kernel (which equals
 // sum_j P Z (dO . V) under dropout factors Z, so dS = P (Z dO . V - delta)).
+// MK 2: the probabilities are normalised by their sum over the row, whose
+// inverse goes to norm (if given) for the dK/dV kernel: beside a mask of the
+// type's lowest value, lse = m + log(l) has no room for log(l), and exp(x -
+// lse) of a row masked throughout by it is 1 for every key.
 template <typename T, int DM, int MK, bool DROP>
 __global__ __launch_bounds__(256) void attn_f32_dq_kernel(const T* __restrict__ q, KVBlocks kv,
                                                           const T* __restrict__ o, const T* __restrict__ dout,
                                                           const float* __restrict__ lse, float* __restrict__ delta,
-                                                          T* __restrict__ dq, AttnShape p, int D, int vec,
-                                                          MaskRef mr, DropoutParams dp) {
+                                                          float* __restrict__ norm, T* __restrict__ dq,
+                                                          AttnShape p, int D, int vec, MaskRef mr,
+                                                          DropoutParams dp) {
   constexpr int DT = DM / 16;
   __shared__ __attribute__((aligned(16))) WaveSums<DM> sums;
   __shared__ uint32_t sBad;  // rows with a NaN
+  __shared__ float sN[4][16];
   if (threadIdx.x == 0) sBad = 0;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, g = lane >> 4;
@@ -315,6 +321,7 @@ __global__ __launch_bounds__(256) void attn_f32_dq_kernel(const T* __restrict__ 
   dl = xor32_sum(xor16_sum(dl));
   if (wave == 0 && g == 0 && qi < p.Sq) delta[row + qi] = dl;
   const float ls = lse[row + qr];
+  float psum = 0.f;
   f32x4 acc[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -358,7 +365,9 @@ __global__ __launch_bounds__(256) void attn_f32_dq_kernel(const T* __restrict__ 
         hidden[e] = x == -__builtin_inff() || ls == -__builtin_inff();
         float dz = dv[e];
         if constexpr (DROP) dz = keep[e] ? dz * dp.scale : 0.f;
-        ds[e] = hidden[e] ? 0.f : expf(x - ls) * (dz - dl);
+        const float pv = hidden[e] ? 0.f : expf(x - ls);
+        if constexpr (MK == 2) psum += pv;
+        ds[e] = hidden[e] ? 0.f : pv * (dz - dl);
       }
       if constexpr (MK != 0) drop_hidden<DM>(hidden, g, kc);
 #pragma unroll
@@ -368,11 +377,20 @@ __global__ __launch_bounds__(256) void attn_f32_dq_kernel(const T* __restrict__ 
     }
   }
   sums.put(wave, l16, g, acc);
+  if constexpr (MK == 2) {
+    psum = xor32_sum(xor16_sum(psum));
+    if (g == 0) sN[wave][l16] = psum;
+  }
   __syncthreads();
   for (int i = threadIdx.x; i < 16 * DM; i += 256) {
     const int r = i / DM, d = i % DM;
     if (q0 + r >= p.Sq || d >= D) continue;
-    const float v = (sums.v[0][r][d] + sums.v[1][r][d]) + (sums.v[2][r][d] + sums.v[3][r][d]);
+    float v = (sums.v[0][r][d] + sums.v[1][r][d]) + (sums.v[2][r][d] + sums.v[3][r][d]);
+    if constexpr (MK == 2) {
+      const float inv = inverse_sum((sN[0][r] + sN[1][r]) + (sN[2][r] + sN[3][r]));
+      if (d == 0 && norm != nullptr) norm[row + q0 + r] = inv;
+      v *= inv;
+    }
     if (v != v) atomicOr(&sBad, 1u << r);
     dq[b * p.q_sb + static_cast<int64_t>(q0 + r) * p.q_ss + h * p.q_sh + d] = from_f32<T>(v * p.scale);
   }
@@ -383,13 +401,15 @@ __global__ __launch_bounds__(256) void attn_f32_dq_kernel(const T* __restrict__ 
     const RowMask rm = row_mask(p, mr, dp, b, h);
     const int64_t q_off = b * p.q_sb + static_cast<int64_t>(i) * p.q_ss + h * p.q_sh;
     const float row_delta = __shfl(dl, r, 64);
-    float ra[2] = {0.f, 0.f};
+    float ra[2] = {0.f, 0.f}, rsum = 0.f;
     for (int blk = 0; blk < p.nblk; ++blk)
       row_dq<T, MK, DROP>(q + q_off, dout + b * p.o_sb + static_cast<int64_t>(i) * p.o_ss + h * p.o_sh,
                           static_cast<const T*>(kv.k[blk]) + b * p.kv_sb + hk * p.kv_sh,
                           static_cast<const T*>(kv.v[blk]) + b * p.kv_sb + hk * p.kv_sh, kv.koff[blk], i,
-                          lse[row + i], row_delta, p, D, rm, lane, ra);
-    row_store(dq + q_off, ra, p.scale, D, lane);
+                          lse[row + i], row_delta, p, D, rm, lane, ra, rsum);
+    const float inv = MK == 2 ? inverse_sum(rsum) : 1.f;
+    if (MK == 2 && lane == 0 && norm != nullptr) norm[row + i] = inv;
+    row_store(dq + q_off, ra, p.scale * inv, D, lane);
   }
 }
 
@@ -399,7 +419,8 @@ template <typename T, int DM, int MK, bool DROP>
 __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const T* __restrict__ q, KVBlocks kv,
                                                             const T* __restrict__ dout,
                                                             const float* __restrict__ lse,
-                                                            const float* __restrict__ delta, AttnShape p, int D,
+                                                            const float* __restrict__ delta,
+                                                            const float* __restrict__ norm, AttnShape p, int D,
                                                             int vec, MaskRef mr, DropoutParams dp) {
   constexpr int DT = DM / 16;
   __shared__ __attribute__((aligned(16))) WaveSums<DM> sums;
@@ -433,7 +454,7 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const T* __restrict_
   const int per_head = n_qt - qt0;
   f32x4 qf[DT], df[DT];
   float qcol[4][DT], dcol[4][DT];
-  float ls[4], dl[4];
+  float ls[4], dl[4], nm[4];
   int h = hk * group, i0 = 0;  // of the tile loaded last
   auto load = [&](int t) {
     h = hk * group + t / per_head;
@@ -451,6 +472,7 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const T* __restrict_
       const int r = min(i0 + 4 * g + e, p.Sq - 1);
       ls[e] = lse[row + r];
       dl[e] = delta[row + r];
+      nm[e] = MK == 2 && norm != nullptr ? norm[row + r] : 1.f;
     }
   };
   const int total = group * per_head;
@@ -460,10 +482,11 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const T* __restrict_
     const int ch = h, ci = i0;
     const f32x4 s = row_product<DM>(qf, kf);
     const f32x4 dpv = row_product<DM>(df, vf);
-    float qc[4][DT], dc[4][DT], lc[4], dlc[4];
+    float qc[4][DT], dc[4][DT], lc[4], dlc[4], nmc[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       lc[e] = ls[e];
+      nmc[e] = nm[e];
       dlc[e] = dl[e];
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
@@ -482,7 +505,8 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const T* __restrict_
       const bool off = i >= p.Sq || (p.causal && koff + key > p.q_offset + i) || lc[e] == -__builtin_inff();
       const float x = score<T, MK>(s[e], p.scale, mr, mask_col + ic * mr.sq, off);
       hidden[e] = x == -__builtin_inff();
-      const float pr = hidden[e] ? 0.f : expf(x - lc[e]);
+      float pr = hidden[e] ? 0.f : expf(x - lc[e]);
+      if constexpr (MK == 2) pr *= nmc[e];
       float z = 1.f;
       if constexpr (DROP) z = drop_factor(dp, static_cast<uint64_t>(row + ic) * p.Sk + key);
       pv[e] = pr * z;
@@ -524,8 +548,9 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const T* __restrict_
       const int64_t row = (static_cast<int64_t>(b) * p.Hq + h) * p.Sq;
       row_dkdv<T, MK, DROP>(static_cast<const T*>(kv.k[blk]) + kv_off + off,
                             static_cast<const T*>(kv.v[blk]) + kv_off + off, q + b * p.q_sb + h * p.q_sh,
-                            dout + b * p.o_sb + h * p.o_sh, lse + row, delta + row, koff, j, p, D,
-                            row_mask(p, mr, dp, b, h), lane, rk, rv);
+                            dout + b * p.o_sb + h * p.o_sh, lse + row, delta + row,
+                            norm != nullptr ? norm + row : nullptr, koff, j, p, D, row_mask(p, mr, dp, b, h), lane, rk,
+                            rv);
     }
     row_store(outs[0] + off, rk, p.scale, D, lane);
     row_store(outs[1] + off, rv, 1.f, D, lane);
@@ -576,7 +601,7 @@ void f32_fwd_launch(const AttnShape& p, const KVBlocks& kv, const MaskRef& mr, c
 template <typename T>
 void f32_bwd_launch(const AttnShape& p, const KVBlocks& kv, const MaskRef& mr, const DropoutParams& dp, int kind,
                     bool drop, const void* q, const void* o, const void* dout, const float* lse, float* delta,
-                    void* dq, int D, hipStream_t stream) {
+                    float* norm, void* dq, int D, hipStream_t stream) {
   const int vec = rows_vec4<T>(p, kv, D, q, o, dout);
   if (p.Sq > 0) {
     const dim3 grid(static_cast<unsigned>((p.Sq + 15) / 16), static_cast<unsigned>(p.Hq),
@@ -584,7 +609,7 @@ void f32_bwd_launch(const AttnShape& p, const KVBlocks& kv, const MaskRef& mr, c
     f32_select(D, kind, drop, [&](auto dm, auto mk, auto dr) {
       hipLaunchKernelGGL((attn_f32_dq_kernel<T, dm.value, mk.value, dr.value>), grid, dim3(256), 0, stream,
                          static_cast<const T*>(q), kv, static_cast<const T*>(o), static_cast<const T*>(dout), lse,
-                         delta, static_cast<T*>(dq), p, D, vec, mr, dp);
+                         delta, norm, static_cast<T*>(dq), p, D, vec, mr, dp);
     });
   }
   if (p.Sk > 0) {
@@ -592,7 +617,7 @@ void f32_bwd_launch(const AttnShape& p, const KVBlocks& kv, const MaskRef& mr, c
                     static_cast<unsigned>(p.B * p.nblk));
     f32_select(D, kind, drop, [&](auto dm, auto mk, auto dr) {
       hipLaunchKernelGGL((attn_f32_dkdv_kernel<T, dm.value, mk.value, dr.value>), grid, dim3(256), 0, stream,
-                         static_cast<const T*>(q), kv, static_cast<const T*>(dout), lse, delta, p, D, vec, mr, dp);
+                         static_cast<const T*>(q), kv, static_cast<const T*>(dout), lse, delta, norm, p, D, vec, mr, dp);
     });
   }
 }

@@ -343,13 +343,15 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_fwd_kernel(
 
 // ---------------------------------------------------------------- dQ
 // As the forward; also writes delta = rowsum(dO o O) (which equals
-// sum_j P Z (dO . V) under dropout factors Z) for the dK/dV kernel.
+// sum_j P Z (dO . V) under dropout factors Z) for the dK/dV kernel, and with
+// an additive mask the inverse of the row's sum of probabilities (norm;
+// attention_f32.h says why).
 template <int D, int MK, bool DROP>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dq_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const bf16* __restrict__ o, const bf16* __restrict__ dout, const float* __restrict__ lse,
-    float* __restrict__ delta, bf16* __restrict__ dq, AttnShape p, MaskRead mr, DropoutParams dp, int n_qt,
-    int items, int per_xcd) {
+    float* __restrict__ delta, float* __restrict__ norm, bf16* __restrict__ dq, AttnShape p, MaskRead mr,
+    DropoutParams dp, int n_qt, int items, int per_xcd) {
   constexpr int BQ = 64, KS = D / 32, DT = D / 16, S = masked_stages<D>();
   using Tile = Tile64<D>;
   constexpr int kLoads = 2 * TileStream<D, 4>::P;
@@ -408,6 +410,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dq_kernel(
 #pragma unroll
   for (int st = 0; st < S - 1; ++st) issue(st);
 
+  float psum = 0.f;  // this lane's 16 keys of every tile
   f32x4 acc[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -439,6 +442,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dq_kernel(
       for (int e = 0; e < 4; ++e) {
         const float x = masked_score<MK>(s[e], p.scale, qm, bits, mk, e, mk * 16 + g * 4 + e, lim);
         const float pv = fast_exp2((x - ls) * kLog2e);
+        if constexpr (MK == kAddMask) psum += pv;
         float dz = t[e];
         if constexpr (DROP) dz = keep[e] ? dz * dp.scale : 0.f;
         const float ds = x == -__builtin_inff() ? 0.f : pv * (dz - dl);
@@ -455,13 +459,20 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dq_kernel(
       }
   }
   wait_vmcnt<0>();  // no load may still write this workgroup's LDS when it ends
+  if constexpr (MK == kAddMask) psum = xor32_sum(xor16_sum(psum));
   uint32_t bad = nan_rows<DT>(acc, qi < p.Sq);
   if (qi < p.Sq && !(bad >> l16 & 1)) {
+    float f = p.scale;
+    if constexpr (MK == kAddMask) {
+      const float inv = inverse_sum(psum);
+      if (g == 0 && norm != nullptr) norm[row] = inv;
+      f *= inv;
+    }
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       bf16x4 wv;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) wv[e] = static_cast<bf16>(acc[dt][e] * p.scale);
+      for (int e = 0; e < 4; ++e) wv[e] = static_cast<bf16>(acc[dt][e] * f);
       *reinterpret_cast<bf16x4*>(dq + q_row + dt * 16 + g * 4) = wv;
     }
   }
@@ -469,11 +480,13 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dq_kernel(
     const int r = __ffs(bad) - 1, i = qt * BQ + 16 * wave + r;
     const float row_delta = __shfl(dl, r, 64);
     const int64_t q_off = b * p.q_sb + h * p.q_sh + static_cast<int64_t>(i) * p.q_ss;
-    float ra[2] = {0.f, 0.f};
+    float ra[2] = {0.f, 0.f}, rsum = 0.f;
     row_dq<bf16, row_kind<MK>, DROP>(q + q_off, dout + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(i) * p.o_ss, kb,
                                      vb, 0, i, lse[static_cast<int64_t>(bh) * p.Sq + i], row_delta, p, D,
-                                     row_mask(p, mr.r, dp, b, h), lane, ra);
-    row_store(dq + q_off, ra, p.scale, D, lane);
+                                     row_mask(p, mr.r, dp, b, h), lane, ra, rsum);
+    const float inv = MK == kAddMask ? inverse_sum(rsum) : 1.f;
+    if (MK == kAddMask && lane == 0 && norm != nullptr) norm[static_cast<int64_t>(bh) * p.Sq + i] = inv;
+    row_store(dq + q_off, ra, p.scale * inv, D, lane);
   }
 }
 
@@ -484,11 +497,12 @@ template <int D, int MK, bool DROP>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dkdv_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const bf16* __restrict__ dout, const float* __restrict__ lse, const float* __restrict__ delta,
-    bf16* __restrict__ dk, bf16* __restrict__ dv, AttnShape p, MaskRead mr, DropoutParams dp, int n_kt,
+    const float* __restrict__ norm, bf16* __restrict__ dk, bf16* __restrict__ dv, AttnShape p, MaskRead mr, DropoutParams dp, int n_kt,
     int items, int per_xcd) {
   constexpr int BQ = 64, KS = D / 32, DT = D / 16, S = masked_stages<D>();
   using Tile = Tile64<D>;
-  // Q, dO and one row statistic (even waves the lse, odd waves delta)
+  // Q, dO and one row statistic (waves 0 and 2 the lse, 1 and 3 delta; with an
+  // additive mask wave 2 the rows' normalisers)
   using TS = TileStream<D, 4>;
   constexpr int kLoads = 2 * TS::P + 1;
   __shared__ __attribute__((aligned(1024))) bf16 sQ[S][Tile::kElems];
@@ -551,7 +565,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dkdv_kernel(
                                  static_cast<uint32_t>(((rows - 1) * p.o_ss + D) * 2));
       lq.issue(rq, sQ[st], 0, rows, 0u, wave);
       ldo.issue(rd, sD[st], 0, rows, 0u, wave);
-      const float* stat = ((wave & 1) ? delta : lse) + (static_cast<int64_t>(b) * p.Hq + h) * p.Sq + r0;
+      const float* stats = wave & 1 ? delta : lse;
+      if constexpr (MK == kAddMask)
+        if (wave == 2 && norm != nullptr) stats = norm;
+      const float* stat = stats + (static_cast<int64_t>(b) * p.Hq + h) * p.Sq + r0;
       load_lds4(make_rsrc(stat, static_cast<uint32_t>(rows * 4)), &sStat[st][wave][0],
                 lane < rows ? static_cast<uint32_t>(4 * lane) : kOOB);
     } else {
@@ -655,6 +672,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dkdv_kernel(
           }
           if constexpr (MK == kBoolMask) off = off || !on[mq][e];
           float pv = fast_exp2((x - ls) * kLog2e);
+          if constexpr (MK == kAddMask) pv *= norm != nullptr ? sStat[it % S][2][ql] : 1.f;
           float dz = t[e];
           if constexpr (DROP) dz = keep[e] ? dz * dp.scale : 0.f;
           const float ds = off ? 0.f : pv * (dz - sDl[ql]);
@@ -709,8 +727,9 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_masked_dkdv_kernel(
     for (int h = hk * group; h < (hk + 1) * group; ++h) {
       const int64_t row = (static_cast<int64_t>(b) * p.Hq + h) * p.Sq;
       row_dkdv<bf16, row_kind<MK>, DROP>(k + r, v + r, q + b * p.q_sb + h * p.q_sh, dout + b * p.o_sb + h * p.o_sh,
-                                         lse + row, delta + row, 0, j, p, D, row_mask(p, mr.r, dp, b, h), lane, rk,
-                                         rv);
+                                         lse + row, delta + row,
+                                         MK == kAddMask && norm != nullptr ? norm + row : nullptr, 0, j, p, D,
+                                         row_mask(p, mr.r, dp, b, h), lane, rk, rv);
     }
     row_store(dk + r, rk, p.scale, D, lane);
     row_store(dv + r, rv, 1.f, D, lane);
@@ -783,7 +802,8 @@ void mfma_fwd_launch(const AttnShape& p, const MaskRef& mref, const DropoutParam
 
 void mfma_bwd_launch(const AttnShape& p, const MaskRef& mref, const DropoutParams& dp, int mask_kind, bool drop,
                      int D, const void* q, const void* k, const void* v, const void* o, const void* dout,
-                     const float* lse, float* delta, void* dq, void* dk, void* dv, hipStream_t stream) {
+                     const float* lse, float* delta, float* norm, void* dq, void* dk, void* dv,
+                     hipStream_t stream) {
   MaskRead mr;
   const int kind = kernel_mask(p, mref, mask_kind, &mr);
   const int n_qt = (p.Sq + 63) / 64, n_kt = (p.Sk + 63) / 64;
@@ -796,7 +816,7 @@ void mfma_bwd_launch(const AttnShape& p, const MaskRef& mref, const DropoutParam
       hipLaunchKernelGGL((attn_masked_dq_kernel<dd.value, mk.value, dr.value>), dim3(blocks), dim3(256), 0, stream,
                          static_cast<const bf16*>(q), static_cast<const bf16*>(k), static_cast<const bf16*>(v),
                          static_cast<const bf16*>(o), static_cast<const bf16*>(dout), lse, delta,
-                         static_cast<bf16*>(dq), p, mr, dp, n_qt, items, per);
+                         norm, static_cast<bf16*>(dq), p, mr, dp, n_qt, items, per);
     });
   }
   const int items = p.B * p.Hkv * n_kt;
@@ -804,8 +824,8 @@ void mfma_bwd_launch(const AttnShape& p, const MaskRef& mref, const DropoutParam
   masked_select(D, kind, drop, [&](auto dd, auto mk, auto dr) {
     hipLaunchKernelGGL((attn_masked_dkdv_kernel<dd.value, mk.value, dr.value>), dim3(blocks), dim3(256), 0, stream,
                        static_cast<const bf16*>(q), static_cast<const bf16*>(k), static_cast<const bf16*>(v),
-                       static_cast<const bf16*>(dout), lse, delta, static_cast<bf16*>(dk), static_cast<bf16*>(dv),
-                       p, mr, dp, n_kt, items, per);
+                       static_cast<const bf16*>(dout), lse, delta, norm, static_cast<bf16*>(dk),
+                       static_cast<bf16*>(dv), p, mr, dp, n_kt, items, per);
   });
 }
 
@@ -909,14 +929,15 @@ extern "C" int nmb_attn_masked_bwd(const void* q, const void* k, const void* v, 
   kv.dv[0] = dv;
   if (batch == 0) return NMB_OK;
   float* delta = static_cast<float*>(workspace);
+  float* norm = mask_kind == 2 && workspace_bytes >= 2 * need ? delta + batch * q_heads * seq_q : nullptr;
   if (nmb::mfma_shape(p, head_dim, dtype, {q, k, v, o, dout, dq}))
     nmb::mfma_bwd_launch(p, mr, dp, mask_kind, dropout_p > 0.f, static_cast<int>(head_dim), q, k, v, o, dout, lse,
-                         delta, dq, dk, dv, stream);
+                         delta, norm, dq, dk, dv, stream);
   else if (dtype == NMB_BF16)
-    nmb::f32_bwd_launch<nmb::bf16>(p, kv, mr, dp, mask_kind, dropout_p > 0.f, q, o, dout, lse, delta, dq,
+    nmb::f32_bwd_launch<nmb::bf16>(p, kv, mr, dp, mask_kind, dropout_p > 0.f, q, o, dout, lse, delta, norm, dq,
                                    static_cast<int>(head_dim), stream);
   else
-    nmb::f32_bwd_launch<float>(p, kv, mr, dp, mask_kind, dropout_p > 0.f, q, o, dout, lse, delta, dq,
+    nmb::f32_bwd_launch<float>(p, kv, mr, dp, mask_kind, dropout_p > 0.f, q, o, dout, lse, delta, norm, dq,
                                static_cast<int>(head_dim), stream);
   NMB_CHECK_LAUNCH("attn_masked_bwd");
   return NMB_OK;

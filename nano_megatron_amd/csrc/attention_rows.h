@@ -86,10 +86,14 @@ __device__ void row_fwd(const T* qr, const T* kb, const T* vb, int64_t koff, int
   }
 }
 
-// dQ of query row i (before the scale), from its lse and delta.
+// 1 / sum of a row's probabilities (0 for a row without any)
+__device__ __forceinline__ float inverse_sum(float s) { return s > 0.f ? 1.f / s : (s == 0.f ? 0.f : s); }
+
+// dQ of query row i (before the scale), from its lse and delta; psum: the sum
+// of its probabilities.
 template <typename T, int MK, bool DROP>
 __device__ void row_dq(const T* qr, const T* dr, const T* kb, const T* vb, int64_t koff, int i, float lse, float delta,
-                       const AttnShape& p, int D, const RowMask& rm, int lane, float (&acc)[2]) {
+                       const AttnShape& p, int D, const RowMask& rm, int lane, float (&acc)[2], float& psum) {
   if (lse == -__builtin_inff()) return;
   for (int j = 0; j < p.Sk; ++j) {
     if (p.causal && koff + j > p.q_offset + i) break;
@@ -98,6 +102,7 @@ __device__ void row_dq(const T* qr, const T* dr, const T* kb, const T* vb, int64
     const T* kr = kb + static_cast<int64_t>(j) * p.kv_ss;
     const T* vr = vb + static_cast<int64_t>(j) * p.kv_ss;
     const float pv = expf(row_dot(qr, kr, D, lane) * p.scale + add - lse);
+    psum += pv;
     const float ds = pv * (row_keep<DROP>(rm, p, i, j) * row_dot(dr, vr, D, lane) - delta);
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
@@ -108,11 +113,11 @@ __device__ void row_dq(const T* qr, const T* dr, const T* kb, const T* vb, int64
 }
 
 // dK (before the scale) and dV of key j (rows kr, vr) from the queries of one
-// head (rows from qb, db; lse and delta of the head).
+// head (rows from qb, db; lse, delta and, if given, norm of the head).
 template <typename T, int MK, bool DROP>
 __device__ void row_dkdv(const T* kr, const T* vr, const T* qb, const T* db, const float* lse, const float* delta,
-                         int64_t koff, int j, const AttnShape& p, int D, const RowMask& rm, int lane, float (&dk)[2],
-                         float (&dv)[2]) {
+                         const float* norm, int64_t koff, int j, const AttnShape& p, int D, const RowMask& rm, int lane,
+                         float (&dk)[2], float (&dv)[2]) {
   for (int i = 0; i < p.Sq; ++i) {
     const float ls = lse[i];
     float add;
@@ -120,7 +125,8 @@ __device__ void row_dkdv(const T* kr, const T* vr, const T* qb, const T* db, con
       continue;
     const T* qr = qb + static_cast<int64_t>(i) * p.q_ss;
     const T* dr = db + static_cast<int64_t>(i) * p.o_ss;
-    const float pv = expf(row_dot(qr, kr, D, lane) * p.scale + add - ls);
+    float pv = expf(row_dot(qr, kr, D, lane) * p.scale + add - ls);
+    if (norm != nullptr) pv *= norm[i];
     const float z = row_keep<DROP>(rm, p, i, j);
     const float ds = pv * (z * row_dot(dr, vr, D, lane) - delta[i]);
     const float pz = pv * z;

@@ -14,6 +14,7 @@ import torch
 import nano_megatron_amd.functional as Fn
 from oracle import reference as R
 from tests.parity import rel_l2
+from tests.test_gpu_attention_f32 import _reference
 
 pytestmark = pytest.mark.gpu
 
@@ -40,7 +41,8 @@ def test_masked_mfma_attention_matches_oracle(kind, causal, offset, hq, hkv, sq,
     rounding: at most 2^-9 of each element, hence of the norm (bf16
     probabilities would add as much again).  dQ and dK also see delta formed
     from the rounded O: twice that bound.  Keys hidden from every query may
-    hold NaN; a row of masks of the lowest value averages over all keys."""
+    hold NaN; a row of masks of the lowest value averages over all keys, forward
+    and backward."""
     g = torch.Generator().manual_seed(11)
     b = 2
     q, do = (torch.randn(b, hq, sq, d, generator=g).bfloat16() for _ in range(2))
@@ -60,13 +62,20 @@ def test_masked_mfma_attention_matches_oracle(kind, causal, offset, hq, hkv, sq,
         mask[2, 1:9] = float("-inf")
         mask[1, 4:] = torch.finfo(torch.bfloat16).min
         mask[0] = torch.finfo(torch.bfloat16).min
-        do[:, :, 0] = 0
         mask[4] = float("-inf")
     qr, kr, vr = (t.float().clone().requires_grad_(True) for t in (q, k, v))
     mr = mask.float() if kind == "add" else mask
-    o_ref = R.local_attention(qr, kr, vr, causal=causal, sequence_offset=offset, attention_mask=mr, dropout_p=p,
-                              dropout_seed=77)
-    o_ref.backward(do.float())
+    if kind == "add":
+        # (the oracle's fused CPU backward forms P as exp(x - lse), which is 1 for
+        # every key of the row of lowest values: the explicit softmax instead, and
+        # zeros for the row of -inf)
+        mr[4] = 0.0
+        o_ref = _reference(qr.double(), kr.double(), vr.double(), causal, offset, mr, p, 77)
+        o_ref = o_ref.index_fill(2, torch.tensor([4]), 0.0)
+    else:
+        o_ref = R.local_attention(qr, kr, vr, causal=causal, sequence_offset=offset, attention_mask=mr, dropout_p=p,
+                                  dropout_seed=77)
+    o_ref.backward(do.to(o_ref.dtype))
     if kind == "keys":
         hidden = ~mask[:, :, 0, :, None].expand(b, hkv, sk, d)
         k, v = k.masked_fill(hidden, float("nan")), v.masked_fill(hidden, float("nan"))
