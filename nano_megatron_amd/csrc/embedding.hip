@@ -65,12 +65,15 @@ __global__ __launch_bounds__(256) void embedding_fwd_kernel(const T* __restrict_
 }
 
 // List (segment blockIdx.y, group blockIdx.x): the segment's tokens whose id is
-// in the group's rows, in token order; counts[segment][group].
+// in the group's rows, in token order.  A segment's lists stand one after the
+// other in its kSegment entries (a token is in one list at most): list g at
+// [starts[segment][g], starts[segment][g + 1]), the start being the number of
+// ids below the group's rows, which the workgroup counts as it goes over them.
 __global__ __launch_bounds__(1024) void embedding_list_kernel(const int64_t* __restrict__ ids, int64_t n_tokens,
-                                                              int64_t vocab, int* __restrict__ counts,
+                                                              int64_t vocab, int* __restrict__ starts,
                                                               int* __restrict__ lists, int row_bits) {
   constexpr int kPer = kSegment / 1024;
-  __shared__ int totals[16];
+  __shared__ int totals[16], below[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t v0 = static_cast<int64_t>(blockIdx.x) << row_bits;
   const int64_t v1 = min(v0 + (int64_t{1} << row_bits), vocab);
@@ -88,13 +91,21 @@ __global__ __launch_bounds__(1024) void embedding_list_kernel(const int64_t* __r
     const int y = __shfl_up(incl, d, 64);
     if (lane >= d) incl += y;
   }
-  if (lane == 63) totals[wave] = incl;
+  int lower = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) lower += static_cast<int>(__popcll(__ballot(id[j] >= 0 && id[j] < v0)));
+  if (lane == 63) {
+    totals[wave] = incl;
+    below[wave] = lower;
+  }
   __syncthreads();
   int pos = incl - hits;
   for (int w = 0; w < wave; ++w) pos += totals[w];
-  const int64_t list = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
-  if (threadIdx.x == 1023) counts[list] = pos + hits;
-  int* out = lists + list * kSegment;
+  for (int w = 0; w < 16; ++w) pos += below[w];
+  int* start = starts + static_cast<int64_t>(blockIdx.y) * (gridDim.x + 1) + blockIdx.x;
+  if (threadIdx.x == 0) start[0] = pos;
+  if (threadIdx.x == 1023 && blockIdx.x + 1 == gridDim.x) start[1] = pos + hits;
+  int* out = lists + base;
 #pragma unroll
   for (int j = 0; j < kPer; ++j)
     if (id[j] >= v0 && id[j] < v1) out[pos++] = (t0 + j) << row_bits | static_cast<int>(id[j] - v0);
@@ -128,7 +139,7 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict_
                                                             const T* __restrict__ grad_in,
                                                             T* __restrict__ grad_out, int64_t n_tokens,
                                                             int64_t vocab, int64_t hidden,
-                                                            const int* __restrict__ counts,
+                                                            const int* __restrict__ starts,
                                                             const int* __restrict__ lists, int groups, int row_bits,
                                                             int chunks) {
   using Raw = typename Quad<T>::Raw;
@@ -170,15 +181,20 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict_
   const int64_t g0 = static_cast<int64_t>(group) << row_bits;
   const int r0 = static_cast<int>(v0 - g0);
   const int segments = LISTS ? static_cast<int>((n_tokens + kSegment - 1) / kSegment) : 1;
-  auto entries = [&](int s) {
-    return LISTS ? counts[static_cast<int64_t>(s) * groups + group] : static_cast<int>(n_tokens);
+  struct List {
+    int start, n;
   };
-  auto fetch = [&](int s, int k, int n, int& row, int& token) {
+  auto entries = [&](int s) {
+    if constexpr (!LISTS) return List{0, static_cast<int>(n_tokens)};
+    const int* st = starts + static_cast<int64_t>(s) * (groups + 1) + group;
+    return List{st[0], st[1] - st[0]};
+  };
+  auto fetch = [&](int s, const List& l, int k, int& row, int& token) {
     row = -1;
     token = 0;
-    if (k + lane >= n) return;
+    if (k + lane >= l.n) return;
     if constexpr (LISTS) {
-      const int e = lists[(static_cast<int64_t>(s) * groups + group) * kSegment + k + lane];
+      const int e = lists[static_cast<int64_t>(s) * kSegment + l.start + k + lane];
       row = e & ((1 << row_bits) - 1);
       token = s * kSegment + (e >> row_bits);
     } else {
@@ -192,14 +208,14 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict_
   int cnt[RV];
 #pragma unroll
   for (int r = 0; r < RV; ++r) cnt[r] = 0;
-  const int n0 = segments > 0 ? entries(0) : 0;
+  const List first = segments > 0 ? entries(0) : List{0, 0};
   int row0 = -1, token0 = 0;  // the first entries, kept
-  fetch(0, 0, n0, row0, token0);
+  fetch(0, first, 0, row0, token0);
   for (int s = 0; s < segments; ++s) {
-    const int n = s == 0 ? n0 : entries(s);
-    for (int k = 0; k < n; k += 64) {
+    const List l = s == 0 ? first : entries(s);
+    for (int k = 0; k < l.n; k += 64) {
       int row = row0, token;
-      if (s != 0 || k != 0) fetch(s, k, n, row, token);
+      if (s != 0 || k != 0) fetch(s, l, k, row, token);
 #pragma unroll
       for (int r = 0; r < RV; ++r) cnt[r] += __popcll(__ballot(row == r0 + r));
     }
@@ -238,10 +254,10 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict_
   // every row loaded together
   int left = (cnt[0] + cnt[1]) + (cnt[2] + cnt[3]);
   for (int s = 0; s < segments && left > 0; ++s) {
-    const int n = s == 0 ? n0 : entries(s);
-    for (int k = 0; k < n && left > 0; k += 64) {
+    const List l = s == 0 ? first : entries(s);
+    for (int k = 0; k < l.n && left > 0; k += 64) {
       int row = row0, token = token0;
-      if (s != 0 || k != 0) fetch(s, k, n, row, token);
+      if (s != 0 || k != 0) fetch(s, l, k, row, token);
       uint64_t mask[RV];
       int n4[RV];
       Raw raw[RV][4];
@@ -300,15 +316,15 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict_
       if (wave == 0) {
         int n = 0;
         while (s < segments && n <= kTokens - 64) {
-          const int ns = entries(s);
-          for (; k < ns && n <= kTokens - 64; k += 64) {
+          const List l = entries(s);
+          for (; k < l.n && n <= kTokens - 64; k += 64) {
             int row, token;
-            fetch(s, k, ns, row, token);
+            fetch(s, l, k, row, token);
             const uint64_t mask = __ballot(row == row_in_group);
             if (row == row_in_group) tok[n + __popcll(mask & ((1ull << lane) - 1))] = token;
             n += static_cast<int>(__popcll(mask));
           }
-          if (k >= ns) {
+          if (k >= l.n) {
             ++s;
             k = 0;
           }
@@ -359,14 +375,15 @@ int list_row_bits(int64_t vocab) {
   return bits;
 }
 
-// Bytes of the counts (rounded up to 256) and lists of n_tokens ids.  Up to 64
-// tokens every wavefront scans the ids itself (one step) instead of a launch
-// for the lists (30 tokens: 5.2 us).
+// Bytes of the starts (rounded up to 256) and lists of n_tokens ids: 4 bytes per
+// token and at most 1 KB per 8,192.  Up to 64 tokens every wavefront scans the
+// ids itself (one step) instead of a launch for the lists (30 tokens: 5.2 us).
+int64_t starts_bytes(int64_t n_tokens, int64_t groups) {
+  return ((n_tokens + kSegment - 1) / kSegment * (groups + 1) * 4 + 255) / 256 * 256;
+}
 int64_t list_bytes(int64_t n_tokens, int64_t vocab) {
   if (n_tokens <= 64) return 0;
-  const int bits = list_row_bits(vocab);
-  const int64_t lists = (n_tokens + kSegment - 1) / kSegment * (((vocab - 1) >> bits) + 1);
-  return (lists * 4 + 255) / 256 * 256 + lists * kSegment * 4;
+  return starts_bytes(n_tokens, ((vocab - 1) >> list_row_bits(vocab)) + 1) + n_tokens * 4;
 }
 
 template <typename T>
@@ -409,25 +426,25 @@ int bwd_impl(const void* dout, const int64_t* ids, const void* grad_in, void* gr
               static_cast<int>(align + 1));
   if (blocks == 0) return NMB_OK;
   const int64_t bytes = workspace != nullptr ? list_bytes(n_tokens, vocab) : 0;
-  int* counts = nullptr;
+  int* starts = nullptr;
   int* lists = nullptr;
   if (bytes > 0) {
     NMB_REQUIRE(workspace_bytes >= bytes, "embedding_bwd: workspace of %lld bytes is smaller than the %lld required",
                 (long long)workspace_bytes, (long long)bytes);
     const int64_t segments = (n_tokens + kSegment - 1) / kSegment;
-    counts = static_cast<int*>(workspace);
-    lists = counts + (segments * groups * 4 + 255) / 256 * 64;
+    starts = static_cast<int*>(workspace);
+    lists = starts + starts_bytes(n_tokens, groups) / 4;
     hipLaunchKernelGGL(embedding_list_kernel, dim3(static_cast<unsigned>(groups), static_cast<unsigned>(segments)),
-                       dim3(1024), 0, stream, ids, n_tokens, vocab, counts, lists, row_bits);
+                       dim3(1024), 0, stream, ids, n_tokens, vocab, starts, lists, row_bits);
     NMB_CHECK_LAUNCH("embedding_bwd(lists)");
     hipLaunchKernelGGL((embedding_bwd_kernel<T, true>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
                        static_cast<const T*>(dout), ids, static_cast<const T*>(grad_in), static_cast<T*>(grad_out),
-                       n_tokens, vocab, hidden, counts, lists, static_cast<int>(groups), row_bits,
+                       n_tokens, vocab, hidden, starts, lists, static_cast<int>(groups), row_bits,
                        static_cast<int>(chunks));
   } else {
     hipLaunchKernelGGL((embedding_bwd_kernel<T, false>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
                        static_cast<const T*>(dout), ids, static_cast<const T*>(grad_in), static_cast<T*>(grad_out),
-                       n_tokens, vocab, hidden, counts, lists, static_cast<int>(groups), row_bits,
+                       n_tokens, vocab, hidden, starts, lists, static_cast<int>(groups), row_bits,
                        static_cast<int>(chunks));
   }
   NMB_CHECK_LAUNCH("embedding_bwd");

@@ -214,3 +214,12 @@ def test_masked_attention_rejects_bad_dropout_and_mask_kind() -> None:
     assert st == _lib.NMB_EINVAL and b"mask_kind" in lib.nmb_last_error()
     st = lib.nmb_attn_masked_fwd(*args, None, 1, None, 1, 0, 0.0, 0.1, 5, _lib.NMB_BF16, None)
     assert st == _lib.NMB_EINVAL and b"null mask" in lib.nmb_last_error()
+
+
+@pytest.mark.parametrize("tokens", [0, 64, 65, 8192, 8193, 262144, (1 << 27) - 1])
+@pytest.mark.parametrize("vocab", [1, 8192, 50304, 1 << 20])
+def test_embedding_lists_take_a_few_bytes_per_token(tokens, vocab) -> None:
+    """A token is in one list at most: 4 bytes each and 256 list starts per 8,192 tokens."""
+    nbytes = ctypes.c_int64()
+    assert _lib.load().nmb_embedding_bwd_workspace_bytes(tokens, vocab, ctypes.byref(nbytes)) == 0
+    assert 0 <= nbytes.value <= 4 * tokens + 4 * 257 * -(-tokens // 8192) + 256
