@@ -36,6 +36,11 @@ constexpr int CW = 256;         // columns per wavefront (4 per lane)
 constexpr int kSegment = 8192;  // tokens per list
 constexpr int kHot = 24;        // more tokens than this: the row is added by the whole workgroup
 constexpr int kTokens = 1024;   // such a row's tokens held in LDS
+constexpr int kFewTokens = 64;  // no lists up to here
+// Without a workspace every wavefront scans the ids up to here, else workgroups
+// walk them (hidden 768, vocabulary 50,304: 65 tokens 22.6 against 29.5 us, 200
+// 28.1 and 29.7, 8,192 746 and 99)
+constexpr int kScanTokens = 192;
 
 template <typename T>
 __global__ __launch_bounds__(256) void embedding_fwd_kernel(const T* __restrict__ table,
@@ -131,8 +136,8 @@ __device__ __forceinline__ void unpack4(const typename Quad<T>::Raw& raw, float 
   for (int i = 0; i < 4; ++i) v[i] = to_f32(e[i]);
 }
 
-// LISTS: the tokens come from embedding_list_kernel's lists; else every id is
-// scanned (few tokens, or a caller without a workspace).
+// LISTS: the tokens come from embedding_list_kernel's lists; else every
+// wavefront scans the ids, 64 at a step (up to kScanTokens).
 template <typename T, bool LISTS>
 __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict__ dout,
                                                             const int64_t* __restrict__ ids,
@@ -366,6 +371,152 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* __restrict_
   }
 }
 
+// Backward of a caller without a workspace for the lists: a workgroup owns 16
+// table rows x 1,024 columns, goes over the ids in rounds of 2,048 (8 consecutive
+// ones per thread, loaded together), lists the tokens of its rows in token order
+// (a workgroup prefix sum of each thread's hits), and once the ids are done (or
+// the list is full) adds their gradient rows, sixteen in flight, to fp32
+// accumulators in LDS in list order.  The ids (8 bytes a token) are read by
+// every workgroup from L2, which bounds it for many tokens.
+constexpr int kWalkRows = 16, kWalkCols = 1024;
+constexpr int kWalkPer = 8, kWalkRound = 256 * kWalkPer;
+constexpr int kWalkList = 3072;  // listed tokens held before their rows are added (12 KB of LDS)
+constexpr int kWalkBatch = 16;   // gradient rows loaded together
+
+template <typename T>
+__device__ __forceinline__ void load4(const T* p, float (&v)[4]) {
+  unpack4<T>(*reinterpret_cast<const typename Quad<T>::Raw*>(p), v);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256, 2) void embedding_bwd_walk_kernel(const T* __restrict__ dout,
+                                                                    const int64_t* __restrict__ ids,
+                                                                    const T* __restrict__ grad_in,
+                                                                    T* __restrict__ grad_out, int64_t n_tokens,
+                                                                    int64_t vocab, int64_t hidden) {
+  __shared__ float4 acc[kWalkRows * kWalkCols / 4];  // 64 KB: row r, this thread's 4 columns at [r * kWalkCols / 4 + thread]
+  __shared__ int list[kWalkList];          // matching tokens in token order: token * kWalkRows + row
+  __shared__ int wave_total[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t row_blocks = (vocab + kWalkRows - 1) / kWalkRows;
+  const int64_t v0 = (blockIdx.x % row_blocks) * kWalkRows;
+  const int64_t c0 = (blockIdx.x / row_blocks) * kWalkCols;
+  const int cols = static_cast<int>(min<int64_t>(kWalkCols, hidden - c0));
+  const int c = threadIdx.x * 4;  // this thread's 4 columns
+  const int cc = c < cols ? c : 0;  // (a thread past the chunk's columns loads column 0, unused)
+#pragma unroll
+  for (int r = 0; r < kWalkRows; ++r) acc[r * (kWalkCols / 4) + threadIdx.x] = make_float4(0.f, 0.f, 0.f, 0.f);
+
+  // the tied LM head's rows of this block, loaded first: nothing depends on
+  // them until the end (rows past the table read its last row, not stored)
+  float prior[kWalkRows][4];
+#pragma unroll
+  for (int r = 0; r < kWalkRows; ++r) {
+    if (grad_in != nullptr) {
+      load4(grad_in + min(v0 + r, vocab - 1) * hidden + c0 + cc, prior[r]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) prior[r][e] = 0.f;
+    }
+  }
+
+  // the listed gradient rows, in token order, into the accumulators: all of
+  // a batch's loads in flight together
+  int listed = 0;  // workgroup-uniform
+  auto add_listed = [&]() {
+    if (c < cols) {
+      for (int k0 = 0; k0 < listed; k0 += kWalkBatch) {
+        float v[kWalkBatch][4];
+        int row[kWalkBatch];
+#pragma unroll
+        for (int u = 0; u < kWalkBatch; ++u) {
+          const int e = list[min(k0 + u, listed - 1)];
+          row[u] = e % kWalkRows;
+          load4(dout + static_cast<int64_t>(e / kWalkRows) * hidden + c0 + c, v[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kWalkBatch; ++u) {
+          if (k0 + u < listed) {  // (no break: the loaded rows stay in registers)
+            float4& a = acc[row[u] * (kWalkCols / 4) + threadIdx.x];
+            float4 t = a;
+            t.x += v[u][0];
+            t.y += v[u][1];
+            t.z += v[u][2];
+            t.w += v[u][3];
+            a = t;
+          }
+        }
+      }
+    }
+    listed = 0;
+  };
+
+  // the ids in rounds of kWalkPer consecutive tokens per thread, the next round's
+  // in flight while this round's are listed; the rows are added once the
+  // list is full or the ids are done, so that their loads are not spread
+  // over the rounds one latency each
+  int64_t id[kWalkPer], next[kWalkPer];
+#pragma unroll
+  for (int j = 0; j < kWalkPer; ++j) next[j] = -1;
+  auto load_ids = [&](int64_t base, int64_t (&dst)[kWalkPer]) {
+    const int64_t t0 = base + threadIdx.x * kWalkPer;
+#pragma unroll
+    for (int j = 0; j < kWalkPer; ++j) dst[j] = t0 + j < n_tokens ? ids[t0 + j] : -1;
+  };
+  load_ids(0, id);
+  for (int64_t base = 0; base < n_tokens; base += kWalkRound) {
+    if (listed > kWalkList - kWalkRound) {
+      // a full round may not fit: add what is listed first (every thread is
+      // past the previous round's list writes: second barrier below)
+      add_listed();
+      __syncthreads();  // every thread is done reading the list
+    }
+    const int t_off = static_cast<int>(base) + threadIdx.x * kWalkPer;
+    int hits = 0;
+#pragma unroll
+    for (int j = 0; j < kWalkPer; ++j) hits += id[j] >= v0 && id[j] < v0 + kWalkRows;
+    // exclusive prefix of the hits over the workgroup (thread order = token order)
+    int incl = hits;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += y;
+    }
+    if (lane == 63) wave_total[wave] = incl;
+    __syncthreads();  // wave totals ready
+    int pos = listed + incl - hits;
+    for (int w = 0; w < wave; ++w) pos += wave_total[w];
+    const int total = wave_total[0] + wave_total[1] + wave_total[2] + wave_total[3];
+#pragma unroll
+    for (int j = 0; j < kWalkPer; ++j)
+      if (id[j] >= v0 && id[j] < v0 + kWalkRows) list[pos++] = (t_off + j) * kWalkRows + static_cast<int>(id[j] - v0);
+    listed += total;
+    __syncthreads();  // the round's list entries are visible; wave totals read
+    if (base + kWalkRound < n_tokens) load_ids(base + kWalkRound, next);
+#pragma unroll
+    for (int j = 0; j < kWalkPer; ++j) id[j] = next[j];
+  }
+  add_listed();
+  __syncthreads();
+  if (c >= cols) return;
+#pragma unroll
+  for (int r = 0; r < kWalkRows; ++r) {
+    if (v0 + r >= vocab) break;
+    const int64_t o = (v0 + r) * hidden + c0 + c;
+    const float4 a4 = acc[r * (kWalkCols / 4) + threadIdx.x];
+    const float av[4] = {a4.x, a4.y, a4.z, a4.w};
+    T out[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float mine = round_as<T>(av[e]);  // as in embedding_bwd_kernel
+      out[e] = from_f32<T>(grad_in != nullptr ? add_rn(prior[r][e], mine) : mine);
+    }
+    typename Quad<T>::Raw raw;
+    __builtin_memcpy(&raw, out, sizeof(out));
+    *reinterpret_cast<typename Quad<T>::Raw*>(grad_out + o) = raw;
+  }
+}
+
 // Rows per list as a power of two: lists as short as 256 of them allow (a
 // wavefront scans its rows' list 64 entries at a time), 32 rows at least; an
 // entry holds a token of 13 bits and a row of at most 18.
@@ -377,12 +528,13 @@ int list_row_bits(int64_t vocab) {
 
 // Bytes of the starts (rounded up to 256) and lists of n_tokens ids: 4 bytes per
 // token and at most 1 KB per 8,192.  Up to 64 tokens every wavefront scans the
-// ids itself (one step) instead of a launch for the lists (30 tokens: 5.2 us).
+// ids itself (one step) instead of a launch for the lists (64 tokens x 768,
+// vocabulary 50,304, forward and backward replayed: 30.5 us, with lists 34).
 int64_t starts_bytes(int64_t n_tokens, int64_t groups) {
   return ((n_tokens + kSegment - 1) / kSegment * (groups + 1) * 4 + 255) / 256 * 256;
 }
 int64_t list_bytes(int64_t n_tokens, int64_t vocab) {
-  if (n_tokens <= 64) return 0;
+  if (n_tokens <= kFewTokens) return 0;
   return starts_bytes(n_tokens, ((vocab - 1) >> list_row_bits(vocab)) + 1) + n_tokens * 4;
 }
 
@@ -441,11 +593,16 @@ int bwd_impl(const void* dout, const int64_t* ids, const void* grad_in, void* gr
                        static_cast<const T*>(dout), ids, static_cast<const T*>(grad_in), static_cast<T*>(grad_out),
                        n_tokens, vocab, hidden, starts, lists, static_cast<int>(groups), row_bits,
                        static_cast<int>(chunks));
-  } else {
+  } else if (n_tokens <= kScanTokens) {
     hipLaunchKernelGGL((embedding_bwd_kernel<T, false>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
                        static_cast<const T*>(dout), ids, static_cast<const T*>(grad_in), static_cast<T*>(grad_out),
                        n_tokens, vocab, hidden, starts, lists, static_cast<int>(groups), row_bits,
                        static_cast<int>(chunks));
+  } else {
+    const int64_t walkers = ((vocab + kWalkRows - 1) / kWalkRows) * ((hidden + kWalkCols - 1) / kWalkCols);
+    hipLaunchKernelGGL(embedding_bwd_walk_kernel<T>, dim3(static_cast<unsigned>(walkers)), dim3(256), 0, stream,
+                       static_cast<const T*>(dout), ids, static_cast<const T*>(grad_in), static_cast<T*>(grad_out),
+                       n_tokens, vocab, hidden);
   }
   NMB_CHECK_LAUNCH("embedding_bwd");
   return NMB_OK;

@@ -48,7 +48,7 @@ def test_listed_tokens_are_added_in_order(dtype, tokens, vocab, hidden, tied) ->
 
 
 @pytest.mark.parametrize("entry,tokens", [("nmb_embedding_bwd_ws", 64), ("nmb_embedding_bwd_ws", 300),
-                                          ("nmb_embedding_bwd", 30), ("nmb_embedding_bwd", 300)])
+                                          ("nmb_embedding_bwd", 30), ("nmb_embedding_bwd", 192), ("nmb_embedding_bwd", 300)])
 @pytest.mark.parametrize("vocab", [17, 8190, 50257])
 def test_repeated_ids_past_the_table_write_nothing(entry, tokens, vocab) -> None:
     """More than 24 tokens of one id (the rows a whole workgroup adds up) at and
