@@ -1,9 +1,8 @@
 """Device ops of the GPT block: thin wrappers over libnmb.so plus autograd Functions.
 
 Every op runs on the GPU through the C ABI; a CPU tensor is an error, never a
-fallback.  Every bf16 op, the dense projections included, is a hand-written
-gfx950 kernel; fp32 (the parity configuration) projections use the library
-GEMM.
+fallback.  Every op, the dense projections included, is a hand-written gfx950
+kernel, in bf16 and in fp32 (the parity configuration).
 
 Attention tensors use one memory layout throughout: ``[batch, seq, heads,
 head_dim]`` (the layout of the Q/K/V projection outputs), seen through a
