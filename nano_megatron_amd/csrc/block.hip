@@ -91,7 +91,15 @@ int forward_ws(const Dims& d, int64_t* bytes) {
   return NMB_OK;
 }
 
-// The backward's scratch: byte offsets of its parts in one buffer.
+// The backward's scratch: byte offsets of its parts in one buffer.  What only
+// the main stream reads and writes shares its place with what comes before or
+// after it there: dn2 (until the post-attention norm) with dqkv, do2 (until the
+// attention) with dn1, fp32's [g|u] and ds (until the SwiGLU backward) with all
+// of these, and the workspaces of the main stream's products, the attention and
+// the input norm with each other.  The second stream reads dgu, act, ws_side
+// and ws_post until it is joined, so those keep theirs.  (All parts side by
+// side: 373 MB against 339 at config 3, 4 x 2048 tokens of hidden 2048 635
+// against 501.)
 struct BwdScratch {
   int64_t dgu, act, dn2, dh, do2, dqkv, dn1, gu, ds, attn, ws_main, ws_side, ws_post, ws_in, total;
   int64_t main_bytes, side_bytes, attn_bytes, norm_bytes;
@@ -128,18 +136,15 @@ int backward_scratch(const nmb_block* b, const Dims& d, BwdScratch* s) {
   };
   s->dgu = take(d.T * 2 * d.F * d.es);
   s->act = take(d.T * d.F * d.es);
-  s->dn2 = take(d.T * d.H * d.es);
+  s->gu = at;
+  s->ds = s->gu + align256(d.T * 2 * d.F * d.es);
   s->dh = take(d.T * d.H * d.es);
-  s->do2 = take(d.T * d.Nq * d.es);
-  s->dqkv = take(d.T * d.N * d.es);
-  s->dn1 = take(d.T * d.H * d.es);
-  s->gu = d.bf16 ? 0 : take(d.T * 2 * d.F * d.es);
-  s->ds = d.bf16 ? 0 : take(d.T * d.F * d.es);
-  s->attn = take(s->attn_bytes);
-  s->ws_main = take(s->main_bytes);
+  s->do2 = s->dn1 = take(d.T * std::max(d.Nq, d.H) * d.es);
+  s->dqkv = s->dn2 = take(d.T * std::max(d.N, d.H) * d.es);
+  if (!d.bf16) at = std::max(at, s->ds + align256(d.T * d.F * d.es));
+  s->attn = s->ws_main = s->ws_in = take(std::max(std::max(s->attn_bytes, s->main_bytes), s->norm_bytes));
   s->ws_side = take(s->side_bytes);
   s->ws_post = take(s->norm_bytes);
-  s->ws_in = take(s->norm_bytes);
   s->total = at;
   return NMB_OK;
 }

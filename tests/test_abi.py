@@ -223,3 +223,37 @@ def test_embedding_lists_take_a_few_bytes_per_token(tokens, vocab) -> None:
     nbytes = ctypes.c_int64()
     assert _lib.load().nmb_embedding_bwd_workspace_bytes(tokens, vocab, ctypes.byref(nbytes)) == 0
     assert 0 <= nbytes.value <= 4 * tokens + 4 * 257 * -(-tokens // 8192) + 256
+
+
+@pytest.mark.parametrize("b,s,h,hq,hkv,d,f", [(16, 512, 1024, 16, 16, 64, 2736), (4, 2048, 2048, 32, 8, 64, 5632),
+                                              (3, 709, 768, 12, 12, 64, 2048), (4, 128, 256, 4, 4, 64, 688)])
+@pytest.mark.parametrize("dtype", [_lib.NMB_BF16, _lib.NMB_F32])
+def test_block_backward_scratch_shares_what_is_not_live_together(b, s, h, hq, hkv, d, f, dtype) -> None:
+    """At any time no more is live than [dg|du], the activation, the norm's dx, one
+    of dO / dn1, one of dn2 / dqkv (fp32 before these: [g|u] and ds), and one
+    workspace per stream besides the post-attention norm's."""
+    lib, t, es = _lib.load(), b * s, 2 if dtype == _lib.NMB_BF16 else 4
+    blk = _lib.Block(batch=b, seq=s, hidden=h, q_heads=hq, kv_heads=hkv, head_dim=d, ffn=f, dtype=dtype)
+    got = ctypes.c_int64()
+    assert lib.nmb_block_sizes(ctypes.byref(blk), None, ctypes.byref(got)) == 0
+    nq, n = hq * d, (hq + 2 * hkv) * d
+
+    def gemm(la, lb, *mnk):
+        v = ctypes.c_int64()
+        if es == 2:
+            assert lib.nmb_gemm_bf16_workspace_bytes(la, lb, *mnk, ctypes.byref(v)) == 0
+        else:
+            assert lib.nmb_gemm_f32_workspace_bytes(*mnk, ctypes.byref(v)) == 0
+        return v.value
+
+    attn, norm = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.nmb_attn_bwd_workspace_bytes_split(b, hq, hkv, s, s, d, 1, dtype, ctypes.byref(attn)) == 0
+    assert lib.nmb_rmsnorm_bwd_workspace_bytes(t, h, ctypes.byref(norm)) == 0
+    side = max(gemm(1, 1, h, f, t), gemm(1, 1, 2 * f, h, t))
+    main = max(gemm(0, 1, t, h, 2 * f), gemm(0, 1, t, nq, h), gemm(1, 1, h, nq, t), gemm(0, 1, t, h, n),
+               gemm(1, 1, n, h, t), attn.value, norm.value)
+    group = t * es * (h + max(nq, h) + max(n, h))
+    if es == 4:
+        main = max(main, gemm(0, 0, t, 2 * f, h), gemm(0, 1, t, f, h))
+        group = max(group, t * es * 3 * f)
+    assert got.value <= t * es * 3 * f + group + main + side + norm.value + 16 * 256
