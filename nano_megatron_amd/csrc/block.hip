@@ -98,8 +98,8 @@ int forward_ws(const Dims& d, int64_t* bytes) {
 // of these, and the workspaces of the main stream's products, the attention and
 // the input norm with each other.  The second stream reads dgu, act, ws_side
 // and ws_post until it is joined, so those keep theirs.  (All parts side by
-// side: 373 MB against 339 at config 3, 4 x 2048 tokens of hidden 2048 635
-// against 501.)
+// side: 374 MB against 338 for 16 x 512 tokens of hidden 1024, 635 against 499
+// for 4 x 2048 of hidden 2048.)
 struct BwdScratch {
   int64_t dgu, act, dn2, dh, do2, dqkv, dn1, gu, ds, attn, ws_main, ws_side, ws_post, ws_in, total;
   int64_t main_bytes, side_bytes, attn_bytes, norm_bytes;
