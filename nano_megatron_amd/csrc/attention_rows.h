@@ -83,6 +83,7 @@ __device__ void row_fwd(const T* qr, const T* kb, const T* vb, int64_t koff, int
       const int d = lane + 64 * c;
       if (d < D) acc[c] = acc[c] * alpha + pz * to_f32(vr[d]);
     }
+    if (l != l) break;  // NaN: sum and outputs stay so
   }
 }
 
